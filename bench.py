@@ -286,8 +286,8 @@ def mix_paths(specs, args):
         row.update({"value": E * args.steps / (total_ms / 1e3), "ms_per_step": total_ms / args.steps,
                     "p50_ms": float(np.percentile(lat, 50)), "p99_ms": float(np.percentile(lat, 99))})
         if prec == "FP64_TILED" and seq:
-            # the node-after-node dot products run in 8 segments at once from candidate starts
-            # (the library's default, the same bits); boundaries summed from the known start instead
+            # the node-after-node dot products by exact parallel rounding (the library's default, the
+            # chain's bits)
             row["dot_segments"] = {"segments": 8, "window": 32,
                                    "fallbacks": int(sum(eng.stats(i)["dot_fallbacks"] for i in ids)),
                                    "steps": args.error_steps + args.warmup + args.steps}

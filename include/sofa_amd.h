@@ -67,10 +67,9 @@ typedef struct sofa_amd_cg_stats {
     double  err;            /* last sqrt(r.r)/|b|                                            */
     double  den;            /* last p.A.p                                                    */
     double  time;           /* context time of the scene                                     */
-    int32_t dot_fallbacks;  /* FP64_TILED in the reference order with segmented dot products:
-                               segment boundaries where no candidate start matched (the segment
-                               was summed from the known start instead) since the scene was
-                               placed; else 0                                                    */
+    int32_t dot_fallbacks;  /* FP64_TILED in the reference order with dot products in segments
+                               without candidates (window 0): boundaries summed by the chain
+                               since the scene was placed; else 0                                */
     int32_t reserved;       /* 0                                                                 */
 } sofa_amd_cg_stats;
 
@@ -279,15 +278,12 @@ int sofa_amd_engine_set_branch_turns(sofa_amd_engine eng, int enable);
 /* FP64_TILED engines in the reference's summation order (set before the scenes are placed): how
  * each scene's node-after-node dot product (|b|^2, p.q, r.r) is computed.  segments = 1: one
  * single-wave chain of dependent adds per scene.  segments = 2, 4, 8 (default) or 16 (with a
- * window of 32 at most): the chain's
- * segments run at once, each segment after the first from 2 `window` candidate start values
- * (consecutive doubles around a prediction of the sum before it: the terms each rounded as the
- * chain would round them; window 0, 32, 64, 96 or 128, default 32), and the sum is then resolved
- * boundary by boundary: the candidate equal to the
- * sum so far, bit for bit, continues it; where none is, the segment is summed from the sum so
- * far (counted in sofa_amd_cg_stats::dot_fallbacks).  Every add of the chain happens in the
- * reference's order on its exact operands: the result has the same bits either way.  Scenes
- * under 8192 nodes always use the single chain.  No reference counterpart. */
+ * window of 32 at most) with a window of 32 (default), 64, 96 or 128: the sum by exact parallel
+ * rounding (terms rounded to the grid of the running sum's binade add up in any order; what that
+ * rule does not cover is added one after the other), whatever the two numbers; with a window of
+ * 0: the chain, each of the segments - 1 boundaries of a scene of 8192 nodes or more counted in
+ * sofa_amd_cg_stats::dot_fallbacks.  Every result is the reference's chain's, bit for bit.  No
+ * reference counterpart. */
 int sofa_amd_engine_set_dot_segments(sofa_amd_engine eng, int segments, int window);
 
 /* SOFA_AMD_FP64 and SOFA_AMD_FP64_TILED engines: order of the sums.  0 (default): CG dot

@@ -465,8 +465,8 @@ class Engine:
         check(lib().sofa_amd_engine_set_branches(self._h, int(branches)))
 
     def set_dot_segments(self, segments, window=32):
-        """Reference-order dot products in `segments` segments run at once (1: the single chain),
-        from 2 `window` candidate starts per boundary."""
+        """Reference-order dot products by exact parallel rounding (segments > 1 with a window) or by
+        the single chain of dependent adds (segments 1, or window 0); the same bits."""
         check(lib().sofa_amd_engine_set_dot_segments(self._h, int(segments), int(window)))
 
     def set_branch_turns(self, enable):

@@ -31,6 +31,7 @@
 #include "sofa_amd.h"
 #include "fem_kernels.h"
 #include "fem_tiled.h"
+#include "fem_dots.h"
 #include "fem_mixed.h"
 #include "tiling.h"
 
@@ -395,9 +396,6 @@ struct EngineT : EngineBase {
     std::vector<std::vector<int>> iperm;           // per scene: original element -> position
     VT* p2 = nullptr;                              // previous CG direction (exact path)
     double* nd = nullptr;                          // per-node dot terms (exact path, reference order)
-    double* spec_part = nullptr;                   // segmented reference-order dots: prediction chunks
-    double* spec_model = nullptr;                  // ... with the chain's roundings modelled
-    double* spec_seg = nullptr;                    // ... and the segments' candidate sums
     double* pinv = nullptr;                        // PCG: inverted preconditioner block per node (9)
     VT* zv = nullptr;                              // PCG: preconditioned residual z = P^-1 r
     int *em_ptr = nullptr, *em_nbr = nullptr;      // MeshMatrixMass edges per node (exact path)
@@ -490,7 +488,7 @@ struct EngineT : EngineBase {
                         ln_inc, sp0, sp1, pbb, pden, prho, p2, em_ptr, em_nbr, em_val, emass, osc_node,
                         osc_mean, osc_amp, osc_w, osc_phase, kmat32, emass32, r32, p32, q32,
                         d32, sp32, pden32, prho32, prr, inst_in, sh_of, nd, x0, x32, x0_32, contact, inc_rank, pinv, zv,
-                        inc_arank, sh_acnt, ln_lead, dinv32, binv32, z32, spec_part, spec_model, spec_seg};
+                        inc_arank, sh_acnt, ln_lead, dinv32, binv32, z32};
         for (void* ptr : ptrs)
             if (ptr) (void)hipFree(ptr);
     }
@@ -963,7 +961,6 @@ struct EngineT : EngineBase {
         r32 = p32 = q32 = d32 = sp32 = nullptr; pden32 = prho32 = prr = nullptr; inst_in = nullptr; sh_of = nullptr; inc_rank = nullptr;
         pinv = nullptr; zv = nullptr; inc_arank = nullptr; sh_acnt = nullptr; ln_lead = nullptr; dinv32 = nullptr;
         binv32 = z32 = nullptr;
-        spec_part = spec_model = spec_seg = nullptr;
         cap = c;
         if (cap.node >= (int64_t)1 << 30 || cap.inc >= (int64_t)1 << 31 || cap.lnode >= (int64_t)1 << 31 ||
             cap.slot >= (int64_t)kSlotOwner)
@@ -1002,11 +999,6 @@ struct EngineT : EngineBase {
         osc_node = dalloc<int>(cap.osc); osc_mean = dalloc<double>(3 * cap.osc); osc_amp = dalloc<double>(3 * cap.osc);
         osc_w = dalloc<double>(cap.osc); osc_phase = dalloc<double>(cap.osc);
         inst = dalloc<InstDev>(cap.sid); ranges_d = dalloc<Ranges>(cap.sid);
-        if (seq_dots && !mixed && std::is_same<R, double>::value) {   // segmented reference-order dots
-            spec_part = dalloc<double>((size_t)std::max<int64_t>(1, cap.sid) * kSpecChunks);
-            spec_model = dalloc<double>((size_t)std::max<int64_t>(1, cap.sid) * kSpecChunks);
-            spec_seg = dalloc<double>((size_t)std::max<int64_t>(1, cap.sid) * kSpecStride);
-        }
         for (double* pb : {pbb, pden}) HIPCHK(hipMemset(pb, 0, std::max<size_t>(1, np) * sizeof(double)));
         HIPCHK(hipMemset(prho, 0, std::max<int64_t>(1, cap.nblk) * sizeof(double)));
         if (mixed) {
@@ -1440,21 +1432,14 @@ struct EngineT : EngineBase {
                                                           pden, prho, contact, nd);
         launch_seqdot(n, s, kDotRR);
     }
-    // a reference-order dot product of the launch set's n scenes into InstDev::dots[which]: the
-    // single chain per scene (k_seqdot), or the chain in dot_segments segments run at once from
-    // 2 dot_window candidate starts per boundary (k_seqdot_part / _model / _spec / _resolve, the
-    // same bits)
-    static constexpr int kSpecMinNodes = 8192;   // smaller scenes: the single chain (under 40 us)
-    void launch_seqdot(int n, hipStream_t s, int which) {
-        if (spec_seg && dot_segments > 1) {
-            const SpecDots sd{spec_part, spec_model, spec_seg, dot_segments, dot_window / 32, kSpecMinNodes};
-            k_seqdot_part<<<n * kSpecChunks, 64, 0, s>>>(cur->scenes, inst, nd, sd);
-            k_seqdot_model<<<n * kSpecChunks, 64, 0, s>>>(cur->scenes, inst, nd, sd);
-            k_seqdot_spec<<<n * (1 + (sd.K - 1) * sd.W), 64, 0, s>>>(cur->scenes, inst, nd, sd, which);
-            k_seqdot_resolve<<<n, 64, 0, s>>>(cur->scenes, inst, nd, sd, which);
-        } else {
-            k_seqdot<<<n, 64, 0, s>>>(cur->scenes, inst, nd, which);
-        }
+    // a reference-order dot product of the launch set's n scenes into InstDev::dots[which]: by
+    // exact parallel rounding (k_scandot), or, asked for (one segment, or a window of 0), by the
+    // single chain of dependent adds per scene (k_seqdot; the same bits)
+    void launch_seqdot(int n, hipStream_t s, int which, bool step = true) {
+        if (dot_segments > 1 && dot_window > 0)
+            k_scandot<<<n, kScanThreads, 0, s>>>(cur->scenes, inst, nd, which);
+        else
+            k_seqdot<<<n, 64, 0, s>>>(cur->scenes, inst, nd, which, step ? dot_segments - 1 : 0);
     }
     // the Euler update and the step's end
     void exact_close(int n, hipStream_t s) {
@@ -1989,7 +1974,7 @@ struct EngineT : EngineBase {
               hipStream_t s) override {
         const int n = scenes[scene].n_nodes;
         if (order == 1) {
-            k_vdot_seq<VT><<<1, 64, 0, s>>>((const VT*)a, (const VT*)b, n, out);
+            k_vdot_seq<VT><<<1, kScanThreads, 0, s>>>((const VT*)a, (const VT*)b, n, out);
         } else {
             const int nb = (n + kBlock - 1) / kBlock;
             if (nb > scratch_len) throw std::length_error("vDot: scene larger than the scratch buffer");
@@ -2046,16 +2031,16 @@ struct EngineT : EngineBase {
                 if constexpr (std::is_same<R, double>::value) {
                     if (cur->nc > 0)
                         k_cg_begin_tiled<VT, true><<<cur->nc, kBlock, 0, s>>>(nbk, (const VT*)bvec, nb0, b, r, xcg, prho, nd);
-                    k_seqdot<<<1, 64, 0, s>>>(cur->scenes, inst, nd, kDotBB);
+                    launch_seqdot(1, s, kDotBB, false);
                     for (int it = 1; it <= cur->maxit; it++) {
                         if (cur->na > 0) launch_apply(cur->na, s, ta, it, r, p, q, sp0, nullptr, pden, 0);
                         if (cur->nb > 0)
                             k_fin_exact<VT><<<cur->nb, kBlock, 0, s>>>(fb, inst, sn, mass, fixed, it, r, p, q, sp0, nd, contact);
-                        k_seqdot<<<1, 64, 0, s>>>(cur->scenes, inst, nd, kDotPQ);
+                        launch_seqdot(1, s, kDotPQ, false);
                         if (cur->nc > 0)
                             k_update<VT, true><<<cur->nc, kBlock, 0, s>>>(nbk, inst, ranges_d, it, sn, sp0, mass, fixed, p, q,
                                                                           xcg, r, pden, prho, contact, nd);
-                        k_seqdot<<<1, 64, 0, s>>>(cur->scenes, inst, nd, kDotRR);
+                        launch_seqdot(1, s, kDotRR, false);
                     }
                 }
             } else {
@@ -3233,9 +3218,9 @@ int sofa_amd_engine_set_dot_segments(sofa_amd_engine eng, int segments, int wind
     if (!eng || !eng->impl) return fail(SOFA_AMD_EINVAL, "null engine");
     if (segments != 1 && segments != 2 && segments != 4 && segments != 8 && segments != 16)
         return fail(SOFA_AMD_EINVAL, "segments must be 1, 2, 4, 8 or 16");
-    if (window < 0 || window > 32 * kSpecMaxWaves || window % 32 != 0)
+    if (window < 0 || window > 128 || window % 32 != 0)
         return fail(SOFA_AMD_EINVAL, "window must be 0, 32, 64, 96 or 128");
-    if (1 + (segments - 1) * (2 * window + 1) > kSpecStride)
+    if (segments == 16 && window > 32)
         return fail(SOFA_AMD_EINVAL, "16 segments take a window of 32 at most");
     HIPCHK(hipSetDevice(eng->impl->device));
     HIPCHK(hipDeviceSynchronize());

@@ -828,38 +828,7 @@ __global__ __launch_bounds__(kBlock) void k_oscillate_vec(Oscillators os, int o0
 }
 
 // BaseMechanicalState::vDot on caller vectors (MechanicalObject::vDot, MechanicalObject.inl
-// :2334-2356), in the reference's order: one wave computes each node's three-term dot product
-// and adds them node after node from 0.0 (the k_seqdot chain, terms formed on the fly; padding
-// with +0.0 leaves the sum unchanged)
-template <typename VT>
-__global__ __launch_bounds__(64) void k_vdot_seq(const VT* __restrict__ a, const VT* __restrict__ b, int n,
-                                                  double* __restrict__ out) {
-    __shared__ double buf[kSeqChunk];
-    const int lane = threadIdx.x;
-    constexpr int PER = kSeqChunk / 64;
-    double s = 0.0;
-    for (int base = 0; base < n; base += kSeqChunk) {
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int i = base + k * 64 + lane;
-            double t = 0.0;
-            if (i < n) {
-                VT x[3], y[3];
-                load3(a, i, x[0], x[1], x[2]);
-                load3(b, i, y[0], y[1], y[2]);
-                t = dot3d(x, y);
-            }
-            buf[k * 64 + lane] = t;
-        }
-        __syncthreads();
-#pragma unroll 64
-        for (int k = 0; k < kSeqChunk; k++) s = s + buf[k];
-        __syncthreads();
-    }
-    if (lane == 0) *out = s;
-}
-
-// the same dot product in the FP64 engine's parallel blocked order: per 256-node block the
+// :2334-2356) in the FP64 engine's parallel blocked order: per 256-node block the
 // fixed tree of block_sum, then the block partials added by one block as last_block_reduce
 // does (each thread a strided sum, then block_sum) -- the oracle's dot_blocked
 template <typename VT>
