@@ -186,6 +186,17 @@ static __global__ __launch_bounds__(64) void k_seqdot(const int* __restrict__ sc
     }
 }
 
+// The work item of this workgroup: consecutive items on one XCD.  Workgroups go to the 8 XCDs
+// round-robin, each XCD with its own L2, so item blockIdx.x would put every two neighbours of a mesh
+// (tiles or node blocks that read the same nodes and contributions) behind different L2s; here XCD
+// x takes the x-th eighth of the items.  Measured on the CG operator: 1.31M tets in FP32 35.4 -> 31.3 us,
+// 385k in FP64 29.5 -> 26.0, 930k over 24 scenes in FP32 27.2 -> 24.1; the untiled FP64 node kernel
+// 28.0 -> 25.7.
+__device__ __forceinline__ int xcd_item() {
+    const int n = (int)gridDim.x, x = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3;
+    return x * (n >> 3) + min(x, n & 7) + i;
+}
+
 struct Blk { int inst, begin, end, pad; };   // a block's scene and [begin, end) range
 
 // ---------------------------------------------------------------------------------------

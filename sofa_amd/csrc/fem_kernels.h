@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_elem(ElemView<R, NR> ev, const B
                                                       const InstDev* __restrict__ inst, const VT* __restrict__ x,
                                                       const VT* __restrict__ v, VT* __restrict__ ef_f,
                                                       VT* __restrict__ ef_v) {
-    const Blk bk = eblk[blockIdx.x];
+    const Blk bk = eblk[xcd_item()];
     const int64_t e = (int64_t)bk.begin + threadIdx.x;
     if (e >= bk.end) return;
     const InstDev& in = inst[bk.inst];
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_node(const Blk* __restrict__ nbl
                                                       double* __restrict__ nd,     // non-null: reference dot order
                                                       const VT* __restrict__ x) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     const int n = bk.begin + threadIdx.x;
     double bb = 0.0;
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_begin(const Blk* __restrict__ nbl
                                                       VT* __restrict__ r, VT* __restrict__ xcg,
                                                       double* __restrict__ partial, double* __restrict__ nd) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     const int n = bk.begin + threadIdx.x;
     double bb = 0.0;
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
                                                      const InstDev* __restrict__ inst, const VT* __restrict__ r_,
                                                      const VT* __restrict__ p_old, VT* __restrict__ ef,
                                                      const VT* __restrict__ z = nullptr) {
-    const Blk bk = eblk[blockIdx.x];
+    const Blk bk = eblk[xcd_item()];
     const InstDev& in = inst[bk.inst];
     if (in.stopped) return;
     // PCG: the direction is built from the preconditioned residual z (w = z + beta w)
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_node(const Blk* __restrict__ nblk
                                                      double* __restrict__ partial, double* __restrict__ nd,
                                                      const VT* __restrict__ z = nullptr) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     if (ins->stopped) return;
     const VT* __restrict__ r = (ins->pcg && z) ? z : r_;
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(const Blk* __restrict__ nb
                                                        const double* __restrict__ pinv = nullptr,
                                                        VT* __restrict__ z = nullptr) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     if (ins->stopped) return;
     const int n = bk.begin + threadIdx.x;
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(kBlock) void k_euler_update(const Blk* __restrict__
                                                           const int8_t* __restrict__ fixed,
                                                           const VT* __restrict__ xcg, VT* __restrict__ v,
                                                           VT* __restrict__ x) {
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     const int n = bk.begin + threadIdx.x;
     if (n >= bk.end) return;
     // MechanicalObject::vMultiOp fast path (MechanicalObject.inl:2209-2230): v += dv (firstOrder:
@@ -1191,7 +1191,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_diag(ElemView<R, NR> ev, const B
                                                       const InstDev* __restrict__ inst, const int* __restrict__ inc_ptr,
                                                       const int* __restrict__ inc, const double* __restrict__ mass,
                                                       const int8_t* __restrict__ fixed, double* __restrict__ pinv) {
-    const BLK bk = nblk[blockIdx.x];
+    const BLK bk = nblk[xcd_item()];
     const InstDev& in = inst[blk_scene(bk)];
     if (!in.pcg) return;
     for (int n = bk.begin + threadIdx.x; n < bk.end; n += kBlock)
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_begin(const Blk* __restrict__ nb
                                                        const double* __restrict__ pinv, double* __restrict__ partial,
                                                        double* __restrict__ nd) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     if (!ins->pcg || ins->stopped) return;
     const int n = bk.begin + threadIdx.x;
@@ -1301,7 +1301,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_warm_begin(const Blk* __restrict_
                                                            VT* __restrict__ r, double* __restrict__ partial,
                                                            double* __restrict__ nd) {
     __shared__ double sh[kBlock];
-    const Blk bk = nblk[blockIdx.x];
+    const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     if (!ins->warm_start || ins->pcg || ins->stopped) return;
     const int n = bk.begin + threadIdx.x;

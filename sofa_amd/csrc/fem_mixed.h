@@ -30,7 +30,7 @@ static __global__ __launch_bounds__(kBlock) void k_ir_residual(const NodeBlk* __
                                                                 const float* __restrict__ binv,
                                                                 float* __restrict__ zbuf) {
     __shared__ double sh[kBlock / 64];
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     if (inst[nb.scene].stopped) return;
     double rr = 0.0, rr32 = 0.0;
 #pragma unroll
@@ -115,7 +115,7 @@ static __global__ __launch_bounds__(kBlock) void k_ir_control(const int* __restr
 static __global__ __launch_bounds__(kBlock) void k_ir_accumulate(const NodeBlk* __restrict__ nb_, InstDev* __restrict__ inst,
                                                                   InstDev* __restrict__ inner,
                                                                   const float* __restrict__ d32, double* __restrict__ x) {
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     InstDev* o = &inst[nb.scene];
     if (o->stopped) return;
     if (nb.first && threadIdx.x == 0) {
@@ -145,7 +145,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi32(ElemView<R, NR> ev, const N
                                                       const int* __restrict__ inc, const double* __restrict__ mass,
                                                       const int8_t* __restrict__ fixed, float* __restrict__ dinv,
                                                       float* __restrict__ binv) {
-    const NodeBlk bk = nblk[blockIdx.x];
+    const NodeBlk bk = nblk[xcd_item()];
     const InstDev& in = inst[bk.scene];
     if (!in.pcg) return;   // z = r: neither array is read
     for (int n = bk.begin + threadIdx.x; n < bk.end; n += kBlock) {

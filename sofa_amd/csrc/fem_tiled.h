@@ -317,7 +317,7 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
     __shared__ uint16_t linc[kTileElems * 4];
     __shared__ int lptr[kTileNodes + 1];
     __shared__ double sh[TB / 64];
-    const TileDesc td = a.tiles[blockIdx.x];
+    const TileDesc td = a.tiles[xcd_item()];
     const InstDev& in = a.inst[td.scene];
     // element records of this thread's elements, in registers for both passes
     R rin[EPT][NR], kk[EPT][3], em[EPT], rot[EPT][9];
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
                                                      const VT* __restrict__ x, int8_t* __restrict__ contact,
                                                      double* __restrict__ nd = nullptr) {
     __shared__ double sh[kBlock / 64];
-    const FinBlk fb = fb_[blockIdx.x];
+    const FinBlk fb = fb_[xcd_item()];
     const InstDev& in = inst[fb.scene];
     const int j = fb.begin + threadIdx.x;
     double bb = 0.0;
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     __shared__ uint16_t linc[kTileElems * 4];
     __shared__ int lptr[kTileNodes + 1];
     __shared__ double sh[TB / 64];
-    const TileDesc td = a.tiles[blockIdx.x];
+    const TileDesc td = a.tiles[xcd_item()];
     const bool consistent = (td.flags & kTileConsistent) != 0;
     const bool kvol = GEO == 2 && (td.flags & kTileOneMaterial) != 0;   // K recomputed, not loaded
     // ---- 1. issue every load that depends on the tile descriptor only: the element records of
@@ -856,7 +856,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_exact(const FinBlk* __restrict__
                                                        const VT* __restrict__ r, VT* __restrict__ p,
                                                        VT* __restrict__ q, const VT* __restrict__ sp,
                                                        double* __restrict__ nd, const int8_t* __restrict__ contact) {
-    const FinBlk fb = fb_[blockIdx.x];
+    const FinBlk fb = fb_[xcd_item()];
     const InstDev& in = inst[fb.scene];
     if (in.stopped) return;
     const int j = fb.begin + threadIdx.x;
@@ -892,7 +892,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_begin_exact(const NodeBlk* __re
                                                               const InstDev* __restrict__ inst,
                                                               const VT* __restrict__ b, const VT* __restrict__ q,
                                                               VT* __restrict__ r, double* __restrict__ nd) {
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     const InstDev& in = inst[nb.scene];
     if (!in.warm_start || in.stopped) return;
     const VT m1 = (VT)(-1.0);
@@ -921,7 +921,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_apply(const FinBlk* __restrict__
                                                        double* __restrict__ pden,
                                                        const int8_t* __restrict__ contact) {
     __shared__ double sh[kBlock / 64];
-    const FinBlk fb = fb_[blockIdx.x];
+    const FinBlk fb = fb_[xcd_item()];
     const InstDev& in = inst[fb.scene];
     if (in.stopped) return;
     const int j = fb.begin + threadIdx.x;
@@ -996,7 +996,7 @@ __global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ n
                                                     const float* __restrict__ dinv = nullptr,
                                                     const float* __restrict__ binv = nullptr, VT* __restrict__ zbuf = nullptr) {
     __shared__ double sh[kBlock / 64];
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     InstDev* ins = &inst[nb.scene];
     // node data first (registers), then the reduction
     VT pv[kNodesPerThread][3], qv[kNodesPerThread][3], xv[kNodesPerThread][3], rv[kNodesPerThread][3];
@@ -1091,7 +1091,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_begin_tiled(const NodeBlk* __rest
                                                             VT* __restrict__ xcg, double* __restrict__ prho,
                                                             double* __restrict__ nd) {
     __shared__ double sh[kBlock / 64];
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     double bb = 0.0;
 #pragma unroll
     for (int k = 0; k < kNodesPerThread; k++) {
@@ -1117,7 +1117,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate(const NodeBlk* __restrict_
                                                        const int8_t* __restrict__ fixed,
                                                        const VT* __restrict__ xcg, VT* __restrict__ v,
                                                        VT* __restrict__ x) {
-    const NodeBlk nb = nb_[blockIdx.x];
+    const NodeBlk nb = nb_[xcd_item()];
     const InstDev& in = inst[nb.scene];
     const VT h = (VT)in.dt;
     // v += dv (firstOrder: v = dv), x += v h, then vdamping's v *= exp(-h d)
