@@ -89,11 +89,51 @@ template <typename VT, typename F>
 __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double factor, F dof, VT out[3]) {
     const int s0 = na.em_ptr[n], s1 = na.em_ptr[n + 1];
     const VT fct = (VT)factor;
-    for (int s = s0; s < s1; s++) {
-        const VT tm = (VT)na.em_val[s] * fct;
-        VT d[3];
-        dof(na.em_nbr[s], d);
-        out[0] += d[0] * tm; out[1] += d[1] * tm; out[2] += d[2] * tm;
+    constexpr int B = 4;                       // edges loaded together (gather_contributions)
+    for (int s = s0; s < s1; s += B) {
+        int nbr[B];
+        VT tm[B], d[B][3];
+#pragma unroll
+        for (int t = 0; t < B; t++) {
+            const int i = min(s + t, s1 - 1);
+            nbr[t] = na.em_nbr[i];
+            tm[t] = (VT)na.em_val[i] * fct;
+        }
+#pragma unroll
+        for (int t = 0; t < B; t++) dof(nbr[t], d[t]);
+#pragma unroll
+        for (int t = 0; t < B; t++)
+            if (s + t < s1) {
+                out[0] += d[t][0] * tm[t]; out[1] += d[t][1] * tm[t]; out[2] += d[t][2] * tm[t];
+            }
+    }
+}
+
+// acc (+|-)= the node's element contributions ef[3 slot ..] over its incidence list [s0, s1), in
+// list order.  Eight incidences at a time: their slots, then their values, are loaded together (the
+// tail at clamped indices), so a node of 24 tetrahedra waits for memory 6 times instead of 48.
+// Latency is what bounds the node kernels (one lane a node, 250 waves for 16,000 nodes): the CG
+// node kernel takes MEASURED.
+template <bool SUB, typename VT>
+__device__ __forceinline__ void gather_contributions(const int* __restrict__ inc, int s0, int s1,
+                                                     const VT* __restrict__ ef, VT acc[3]) {
+    constexpr int B = 8;
+    for (int s = s0; s < s1; s += B) {
+        int slot[B];
+        VT c[B][3];
+#pragma unroll
+        for (int t = 0; t < B; t++) slot[t] = inc[min(s + t, s1 - 1)];
+#pragma unroll
+        for (int t = 0; t < B; t++) load3(ef, slot[t], c[t][0], c[t][1], c[t][2]);
+#pragma unroll
+        for (int t = 0; t < B; t++)
+            if (s + t < s1) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    if (SUB) acc[i] -= c[t][i];
+                    else acc[i] += c[t][i];
+                }
+            }
     }
 }
 
@@ -240,10 +280,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_node(const Blk* __restrict__ nbl
         VT fn[3];
         mass_gravity(in, na.mass, n, fn);
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = na.inc[s];
-            fn[0] += ef_f[3 * slot]; fn[1] += ef_f[3 * slot + 1]; fn[2] += ef_f[3 * slot + 2];
-        }
+        gather_contributions<false>(na.inc, s0, s1, ef_f, fn);
         // PlaneForceField after the FEM (scene order); its contacts are kept for addDForce
         const bool touch = in.plane_on && plane_force(in, xn, vn, fn);
         if (in.plane_on) na.contact[n] = touch ? 1 : 0;
@@ -257,10 +294,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_node(const Blk* __restrict__ nbl
             if (in.mass_kind == kMassMatrix)
                 mass_edges(na, n, in.m_rhs, [&](int j, VT d[3]) { load3(v, j, d[0], d[1], d[2]); }, bn);
         }
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = na.inc[s];
-            bn[0] -= ef_v[3 * slot]; bn[1] -= ef_v[3 * slot + 1]; bn[2] -= ef_v[3 * slot + 2];
-        }
+        gather_contributions<true>(na.inc, s0, s1, ef_v, bn);
         if (touch && in.k_rhs != 0.0) plane_dforce(in, in.k_rhs, vn, bn);
         const VT h = (VT)in.b_scale;   // h (firstOrder: 1, b = f)
         bn[0] *= h; bn[1] *= h; bn[2] *= h;
@@ -391,10 +425,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_node(const Blk* __restrict__ nblk
             if (in.mass_kind == kMassMatrix) mass_edges(na, n, in.m_cg, pdir, qn);
         }
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = na.inc[s];
-            qn[0] -= ef[3 * slot]; qn[1] -= ef[3 * slot + 1]; qn[2] -= ef[3 * slot + 2];
-        }
+        gather_contributions<true>(na.inc, s0, s1, ef, qn);
         if (in.plane_on && na.contact[n]) plane_dforce(in, in.k_cg, pn, qn);
         if (na.fixed[n]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
         q[o] = qn[0]; q[o + 1] = qn[1]; q[o + 2] = qn[2];
@@ -712,17 +743,8 @@ __global__ __launch_bounds__(kBlock) void k_gather(const int* __restrict__ inc_p
     const int64_t o = 3 * (int64_t)(n - n0);
     VT a[3] = {out[o], out[o + 1], out[o + 2]};
     const int s0 = inc_ptr[n], s1 = inc_ptr[n + 1];
-    if (subtract) {
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = inc[s];
-            a[0] -= ef[3 * slot]; a[1] -= ef[3 * slot + 1]; a[2] -= ef[3 * slot + 2];
-        }
-    } else {
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = inc[s];
-            a[0] += ef[3 * slot]; a[1] += ef[3 * slot + 1]; a[2] += ef[3 * slot + 2];
-        }
-    }
+    if (subtract) gather_contributions<true>(inc, s0, s1, ef, a);
+    else gather_contributions<false>(inc, s0, s1, ef, a);
     out[o] = a[0]; out[o + 1] = a[1]; out[o + 2] = a[2];
 }
 
@@ -1253,10 +1275,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_begin(const Blk* __restrict__ nb
                 mass_edges(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
         }
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = na.inc[s];
-            qn[0] -= ef[3 * slot]; qn[1] -= ef[3 * slot + 1]; qn[2] -= ef[3 * slot + 2];
-        }
+        gather_contributions<true>(na.inc, s0, s1, ef, qn);
         if (in.plane_on && na.contact[n]) plane_dforce(in, in.k_cg, xn, qn);
         if (na.fixed[n]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
         VT rn[3], zn[3];
@@ -1318,10 +1337,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_warm_begin(const Blk* __restrict_
                 mass_edges(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
         }
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
-        for (int s = s0; s < s1; s++) {
-            const int64_t slot = na.inc[s];
-            qn[0] -= ef[3 * slot]; qn[1] -= ef[3 * slot + 1]; qn[2] -= ef[3 * slot + 2];
-        }
+        gather_contributions<true>(na.inc, s0, s1, ef, qn);
         if (in.plane_on && na.contact[n]) plane_dforce(in, in.k_cg, xn, qn);
         if (na.fixed[n]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
         VT rn[3];
