@@ -407,7 +407,7 @@ struct EngineT : EngineBase {
     InstDev* inst = nullptr;
     // exact path: block lists of every scene, reduction partials
     std::vector<Blk> eblk_h, nblk_h;
-    double* partial = nullptr;
+    double *partial = nullptr, *partial2 = nullptr;   // r.r (and |b|^2), p.q per node block
     // tiled path: device tables, partial buffers
     TileDesc* tiles_d = nullptr;
     Ranges* ranges_d = nullptr;
@@ -453,7 +453,7 @@ struct EngineT : EngineBase {
         void *a = nullptr, *b = nullptr, *c = nullptr, *o = nullptr, *l = nullptr;
         int* scenes = nullptr;          // scene record indices
         int na = 0, nb = 0, nc = 0, no = 0, nl = 0, maxit = 0, maxsw = 0, n = 0;
-        int maxpart = 0;                // most partial sums the operator reduces for one scene
+        int maxpart = 0;                // most partial sums the operator (untiled: any kernel) reduces for one scene
         bool plane = false;             // some scene has a PlaneForceField
         bool pcg = false;               // some scene solves with PCGLinearSolver
         bool warm = false;              // some scene's CGLinearSolver has warmStart
@@ -484,7 +484,7 @@ struct EngineT : EngineBase {
     }
     void free_device() {
         void* ptrs[] = {x, v, f, b, r, p, q, xcg, mass, fixed, inc_ptr, inc, tet, rot, rest, kmat, ef, ef2,
-                        inst, partial, tiles_d, ranges_d, ltet, ln_gid, ln_inc_ptr, ln_pslot, sh_gid, sh_ptr,
+                        inst, partial, partial2, tiles_d, ranges_d, ltet, ln_gid, ln_inc_ptr, ln_pslot, sh_gid, sh_ptr,
                         ln_inc, sp0, sp1, pbb, pden, prho, p2, em_ptr, em_nbr, em_val, emass, osc_node,
                         osc_mean, osc_amp, osc_w, osc_phase, kmat32, emass32, r32, p32, q32,
                         d32, sp32, pden32, prho32, prr, inst_in, sh_of, nd, x0, x32, x0_32, contact, inc_rank, pinv, zv,
@@ -886,6 +886,8 @@ struct EngineT : EngineBase {
         upload(inst, inst_h);
         partial = dalloc<double>(nblk_h.size());
         HIPCHK(hipMemset(partial, 0, std::max<size_t>(1, nblk_h.size()) * sizeof(double)));
+        partial2 = dalloc<double>(nblk_h.size());
+        HIPCHK(hipMemset(partial2, 0, std::max<size_t>(1, nblk_h.size()) * sizeof(double)));
         HIPCHK(hipDeviceSynchronize());
     }
 
@@ -955,7 +957,7 @@ struct EngineT : EngineBase {
         x = v = f = b = r = p = q = xcg = x0 = nullptr; mass = nullptr; fixed = nullptr; contact = nullptr; inc_ptr = inc = nullptr;
         tet = nullptr; rot = rest = kmat = nullptr; ef = ef2 = nullptr; p2 = nullptr; em_ptr = em_nbr = nullptr;
         em_val = nullptr; emass = nullptr; osc_node = nullptr; osc_mean = osc_amp = osc_w = osc_phase = nullptr;
-        inst = nullptr; partial = nullptr; tiles_d = nullptr; ranges_d = nullptr; ltet = nullptr;
+        inst = nullptr; partial = partial2 = nullptr; tiles_d = nullptr; ranges_d = nullptr; ltet = nullptr;
         ln_gid = ln_inc_ptr = ln_pslot = sh_gid = sh_ptr = nullptr; ln_inc = nullptr; sp0 = sp1 = nullptr;
         pbb = pden = prho = nullptr; kmat32 = emass32 = nullptr; x32 = x0_32 = nullptr;
         r32 = p32 = q32 = d32 = sp32 = nullptr; pden32 = prho32 = prr = nullptr; inst_in = nullptr; sh_of = nullptr; inc_rank = nullptr;
@@ -1277,6 +1279,7 @@ struct EngineT : EngineBase {
                 const SceneHost& sc = scenes[id];
                 push_range(eb, eblk_h, sc.eblk_begin, sc.eblk_count);
                 push_range(nb, nblk_h, sc.nblk_begin, sc.nblk_count);
+                ls->maxpart = std::max(ls->maxpart, sc.nblk_count);
                 ls->pcg = ls->pcg || sc.precond != 0;
                 ls->warm = ls->warm || (sc.warm_start && sc.precond == 0);
                 maxit = std::max(maxit, sc.cg_iter);
@@ -1346,30 +1349,53 @@ struct EngineT : EngineBase {
                 k_pcg_diag<R, NR, Blk><<<cur->nb, kBlock, 0, s>>>(ev, nb, inst, na.inc_ptr, na.inc, mass, fixed, pinv);
             if (cur->nl > 0) k_pcg_lm_identity<<<cur->nl, kBlock, 0, s>>>((const Blk*)cur->l, inst, pinv);
             k_pcg_open<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
-            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, xcg, p2, ef);
+            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, xcg, p2, ef, 1, partial, 0);
             if (cur->nb > 0) k_pcg_begin<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, na, ef, xcg, b, r, zv, pinv, partial, ndp);
         }
         if (cur->warm) {
             // CGLinearSolver warmStart: r = b - A x from the previous solution (other scenes of the
             // set pass through untouched)
             k_warm_open<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
-            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, xcg, p2, ef);
+            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, xcg, p2, ef, 1, partial, 0);
             if (cur->nb > 0) k_cg_warm_begin<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, na, ef, xcg, b, r, partial, ndp);
         }
+        iterate_exact(ev, na, n, s, pinv, zv);
+        if (cur->nb > 0) k_euler_update<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, fixed, xcg, v, x);
+        if (cur->no > 0) k_oscillate<VT><<<cur->no, kBlock, 0, s>>>((const Blk*)cur->o, inst, oscillators(), x, v);
+        if (cur->nl > 0) k_lm_project<VT><<<cur->nl, kBlock, 0, s>>>((const Blk*)cur->l, inst, x, v);
+        k_finalize<true><<<n, kBlock, 0, s>>>(cur->scenes, inst, partial, exact_ready());
+    }
+
+    // the CG iterations of the untiled engine on the current launch set's n scenes: the dot products'
+    // partials are added by the kernel that needs them, or first brought to the scene records: in the
+    // reference's order (k_scandot), or when a scene has more than kSumBlocks node blocks, where every
+    // block adding all of them costs more than a launch (131,072 nodes: 512 partials read by each of
+    // 2,400 element blocks)
+    static constexpr int kSumBlocks = 512;
+    int exact_ready() const { return seq_dots || cur->maxpart > kSumBlocks ? 1 : 0; }
+    void exact_total(int n, hipStream_t s, const double* part, int which) {
+        if (seq_dots) k_scandot<<<n, kScanThreads, 0, s>>>(cur->scenes, inst, nd, which);
+        else if (cur->maxpart > kSumBlocks) k_cg_total<<<n, kBlock, 0, s>>>(cur->scenes, inst, part, which);
+    }
+    void iterate_exact(const ElemView<R, NR>& ev, const NodeArrays& na, int n, hipStream_t s, const double* pi, VT* zi) {
+        const Blk* eb = (const Blk*)cur->a;
+        const Blk* nb = (const Blk*)cur->b;
+        double* ndp = seq_dots ? nd : nullptr;
+        const int ready = exact_ready();
         for (int it = 1; it <= cur->maxit; it++) {
             // direction of iteration it in buffer it & 1, the previous one in the other
             VT* p_new = (it & 1) ? p : p2;
             const VT* p_old = (it & 1) ? p2 : p;
-            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, r, p_old, ef, zv);
+            if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, r, p_old, ef, it, partial, ready, zi);
             if (cur->nb > 0) {
-                k_cg_node<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, na, ef, r, p_old, p_new, q, partial, ndp, zv);
-                k_cg_update<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, p_new, q, xcg, r, partial, ndp, pinv, zv);
+                k_cg_node<VT><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, na, ef, r, p_old, p_new, q, it, partial, ready,
+                                                               partial2, ndp, zi);
+                exact_total(n, s, partial2, kDotPQ);
+                k_cg_update<VT><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, p_new, q, xcg, r, it, partial2, ready, partial, ndp,
+                                                                 pi, zi);
+                exact_total(n, s, partial, kDotRR);
             }
         }
-        if (cur->nb > 0) k_euler_update<VT><<<cur->nb, kBlock, 0, s>>>(nb, inst, fixed, xcg, v, x);
-        if (cur->no > 0) k_oscillate<VT><<<cur->no, kBlock, 0, s>>>((const Blk*)cur->o, inst, oscillators(), x, v);
-        if (cur->nl > 0) k_lm_project<VT><<<cur->nl, kBlock, 0, s>>>((const Blk*)cur->l, inst, x, v);
-        k_finalize<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
     }
 
     // the reference's summation order on the tiled kernels (FP64 tiled engines, chosen before
@@ -2006,20 +2032,11 @@ struct EngineT : EngineBase {
         if (!tiled) {
             const ElemView<R, NR> ev = view();
             const NodeArrays na = nodes();
-            const Blk* eb = (const Blk*)cur->a;
             const Blk* nbk = (const Blk*)cur->b;
             double* ndp = seq_dots ? nd : nullptr;
             if (cur->nb > 0) k_cg_begin<VT><<<cur->nb, kBlock, 0, s>>>(nbk, inst, (const VT*)bvec, nb0, b, r, xcg, partial, ndp);
-            for (int it = 1; it <= cur->maxit; it++) {
-                VT* p_new = (it & 1) ? p : p2;
-                const VT* p_old = (it & 1) ? p2 : p;
-                if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, r, p_old, ef);
-                if (cur->nb > 0) {
-                    k_cg_node<VT><<<cur->nb, kBlock, 0, s>>>(nbk, inst, na, ef, r, p_old, p_new, q, partial, ndp);
-                    k_cg_update<VT><<<cur->nb, kBlock, 0, s>>>(nbk, inst, p_new, q, xcg, r, partial, ndp);
-                }
-            }
-            k_solve_end<<<1, 64, 0, s>>>(cur->scenes, 1, inst, 0);
+            iterate_exact(ev, na, 1, s, nullptr, nullptr);
+            k_finalize<false><<<1, kBlock, 0, s>>>(cur->scenes, inst, partial, exact_ready());
         } else {
             const TileArgs<R, NR> ta = tile_args();
             const FinBlk* fb = (const FinBlk*)cur->b;
@@ -2053,7 +2070,7 @@ struct EngineT : EngineBase {
                                                                 pden, prho, contact);
                 }
             }
-            k_solve_end<<<1, 64, 0, s>>>(cur->scenes, 1, inst, 1);
+            k_solve_end<<<1, 64, 0, s>>>(cur->scenes, 1, inst);
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(xvec, xcg + 3 * (int64_t)nb0, 3 * (size_t)n * sizeof(VT), hipMemcpyDeviceToDevice, s));

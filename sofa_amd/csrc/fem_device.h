@@ -45,7 +45,7 @@ struct InstDev {
     double k_cg, m_cg;                // -h(h + rs), 1 + h rm    (EulerImplicitSolver.cpp:169-171)
     double tol, thr;
     // CG scalars (CGLinearSolver.inl:86-270)
-    double normb, rho, rho_1, den, alpha, beta, err;
+    double normb, den, alpha, beta, err;
     int iter;                         // current nb_iter
     int stopped;                      // 1 once the loop has exited
     int end_reason;                   // 0 iterations, 1 tolerance, 2 threshold, 3 den==0, 4 |b|==0
@@ -55,7 +55,7 @@ struct InstDev {
     double time;
     unsigned int counter;             // arrivals of the current reduction (exact path)
     int pad_;
-    double rho_slot[2];               // rho of iterations k-1 and k (tiled path), by k & 1
+    double rho_slot[2];               // rho of iterations k-1 and k, by k & 1
     // iterative refinement (MIXED engines; the scene record of the inner FP32 CG is separate)
     int max_sweeps;                   // inner solves per step at most
     int ir_sweeps;                    // inner solves done in the last step
@@ -668,6 +668,14 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
     const double r = sh[0];
     __syncthreads();
     return r;
+}
+
+// v of the lane CTRL names within the row of 16, 0.0 where there is none
+template <int CTRL>
+__device__ __forceinline__ double dpp_row_from(double v) {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
 }
 
 // returns true in every thread of the last-arriving block of scene `ins`; `total` then holds

@@ -10,9 +10,9 @@
 //   k_rhs_node    f = m g + sum F; b = h (f - rm M v - (h+rs) K v); project;
 //                 r = b; x_cg = 0; |b| and rho = r.r                          (1 node pass)
 //   per CG iteration:
-//     k_cg_elem   p = r + beta p at the 4 gathered nodes; element K p        (1 element pass)
+//     k_cg_elem   beta; p = r + beta p at the 4 gathered nodes; element K p  (1 element pass)
 //     k_cg_node   p (owned node); q = (1 + h rm) M p - h(h+rs) K p; project; p.q
-//     k_cg_update x_cg += alpha p; r -= alpha q; r.r
+//     k_cg_update alpha; x_cg += alpha p; r -= alpha q; r.r
 //   k_euler_update  v += x_cg; x += h v
 //   k_finalize      time += dt, timeStepCount++
 // Node sums run over each node's incidence list in ascending element id: the order in which
@@ -83,16 +83,17 @@ __device__ __forceinline__ void mass_gravity(const InstDev& in, const double* __
 }
 
 // edge part of the consistent MeshMatrixMass addMDx (MeshMatrixMass.inl:2014-2026): for each
-// edge of node n in ascending edge id, out += d[other] * (edgeMass * factor); `dof(j, v)` gives
-// the value of the multiplied vector at node j
-template <typename VT, typename F>
-__device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double factor, F dof, VT out[3]) {
+// edge of node n in ascending edge id, out += d[other] * (edgeMass * factor); `dof(j, v)` gives the
+// NC components of the multiplied vector at node j.  Edges are loaded four at a time, as
+// gather_contributions does.
+template <int NC, typename VT, typename F>
+__device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double factor, F dof, VT out[NC]) {
     const int s0 = na.em_ptr[n], s1 = na.em_ptr[n + 1];
     const VT fct = (VT)factor;
-    constexpr int B = 4;                       // edges loaded together (gather_contributions)
+    constexpr int B = 4;
     for (int s = s0; s < s1; s += B) {
         int nbr[B];
-        VT tm[B], d[B][3];
+        VT tm[B], d[B][NC];
 #pragma unroll
         for (int t = 0; t < B; t++) {
             const int i = min(s + t, s1 - 1);
@@ -104,32 +105,35 @@ __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double f
 #pragma unroll
         for (int t = 0; t < B; t++)
             if (s + t < s1) {
-                out[0] += d[t][0] * tm[t]; out[1] += d[t][1] * tm[t]; out[2] += d[t][2] * tm[t];
+#pragma unroll
+                for (int i = 0; i < NC; i++) out[i] += d[t][i] * tm[t];
             }
     }
 }
 
-// acc (+|-)= the node's element contributions ef[3 slot ..] over its incidence list [s0, s1), in
-// list order.  Eight incidences at a time: their slots, then their values, are loaded together (the
-// tail at clamped indices), so a node of 24 tetrahedra waits for memory 6 times instead of 48.
-// Latency is what bounds the node kernels (one lane a node, 250 waves for 16,000 nodes): the CG
-// node kernel takes MEASURED.
-template <bool SUB, typename VT>
+// acc (+|-)= the NC components ef[3 slot ..] of the node's element contributions over its incidence
+// list [s0, s1), in list order.  Eight incidences at a time: their slots, then their values, are
+// loaded together (the tail at clamped indices), so a node of 24 tetrahedra waits for memory 6 times
+// instead of 48: latency is what bounds the node kernels (the CG node kernel, a lane per node, went
+// from 14.0 to 10.3 us on 525 nodes and from 25.7 to 21.7 on 57,000).
+template <bool SUB, int NC = 3, typename VT>
 __device__ __forceinline__ void gather_contributions(const int* __restrict__ inc, int s0, int s1,
-                                                     const VT* __restrict__ ef, VT acc[3]) {
+                                                     const VT* __restrict__ ef, VT acc[NC]) {
     constexpr int B = 8;
     for (int s = s0; s < s1; s += B) {
         int slot[B];
-        VT c[B][3];
+        VT c[B][NC];
 #pragma unroll
         for (int t = 0; t < B; t++) slot[t] = inc[min(s + t, s1 - 1)];
 #pragma unroll
-        for (int t = 0; t < B; t++) load3(ef, slot[t], c[t][0], c[t][1], c[t][2]);
+        for (int t = 0; t < B; t++)
+#pragma unroll
+            for (int i = 0; i < NC; i++) c[t][i] = ef[3 * (int64_t)slot[t] + i];
 #pragma unroll
         for (int t = 0; t < B; t++)
             if (s + t < s1) {
 #pragma unroll
-                for (int i = 0; i < 3; i++) {
+                for (int i = 0; i < NC; i++) {
                     if (SUB) acc[i] -= c[t][i];
                     else acc[i] += c[t][i];
                 }
@@ -164,14 +168,51 @@ __device__ __forceinline__ void precond_apply(int kind, const double* __restrict
     }
 }
 
+// mass_mdx for one component
+template <typename VT>
+__device__ __forceinline__ void mass_mdx_1(const InstDev& in, const double* __restrict__ mass, int n, double factor,
+                                           VT d, VT& out) {
+    if (in.mass_kind == kMassUniform) {
+        VT m = (VT)in.vertex_mass;
+        if (factor != 1.0) m *= (VT)factor;
+        out += d * m;
+    } else {
+        const VT m = (VT)mass[n], fct = (VT)factor;
+        if (in.mass_kind == kMassDiagonal && factor == 1.0) out += d * m;
+        else if (in.mass_kind == kMassMatrixLumped) out += ((d * m) * (VT)kLumpTet) * fct;
+        else out += (d * m) * fct;
+    }
+}
+
+// the end of a node kernel of three threads per node: each node's three products added in dot3d's
+// order, to nd (reference order) or, by block_sum's tree over the block's 256 nodes, to one partial
+__device__ __forceinline__ double tree_256(const double* sh);
+__device__ __forceinline__ void node_partial(const double* pr, double* sh, double* __restrict__ nd, const Blk& bk,
+                                             double* __restrict__ partial) {
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < kBlock) {
+        double v = pr[3 * t];
+        v += pr[3 * t + 1];
+        v += pr[3 * t + 2];
+        sh[t] = v;
+        if (nd && bk.begin + t < bk.end) nd[bk.begin + t] = v;
+    }
+    if (nd) return;
+    __syncthreads();
+    if (t < 64) {
+        const double v = tree_256(sh);
+        if (t == 0) partial[bk.pad] = v;
+    }
+}
+
 __device__ __forceinline__ int blk_scene(const Blk& b) { return b.inst; }
 
 // CGLinearSolver.inl:86-160 for nb_iter = 1 (rho = r.r = b.b), once |b|^2 is known: the exact
 // path's CG scalars of a scene at the start of a solve
 __device__ __forceinline__ void cg_start(InstDev* ins, double total) {
     ins->normb = sqrt(total);
-    ins->rho = total;
-    ins->rho_1 = 0.0;
+    ins->rho_slot[1] = total;
     ins->iter = 1;
     ins->stopped = 0;
     ins->end_reason = 0;
@@ -190,8 +231,7 @@ __device__ __forceinline__ void cg_start(InstDev* ins, double total) {
 // iteration-1 tolerance test with the first step's exemption (CGLinearSolver.inl:94-105,139-170)
 __device__ __forceinline__ void cg_start_warm(InstDev* ins, double bb, double rr) {
     ins->normb = sqrt(bb);
-    ins->rho = rr;
-    ins->rho_1 = 0.0;
+    ins->rho_slot[1] = rr;
     ins->iter = 1;
     ins->stopped = 0;
     ins->end_reason = 0;
@@ -206,16 +246,16 @@ __device__ __forceinline__ void cg_start_warm(InstDev* ins, double bb, double rr
     }
 }
 
-// end of a component-level CG solve (no time step): the loop's exit record, timeStepCount++
-// (CGLinearSolver.inl:300); reopen = 1 for the tiled kernels, which run with stopped == 0
-static __global__ void k_solve_end(const int* __restrict__ scenes, int n, InstDev* __restrict__ inst, int reopen) {
+// end of a component-level CG solve (no time step) on the tiled kernels: the loop's exit record,
+// timeStepCount++ (CGLinearSolver.inl:300), reopened (they run with stopped == 0)
+static __global__ void k_solve_end(const int* __restrict__ scenes, int n, InstDev* __restrict__ inst) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     InstDev* in = &inst[scenes[i]];
-    if (!in->stopped) { in->stopped = 1; in->end_reason = 0; in->last_iters = in->max_iter; }
+    if (!in->stopped) { in->end_reason = 0; in->last_iters = in->max_iter; }
     in->first_solve = 0;
     in->step_count += 1;
-    if (reopen) in->stopped = 0;
+    in->stopped = 0;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -292,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void k_rhs_node(const Blk* __restrict__ nbl
             load3(v, n, vm[0], vm[1], vm[2]);
             mass_mdx(in, na, n, in.m_rhs, vm, bn);
             if (in.mass_kind == kMassMatrix)
-                mass_edges(na, n, in.m_rhs, [&](int j, VT d[3]) { load3(v, j, d[0], d[1], d[2]); }, bn);
+                mass_edges<3>(na, n, in.m_rhs, [&](int j, VT d[3]) { load3(v, j, d[0], d[1], d[2]); }, bn);
         }
         gather_contributions<true>(na.inc, s0, s1, ef_v, bn);
         if (touch && in.k_rhs != 0.0) plane_dforce(in, in.k_rhs, vn, bn);
@@ -345,40 +385,129 @@ __global__ __launch_bounds__(kBlock) void k_cg_begin(const Blk* __restrict__ nbl
 }
 
 // ---------------------------------------------------------------------------------------
-// CG iteration
+// CG iteration.  The two node kernels run three threads per node, one per component (a lane's loads
+// are then coalesced, and 57,000 nodes give 2,700 waves instead of 890), and leave their dot product
+// as one partial per 256-node block; whoever needs the sum adds the partials itself, in the order the
+// scalars of a solve have always been summed, so no block waits for or fences against another.  The
+// scene's record is written by its first node block only: every field that the other blocks of the
+// same kernel read (rho_slot of the other parity, limits) is left alone there, and a stop they may see
+// early is the one they reach themselves.
 // ---------------------------------------------------------------------------------------
+constexpr int kNodeThreads = 3 * kBlock;
+
+// the tree of block_sum over sh[0 .. 255], by the first wave (lane 0 has the sum)
+__device__ __forceinline__ double tree_256(const double* sh) {
+    const int l = threadIdx.x;
+    double v = (sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]);
+    v = v + __shfl_down(v, 32, 64);
+    v = v + __shfl_down(v, 16, 64);
+    v = v + dpp_row_from<0x108>(v);
+    v = v + dpp_row_from<0x104>(v);
+    v = v + dpp_row_from<0x102>(v);
+    return v + dpp_row_from<0x101>(v);
+}
+// the scene's sum of its node blocks' partials, in every thread: each of 256 threads a strided sum,
+// then block_sum's tree (last_block_reduce's order)
+__device__ __forceinline__ double block_partials(const double* __restrict__ partial, const InstDev* ins, double* sh) {
+    const int nb = ins->nblk_count, b0 = ins->nblk_begin;
+    if (threadIdx.x < kBlock) {
+        double acc = 0.0;
+        for (int k = threadIdx.x; k < nb; k += kBlock) acc = acc + partial[b0 + k];
+        sh[threadIdx.x] = acc;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const double v = tree_256(sh);
+        if (threadIdx.x == 0) sh[0] = v;
+    }
+    __syncthreads();
+    return sh[0];
+}
+// a dot product of the scene: already in its record (`ready`: summed in the reference's order, or
+// by k_cg_total), or from the partials
+__device__ __forceinline__ double cg_dot(const double* __restrict__ partial, const InstDev* ins, int which, int ready,
+                                         double* sh) {
+    return ready ? ins->dots[which] : block_partials(partial, ins, sh);
+}
+// a scene of many node blocks: its partials added once, by one block per scene, instead of by every
+// block of the next kernel
+static __global__ __launch_bounds__(kBlock) void k_cg_total(const int* __restrict__ scenes, InstDev* __restrict__ inst,
+                                                             const double* __restrict__ partial, int which) {
+    __shared__ double sh[kBlock];
+    InstDev* ins = &inst[scenes[blockIdx.x]];
+    if (ins->stopped) return;
+    const double v = block_partials(partial, ins, sh);
+    if (threadIdx.x == 0) ins->dots[which] = v;
+}
+
+// the tests before iteration `it` (2 or later) with rho = r.r (PCG: r.z) of the last one: false when
+// the loop ends, else beta.  CGLinearSolver.inl:130-196; PCGLinearSolver.inl:241-246 (while iter <=
+// maxIter && r_norm > tol).  `first` (the scene's first node block): recorded.
+__device__ __forceinline__ bool cg_next(InstDev* ins, int it, double rho, bool first, double& beta) {
+    const bool record = first && threadIdx.x == 0;
+    const bool over = it > ins->max_iter;
+    double err = 0.0;
+    bool stop = over;
+    if (ins->pcg) {
+        err = ins->bnorm2 != 0.0 ? rho / ins->bnorm2 : 0.0;
+        stop = over || !(rho > ins->pcg_tol);
+    } else if (!over) {
+        err = sqrt(rho) / ins->normb;
+        stop = err <= ins->tol;
+    }
+    beta = rho / ins->rho_slot[(it - 1) & 1];
+    if (record) {
+        if (ins->pcg || !over) ins->err = err;
+        if (stop) {
+            ins->stopped = 1;
+            ins->end_reason = over ? 0 : 1;
+            ins->last_iters = over && !ins->pcg ? ins->max_iter : it;
+        } else {
+            ins->rho_slot[it & 1] = rho;
+            ins->beta = beta;
+            ins->iter = it;
+        }
+    }
+    return !stop;
+}
+
+// prr: partials of r.r (r.z) of the previous iteration
 template <typename R, int NR, typename VT>
 __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Blk* __restrict__ eblk,
-                                                     const InstDev* __restrict__ inst, const VT* __restrict__ r_,
-                                                     const VT* __restrict__ p_old, VT* __restrict__ ef,
+                                                     InstDev* __restrict__ inst, const VT* __restrict__ r_,
+                                                     const VT* __restrict__ p_old, VT* __restrict__ ef, int it,
+                                                     const double* __restrict__ prr, int ready,
                                                      const VT* __restrict__ z = nullptr) {
+    __shared__ double sh[kBlock];
     const Blk bk = eblk[xcd_item()];
-    const InstDev& in = inst[bk.inst];
+    InstDev* ins = &inst[bk.inst];
+    const InstDev& in = *ins;
     if (in.stopped) return;
     // PCG: the direction is built from the preconditioned residual z (w = z + beta w)
     const VT* __restrict__ r = (in.pcg && z) ? z : r_;
-    const int64_t e = (int64_t)bk.begin + threadIdx.x;
-    if (e >= bk.end) return;
+    const int64_t e = min((int64_t)bk.begin + threadIdx.x, (int64_t)bk.end - 1);
     const int4 t = ev.tet[e];
-    const int first = in.iter == 1;
-    const VT beta = (VT)in.beta;
-    R u[12];
     const int nid[4] = {t.x, t.y, t.z, t.w};
+    VT rn[4][3], po[4][3];
 #pragma unroll
     for (int n = 0; n < 4; n++) {
-        VT r0, r1, r2;
-        load3(r, nid[n], r0, r1, r2);
-        if (!first) {
-            // cgstep_beta, GraphScattered: p *= beta; p += r (CGLinearSolver.cpp:40-44)
-            VT p0, p1, p2;
-            load3(p_old, nid[n], p0, p1, p2);
-            p0 *= beta; p0 += r0;
-            p1 *= beta; p1 += r1;
-            p2 *= beta; p2 += r2;
-            r0 = p0; r1 = p1; r2 = p2;
-        }
-        u[3 * n] = (R)r0; u[3 * n + 1] = (R)r1; u[3 * n + 2] = (R)r2;
+        load3(r, nid[n], rn[n][0], rn[n][1], rn[n][2]);
+        if (it > 1) load3(p_old, nid[n], po[n][0], po[n][1], po[n][2]);
     }
+    double beta_d = 0.0;
+    if (it > 1 && !cg_next(ins, it, cg_dot(prr, ins, kDotRR, ready, sh), false, beta_d)) return;
+    if ((int64_t)bk.begin + threadIdx.x >= bk.end) return;
+    const VT beta = (VT)beta_d;
+    R u[12];
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            VT d = rn[n][i];
+            // cgstep_beta, GraphScattered: p *= beta; p += r (CGLinearSolver.cpp:40-44)
+            if (it > 1) { VT w = po[n][i] * beta; w += d; d = w; }
+            u[3 * n + i] = (R)d;
+        }
     R rot[9], c[12];
     load_rot(ev, e, rot);
     elem_dforce<R, NR>(ev, e, rot, u, (R)in.k_cg, c);
@@ -386,139 +515,118 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
     for (int k = 0; k < 12; k++) ef[12 * e + k] = (VT)c[k];
 }
 
+// p (owned node), q = (1 + h rm) M p - h(h + rs) K p, projected; p.q per 256-node block into ppq, or
+// per node into nd (reference order)
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void k_cg_node(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
-                                                     NodeArrays na, const VT* __restrict__ ef,
-                                                     const VT* __restrict__ r_, const VT* __restrict__ p_old,
-                                                     VT* __restrict__ p, VT* __restrict__ q,
-                                                     double* __restrict__ partial, double* __restrict__ nd,
-                                                     const VT* __restrict__ z = nullptr) {
-    __shared__ double sh[kBlock];
+__global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
+                                                           NodeArrays na, const VT* __restrict__ ef,
+                                                           const VT* __restrict__ r_, const VT* __restrict__ p_old,
+                                                           VT* __restrict__ p, VT* __restrict__ q, int it,
+                                                           const double* __restrict__ prr, int ready,
+                                                           double* __restrict__ ppq, double* __restrict__ nd,
+                                                           const VT* __restrict__ z = nullptr) {
+    __shared__ double sh[kBlock], pr[kNodeThreads];
     const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
-    if (ins->stopped) return;
-    const VT* __restrict__ r = (ins->pcg && z) ? z : r_;
-    const int n = bk.begin + threadIdx.x;
-    double pq = 0.0;
-    if (n < bk.end) {
-        const InstDev& in = *ins;
-        const int64_t o = 3 * (int64_t)n;
-        const bool first = in.iter == 1;
-        const VT beta = (VT)in.beta;
-        // p = r (first iteration) or p *= beta; p += r (cgstep_beta), from the previous p
-        auto pdir = [&](int j, VT d[3]) {
-            load3(r, j, d[0], d[1], d[2]);
-            if (!first) {
-                VT po[3];
-                load3(p_old, j, po[0], po[1], po[2]);
-#pragma unroll
-                for (int k = 0; k < 3; k++) { po[k] *= beta; po[k] += d[k]; d[k] = po[k]; }
-            }
-        };
-        VT pn[3];
-        pdir(n, pn);
-        p[o] = pn[0]; p[o + 1] = pn[1]; p[o + 2] = pn[2];
-        // q = 0; mass addMDx(q, p, 1 + h rm); FEM addDForce(q, p, -h(h+rs)); projectResponse(q)
-        VT qn[3] = {0, 0, 0};
-        if (in.m_cg != 0.0) {
-            mass_mdx(in, na, n, in.m_cg, pn, qn);
-            if (in.mass_kind == kMassMatrix) mass_edges(na, n, in.m_cg, pdir, qn);
-        }
-        const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
-        gather_contributions<true>(na.inc, s0, s1, ef, qn);
-        if (in.plane_on && na.contact[n]) plane_dforce(in, in.k_cg, pn, qn);
-        if (na.fixed[n]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
-        q[o] = qn[0]; q[o + 1] = qn[1]; q[o + 2] = qn[2];
-        pq = dot3d(pn, qn);
-        if (nd) nd[n] = pq;
+    const InstDev& in = *ins;
+    if (in.stopped) return;
+    const VT* __restrict__ r = (in.pcg && z) ? z : r_;
+    const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
+    const int n = min(bk.begin + j, bk.end - 1);
+    const bool live = bk.begin + j < bk.end;
+    const int64_t o = 3 * (int64_t)n + c;
+    const VT rc = r[o], pc = p_old[o];
+    const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
+    const bool fixed = na.fixed[n] != 0;
+    double beta_d = 0.0;
+    if (it > 1 && !cg_next(ins, it, cg_dot(prr, ins, kDotRR, ready, sh), in.nblk_begin == bk.pad, beta_d)) return;
+    const VT beta = (VT)beta_d;
+    // p = r (first iteration) or p *= beta; p += r (cgstep_beta), from the previous p
+    VT pn = rc;
+    if (it > 1) { pn = pc * beta; pn += rc; }
+    if (live) p[o] = pn;
+    // q = 0; mass addMDx(q, p, 1 + h rm); FEM addDForce(q, p, -h(h+rs)); projectResponse(q)
+    VT qn = 0;
+    if (in.m_cg != 0.0) {
+        mass_mdx_1(in, na.mass, n, in.m_cg, pn, qn);
+        if (in.mass_kind == kMassMatrix)
+            mass_edges<1>(na, n, in.m_cg, [&](int k, VT d[1]) {
+                const int64_t w = 3 * (int64_t)k + c;
+                d[0] = r[w];
+                if (it > 1) { VT t = p_old[w] * beta; t += d[0]; d[0] = t; }
+            }, &qn);
     }
-    double den;
-    const bool last = nd ? last_block_sequential(nd, ins, den)
-                         : last_block_reduce(block_sum(pq, sh), partial, ins, bk.pad, sh, den);
-    if (last && threadIdx.x == 0) {
-        ins->den = den;
-        if (ins->pcg) {                     // PCGLinearSolver.inl:222-224: alpha = r.z / w.s
-            ins->alpha = ins->rho / den;
-            return;
+    gather_contributions<true, 1>(na.inc, s0, s1, ef + c, &qn);
+    if (in.plane_on) {
+        pr[threadIdx.x] = (double)pn;
+        __syncthreads();
+        if (na.contact[n]) {
+            const VT dx[3] = {(VT)pr[3 * j], (VT)pr[3 * j + 1], (VT)pr[3 * j + 2]};
+            VT df[3] = {qn, qn, qn};
+            plane_dforce(in, in.k_cg, dx, df);
+            qn = c == 0 ? df[0] : c == 1 ? df[1] : df[2];
         }
-        // CGLinearSolver.inl:207-265
-        const bool exempt = (ins->iter == 1 && ins->first_solve);
-        if (den != 0.0) {
-            if (fabs(den) <= ins->thr && !exempt) {
-                ins->stopped = 1; ins->end_reason = 2; ins->last_iters = ins->iter;
-            } else {
-                ins->alpha = ins->rho / den;
-            }
-        } else {
-            ins->stopped = 1; ins->end_reason = 3; ins->last_iters = ins->iter;
-        }
+        __syncthreads();
     }
+    if (fixed) qn = 0;
+    if (live) q[o] = qn;
+    pr[threadIdx.x] = live ? (double)pn * (double)qn : 0.0;
+    node_partial(pr, sh, nd, bk, ppq);
 }
 
+// den = p.q, the threshold test and alpha (CGLinearSolver.inl:207-265; PCG: alpha = r.z / w.s,
+// PCGLinearSolver.inl:222-224), then x += p alpha; r += q (-alpha) (CGLinearSolver.cpp:46-64,
+// vOp_v_inc_bf) and the partials of r.r (PCG: s = P^-1 r, r.s, PCGLinearSolver.inl:229-244)
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void k_cg_update(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
-                                                       const VT* __restrict__ p, const VT* __restrict__ q,
-                                                       VT* __restrict__ xcg, VT* __restrict__ r,
-                                                       double* __restrict__ partial, double* __restrict__ nd,
-                                                       const double* __restrict__ pinv = nullptr,
-                                                       VT* __restrict__ z = nullptr) {
-    __shared__ double sh[kBlock];
+__global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
+                                                             const VT* __restrict__ p, const VT* __restrict__ q,
+                                                             VT* __restrict__ xcg, VT* __restrict__ r, int it,
+                                                             const double* __restrict__ ppq, int ready,
+                                                             double* __restrict__ prr, double* __restrict__ nd,
+                                                             const double* __restrict__ pinv = nullptr,
+                                                             VT* __restrict__ z = nullptr) {
+    __shared__ double sh[kBlock], pr[kNodeThreads];
     const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     if (ins->stopped) return;
-    const int n = bk.begin + threadIdx.x;
-    double rr = 0.0;
-    if (n < bk.end) {
-        // cgstep_alpha: x += p alpha; r += q (-alpha) (CGLinearSolver.cpp:46-64, vOp_v_inc_bf)
-        const VT a = (VT)ins->alpha, ma = (VT)(-ins->alpha);
-        const int64_t o = 3 * (int64_t)n;
-        VT rn[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            xcg[o + k] += p[o + k] * a;
-            rn[k] = r[o + k] + q[o + k] * ma;
-            r[o + k] = rn[k];
-        }
-        if (ins->pcg && pinv) {             // s = P^-1 r; r_norm = r.s (PCGLinearSolver.inl:229-244)
-            VT zn[3];
-            precond_apply(ins->pcg, pinv + 9 * (int64_t)n, rn, zn);
-            z[o] = zn[0]; z[o + 1] = zn[1]; z[o + 2] = zn[2];
-            rr = dot3d(rn, zn);
-        } else {
-            rr = dot3d(rn, rn);
-        }
-        if (nd) nd[n] = rr;
-    }
-    double rho;
-    const bool last = nd ? last_block_sequential(nd, ins, rho)
-                         : last_block_reduce(block_sum(rr, sh), partial, ins, bk.pad, sh, rho);
-    if (last && threadIdx.x == 0) {
-        // rho_1 = rho; next iteration: rho = r.r, err test, beta = rho / rho_1
-        ins->rho_1 = ins->rho;
-        ins->rho = rho;
-        const int it = ins->iter + 1;
-        ins->iter = it;
-        if (ins->pcg) {                     // while (iter <= maxIter && r_norm > tol)
-            ins->err = ins->bnorm2 != 0.0 ? rho / ins->bnorm2 : 0.0;
-            if (it > ins->max_iter || !(rho > ins->pcg_tol)) {
-                ins->stopped = 1; ins->end_reason = it > ins->max_iter ? 0 : 1; ins->last_iters = it;
-            } else {
-                ins->beta = rho / ins->rho_1;
-            }
+    const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
+    const int n = min(bk.begin + j, bk.end - 1);
+    const bool live = bk.begin + j < bk.end;
+    const int64_t o = 3 * (int64_t)n + c;
+    const VT pc = p[o], qc = q[o], xc = xcg[o], rc = r[o];
+    const bool pcg = ins->pcg && pinv;
+    const double den = cg_dot(ppq, ins, kDotPQ, ready, sh);
+    const bool record = ins->nblk_begin == bk.pad && threadIdx.x == 0;
+    if (!ins->pcg) {
+        const bool exempt = it == 1 && ins->first_solve;
+        const int stop = den == 0.0 ? 3 : fabs(den) <= ins->thr && !exempt ? 2 : 0;
+        if (stop) {
+            if (record) { ins->den = den; ins->stopped = 1; ins->end_reason = stop; ins->last_iters = it; }
             return;
         }
-        if (it > ins->max_iter) {
-            ins->stopped = 1; ins->end_reason = 0; ins->last_iters = ins->max_iter;
-        } else {
-            const double err = sqrt(rho) / ins->normb;
-            ins->err = err;
-            if (err <= ins->tol) {
-                ins->stopped = 1; ins->end_reason = 1; ins->last_iters = it;
-            } else {
-                ins->beta = rho / ins->rho_1;
-            }
-        }
     }
+    const double alpha = ins->rho_slot[it & 1] / den;
+    if (record) { ins->den = den; ins->alpha = alpha; }
+    const VT a = (VT)alpha, ma = (VT)(-alpha);
+    const VT rn = rc + qc * ma;
+    if (live) {
+        xcg[o] = xc + pc * a;
+        r[o] = rn;
+    }
+    double w = (double)rn;
+    if (pcg) {
+        pr[threadIdx.x] = (double)rn;
+        __syncthreads();
+        const VT rv[3] = {(VT)pr[3 * j], (VT)pr[3 * j + 1], (VT)pr[3 * j + 2]};
+        VT zn[3];
+        precond_apply(ins->pcg, pinv + 9 * (int64_t)n, rv, zn);
+        const VT zc = c == 0 ? zn[0] : c == 1 ? zn[1] : zn[2];
+        if (live) z[o] = zc;
+        w = (double)zc;
+        __syncthreads();
+    }
+    pr[threadIdx.x] = live ? (double)rn * w : 0.0;
+    node_partial(pr, sh, nd, bk, prr);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -550,15 +658,32 @@ __global__ __launch_bounds__(kBlock) void k_euler_update(const Blk* __restrict__
     }
 }
 
-static __global__ void k_finalize(const int* __restrict__ scenes, int n, InstDev* __restrict__ inst) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    InstDev* in = &inst[scenes[i]];
-    if (!in->stopped) { in->stopped = 1; in->last_iters = in->max_iter; }
+// the end of a solve and, STEP, of its time step (one block per scene).  A loop that ran its whole
+// budget is recorded here: PCG's last r.z still gives its err.
+template <bool STEP>
+__global__ __launch_bounds__(kBlock) void k_finalize(const int* __restrict__ scenes, InstDev* __restrict__ inst,
+                                                      const double* __restrict__ prr, int ready) {
+    __shared__ double sh[kBlock];
+    InstDev* in = &inst[scenes[blockIdx.x]];
+    const bool open = !in->stopped, pcg = in->pcg && in->max_iter > 0;
+    double rho = 0.0;
+    if (open && pcg) rho = cg_dot(prr, in, kDotRR, ready, sh);
+    if (threadIdx.x != 0) return;
+    if (open) {
+        in->stopped = 1;
+        in->last_iters = in->max_iter;
+        if (pcg) {
+            in->err = in->bnorm2 != 0.0 ? rho / in->bnorm2 : 0.0;
+            in->end_reason = 0;
+            in->last_iters = in->max_iter + 1;
+        }
+    }
     in->first_solve = 0;
     in->step_count += 1;
-    in->time += in->dt;
-    in->lm_x0_set = 1;         // LinearMovementProjectiveConstraint's x0 captured by this step
+    if (STEP) {
+        in->time += in->dt;
+        in->lm_x0_set = 1;     // LinearMovementProjectiveConstraint's x0 captured by this step
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -768,7 +893,7 @@ __global__ __launch_bounds__(kBlock) void k_mass_mdx(const InstDev* __restrict__
     load3(res, i, o[0], o[1], o[2]);
     mass_mdx(in, na, nb0 + i, factor, d, o);
     if (in.mass_kind == kMassMatrix)
-        mass_edges(na, nb0 + i, factor, [&](int j, VT e[3]) { load3(dx, j - nb0, e[0], e[1], e[2]); }, o);
+        mass_edges<3>(na, nb0 + i, factor, [&](int j, VT e[3]) { load3(dx, j - nb0, e[0], e[1], e[2]); }, o);
     const int64_t q = 3 * (int64_t)i;
     res[q] = o[0]; res[q + 1] = o[1]; res[q + 2] = o[2];
 }
@@ -1272,7 +1397,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_begin(const Blk* __restrict__ nb
         if (in.m_cg != 0.0) {
             mass_mdx(in, na, n, in.m_cg, xn, qn);
             if (in.mass_kind == kMassMatrix)
-                mass_edges(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
+                mass_edges<3>(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
         }
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
         gather_contributions<true>(na.inc, s0, s1, ef, qn);
@@ -1290,8 +1415,7 @@ __global__ __launch_bounds__(kBlock) void k_pcg_begin(const Blk* __restrict__ nb
     const bool last = nd ? last_block_sequential(nd, ins, rho)
                          : last_block_reduce(block_sum(rz, sh), partial, ins, bk.pad, sh, rho);
     if (last && threadIdx.x == 0) {
-        ins->rho = rho;
-        ins->rho_1 = 0.0;
+        ins->rho_slot[1] = rho;
         ins->err = ins->bnorm2 != 0.0 ? rho / ins->bnorm2 : 0.0;
         if (ins->max_iter < 1 || !(rho > ins->pcg_tol)) {
             ins->stopped = 1; ins->end_reason = 1; ins->last_iters = 1;
@@ -1334,7 +1458,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_warm_begin(const Blk* __restrict_
         if (in.m_cg != 0.0) {
             mass_mdx(in, na, n, in.m_cg, xn, qn);
             if (in.mass_kind == kMassMatrix)
-                mass_edges(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
+                mass_edges<3>(na, n, in.m_cg, [&](int j, VT d[3]) { load3(xcg, j, d[0], d[1], d[2]); }, qn);
         }
         const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
         gather_contributions<true>(na.inc, s0, s1, ef, qn);
