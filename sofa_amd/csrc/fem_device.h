@@ -31,52 +31,62 @@ constexpr int kBlock = 256;   // threads per block for every kernel (4 wave64)
 // ---------------------------------------------------------------------------------------
 // per-scene device record; one per scene, written by the last block of each reduction
 // ---------------------------------------------------------------------------------------
-struct InstDev {
-    // ranges in the flattened index spaces
-    int node_begin, node_count, elem_begin, elem_count;
-    int nblk_begin, nblk_count;      // node blocks of this scene (reduction partials)
-    int mass_kind;                    // 0 uniform, 1 diagonal
+// A kernel copies the record at its head (const InstDev in = *ins) and reads the copy: the fields it
+// uses are then fetched by scalar loads that are all in flight with its first gathers.  Read where
+// they are needed, each waited for memory on its own (five to eight waits of 0.3 to 0.8 us in a 7 us
+// kernel).  Fields are written through the pointer.
+struct alignas(64) InstDev {
+    // what the kernels of a CG iteration read: two cache lines (CGLinearSolver.inl:86-270)
+    int stopped;                      // 1 once the loop has exited
+    int first_solve;                  // timeStepCount == 0
     int max_iter;
-    double dt, rm, rs;
+    int mass_kind;                    // 0 uniform, 1 diagonal
+    int keep_dir;                     // inner record: sweeps continue the previous search direction
+    int sweep;                        // inner record: current sweep (1-based)
+    // PCGLinearSolver (PCGLinearSolver.inl:178-262) in place of CGLinearSolver: 0 none, 1 with a
+    // JacobiPreconditioner, 2 with a BlockJacobiPreconditioner.  warm_start: CGLinearSolver warmStart
+    // (CGLinearSolver.inl:94-105), the solve starting from the previous step's solution
+    int pcg, warm_start;
+    double tol, thr;
+    double normb, beta;
+    double rho_slot[2];               // rho of iterations k-1 and k, by k & 1
+    double rho_last;                  // inner record: r.r that built the current direction
+    // tiled engines in the reference's summation order: |b|^2, p.q and r.r of the current
+    // iteration, each summed node after node (MechanicalObject::vDot's order)
+    double dots[3];
+    double k_cg, m_cg;                // -h(h + rs), 1 + h rm    (EulerImplicitSolver.cpp:169-171)
     double vertex_mass;
+    double ks[3];                     // one material for the whole scene: K00, K01, K33 times
+                                      // 36 V (computeMaterialStiffness before the volume division)
+    int plane_on, plane_bilateral;
+    int nblk_begin, nblk_count;       // node blocks of this scene (reduction partials)
+    double bnorm2, pcg_tol;           // PCG: b.b of the step, the tolerance on r.z (tolerance b.b)
+    // PlaneForceField (PlaneForceField.inl:86-98), after the FEM in scene order
+    double plane_n[3], plane_d, plane_k, plane_damp, plane_max;
+    // the rest: ranges in the flattened index spaces, parameters, the record of the last solve
+    int node_begin, node_count, elem_begin, elem_count;
+    double dt, rm, rs;
     double gravity[3];
     double mg[3];                     // gravity * vertexMass (UniformMass.inl:486-487)
     double k_rhs, m_rhs;              // (h + rs), -rm           (EulerImplicitSolver.cpp:152-154)
-    double k_cg, m_cg;                // -h(h + rs), 1 + h rm    (EulerImplicitSolver.cpp:169-171)
-    double tol, thr;
-    // CG scalars (CGLinearSolver.inl:86-270)
-    double normb, den, alpha, beta, err;
+    double den, alpha, err;
     int iter;                         // current nb_iter
-    int stopped;                      // 1 once the loop has exited
     int end_reason;                   // 0 iterations, 1 tolerance, 2 threshold, 3 den==0, 4 |b|==0
-    int first_solve;                  // timeStepCount == 0
     int step_count;
     int last_iters;
     double time;
     unsigned int counter;             // arrivals of the current reduction (exact path)
     int pad_;
-    double rho_slot[2];               // rho of iterations k-1 and k, by k & 1
     // iterative refinement (MIXED engines; the scene record of the inner FP32 CG is separate)
     int max_sweeps;                   // inner solves per step at most
     int ir_sweeps;                    // inner solves done in the last step
     int cg_total;                     // inner CG iterations summed over the sweeps of a step
-    int keep_dir;                     // inner record: sweeps continue the previous search direction
-    int sweep;                        // inner record: current sweep (1-based)
     int pad3_;
-    double rho_last;                  // inner record: r.r that built the current direction
-    double ks[3];                     // one material for the whole scene: K00, K01, K33 times
-                                      // 36 V (computeMaterialStiffness before the volume division)
     // EulerImplicitSolver options (EulerImplicitSolver.cpp:40-51,136-173,246-299)
     double b_scale;                   // the right-hand side's factor: h, or 1 with firstOrder
     double vdamp;                     // exp(-h vdamping), 1 without damping
     int first_order;                  // v = dv instead of v += dv
     int project_velocity;             // FixedProjectiveConstraint activate_projectVelocity
-    // PlaneForceField (PlaneForceField.inl:86-98), after the FEM in scene order
-    double plane_n[3], plane_d, plane_k, plane_damp, plane_max;
-    int plane_on, plane_bilateral;
-    // tiled engines in the reference's summation order: |b|^2, p.q and r.r of the current
-    // iteration, each summed node after node by k_seqdot (MechanicalObject::vDot's order)
-    double dots[3];
     // LinearMovementProjectiveConstraint (LinearMovementProjectiveConstraint.inl:160-330), one
     // per scene: lm_n constrained nodes (global ids), the mask each has without the movement's bit,
     // their positions at the first projection (x0, captured then), lm_nk key times followed by
@@ -86,12 +96,6 @@ struct InstDev {
     double* lm_x0;
     const double* lm_keys;
     int lm_n, lm_nk, lm_relative, lm_x0_set;
-    // PCGLinearSolver (PCGLinearSolver.inl:178-262) in place of CGLinearSolver: 0 none, 1 with a
-    // JacobiPreconditioner, 2 with a BlockJacobiPreconditioner; b.b of the step and the tolerance
-    // on r.z (tolerance b.b).  warm_start: CGLinearSolver warmStart (CGLinearSolver.inl:94-105),
-    // the solve starting from the previous step's solution
-    int pcg, warm_start;
-    double bnorm2, pcg_tol;
     // reference-order dot products asked for in segments without candidates: boundaries summed by
     // the chain (counted since the scene was placed)
     int dot_fallbacks, pad_fb;

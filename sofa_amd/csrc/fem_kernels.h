@@ -84,13 +84,13 @@ __device__ __forceinline__ void mass_gravity(const InstDev& in, const double* __
 
 // edge part of the consistent MeshMatrixMass addMDx (MeshMatrixMass.inl:2014-2026): for each
 // edge of node n in ascending edge id, out += d[other] * (edgeMass * factor); `dof(j, v)` gives the
-// NC components of the multiplied vector at node j.  Edges are loaded four at a time, as
-// gather_contributions does.
+// NC components of the multiplied vector at node j.  Edges are loaded several at a
+// time, as Contributions does.
 template <int NC, typename VT, typename F>
 __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double factor, F dof, VT out[NC]) {
     const int s0 = na.em_ptr[n], s1 = na.em_ptr[n + 1];
     const VT fct = (VT)factor;
-    constexpr int B = 4;
+    constexpr int B = NC == 1 ? 8 : 4;
     for (int s = s0; s < s1; s += B) {
         int nbr[B];
         VT tm[B], d[B][NC];
@@ -111,29 +111,45 @@ __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double f
     }
 }
 
-// acc (+|-)= the NC components ef[3 slot ..] of the node's element contributions over its incidence
-// list [s0, s1), in list order.  Eight incidences at a time: their slots, then their values, are
-// loaded together (the tail at clamped indices), so a node of 24 tetrahedra waits for memory 6 times
-// instead of 48: latency is what bounds the node kernels (the CG node kernel, a lane per node, went
-// from 14.0 to 10.3 us on 525 nodes and from 25.7 to 21.7 on 57,000).
-template <bool SUB, int NC = 3, typename VT>
+// A node's element contributions ef[3 slot ..] over its incidence list, in list order, eight
+// incidences at a time: their slots, then their values, are loaded together (the tail at clamped
+// indices), so a node of 24 tetrahedra waits for memory 6 times instead of 48.  Latency is what
+// bounds the node kernels: the CG node kernel, a lane per node, went from 14.0 to 10.3 us on 525 nodes
+// and from 25.7 to 21.7 on 57,000.  Contributions: one component, the loads apart from the adds, so
+// that the first can be in flight while the scene's scalars are summed.
+template <typename VT>
+struct Contributions {
+    static constexpr int B = 8;
+    VT c[B];
+    __device__ __forceinline__ void load(const int* __restrict__ inc, int s, int s1, const VT* __restrict__ ef) {
+        int slot[B];
+#pragma unroll
+        for (int t = 0; t < B; t++) slot[t] = inc[max(min(s + t, s1 - 1), 0)];   // (an empty list: entry 0)
+#pragma unroll
+        for (int t = 0; t < B; t++) c[t] = ef[3 * (int64_t)slot[t]];
+    }
+    __device__ __forceinline__ void subtract(int s, int s1, VT& acc) const {
+#pragma unroll
+        for (int t = 0; t < B; t++)
+            if (s + t < s1) acc -= c[t];
+    }
+};
+template <bool SUB, typename VT>
 __device__ __forceinline__ void gather_contributions(const int* __restrict__ inc, int s0, int s1,
-                                                     const VT* __restrict__ ef, VT acc[NC]) {
+                                                     const VT* __restrict__ ef, VT acc[3]) {
     constexpr int B = 8;
     for (int s = s0; s < s1; s += B) {
         int slot[B];
-        VT c[B][NC];
+        VT c[B][3];
 #pragma unroll
         for (int t = 0; t < B; t++) slot[t] = inc[min(s + t, s1 - 1)];
 #pragma unroll
-        for (int t = 0; t < B; t++)
-#pragma unroll
-            for (int i = 0; i < NC; i++) c[t][i] = ef[3 * (int64_t)slot[t] + i];
+        for (int t = 0; t < B; t++) load3(ef, slot[t], c[t][0], c[t][1], c[t][2]);
 #pragma unroll
         for (int t = 0; t < B; t++)
             if (s + t < s1) {
 #pragma unroll
-                for (int i = 0; i < NC; i++) {
+                for (int i = 0; i < 3; i++) {
                     if (SUB) acc[i] -= c[t][i];
                     else acc[i] += c[t][i];
                 }
@@ -267,9 +283,9 @@ __global__ __launch_bounds__(kBlock) void k_rhs_elem(ElemView<R, NR> ev, const B
                                                       const VT* __restrict__ v, VT* __restrict__ ef_f,
                                                       VT* __restrict__ ef_v) {
     const Blk bk = eblk[xcd_item()];
+    const InstDev in = inst[bk.inst];
     const int64_t e = (int64_t)bk.begin + threadIdx.x;
     if (e >= bk.end) return;
-    const InstDev& in = inst[bk.inst];
     const int4 t = ev.tet[e];
     R rot[9], c[12], g[12];
     elem_force<R, NR, VT>(ev, e, t, x, rot, c, g);
@@ -408,8 +424,8 @@ __device__ __forceinline__ double tree_256(const double* sh) {
 }
 // the scene's sum of its node blocks' partials, in every thread: each of 256 threads a strided sum,
 // then block_sum's tree (last_block_reduce's order)
-__device__ __forceinline__ double block_partials(const double* __restrict__ partial, const InstDev* ins, double* sh) {
-    const int nb = ins->nblk_count, b0 = ins->nblk_begin;
+__device__ __forceinline__ double block_partials(const double* __restrict__ partial, const InstDev& in, double* sh) {
+    const int nb = in.nblk_count, b0 = in.nblk_begin;
     if (threadIdx.x < kBlock) {
         double acc = 0.0;
         for (int k = threadIdx.x; k < nb; k += kBlock) acc = acc + partial[b0 + k];
@@ -425,9 +441,9 @@ __device__ __forceinline__ double block_partials(const double* __restrict__ part
 }
 // a dot product of the scene: already in its record (`ready`: summed in the reference's order, or
 // by k_cg_total), or from the partials
-__device__ __forceinline__ double cg_dot(const double* __restrict__ partial, const InstDev* ins, int which, int ready,
+__device__ __forceinline__ double cg_dot(const double* __restrict__ partial, const InstDev& in, int which, int ready,
                                          double* sh) {
-    return ready ? ins->dots[which] : block_partials(partial, ins, sh);
+    return ready ? in.dots[which] : block_partials(partial, in, sh);
 }
 // a scene of many node blocks: its partials added once, by one block per scene, instead of by every
 // block of the next kernel
@@ -436,32 +452,32 @@ static __global__ __launch_bounds__(kBlock) void k_cg_total(const int* __restric
     __shared__ double sh[kBlock];
     InstDev* ins = &inst[scenes[blockIdx.x]];
     if (ins->stopped) return;
-    const double v = block_partials(partial, ins, sh);
+    const double v = block_partials(partial, *ins, sh);
     if (threadIdx.x == 0) ins->dots[which] = v;
 }
 
 // the tests before iteration `it` (2 or later) with rho = r.r (PCG: r.z) of the last one: false when
 // the loop ends, else beta.  CGLinearSolver.inl:130-196; PCGLinearSolver.inl:241-246 (while iter <=
 // maxIter && r_norm > tol).  `first` (the scene's first node block): recorded.
-__device__ __forceinline__ bool cg_next(InstDev* ins, int it, double rho, bool first, double& beta) {
+__device__ __forceinline__ bool cg_next(InstDev* ins, const InstDev& in, int it, double rho, bool first, double& beta) {
     const bool record = first && threadIdx.x == 0;
-    const bool over = it > ins->max_iter;
+    const bool over = it > in.max_iter;
     double err = 0.0;
     bool stop = over;
-    if (ins->pcg) {
-        err = ins->bnorm2 != 0.0 ? rho / ins->bnorm2 : 0.0;
-        stop = over || !(rho > ins->pcg_tol);
+    if (in.pcg) {
+        err = in.bnorm2 != 0.0 ? rho / in.bnorm2 : 0.0;
+        stop = over || !(rho > in.pcg_tol);
     } else if (!over) {
-        err = sqrt(rho) / ins->normb;
-        stop = err <= ins->tol;
+        err = sqrt(rho) / in.normb;
+        stop = err <= in.tol;
     }
-    beta = rho / ins->rho_slot[(it - 1) & 1];
+    beta = rho / (it & 1 ? in.rho_slot[0] : in.rho_slot[1]);
     if (record) {
-        if (ins->pcg || !over) ins->err = err;
+        if (in.pcg || !over) ins->err = err;
         if (stop) {
             ins->stopped = 1;
             ins->end_reason = over ? 0 : 1;
-            ins->last_iters = over && !ins->pcg ? ins->max_iter : it;
+            ins->last_iters = over && !in.pcg ? in.max_iter : it;
         } else {
             ins->rho_slot[it & 1] = rho;
             ins->beta = beta;
@@ -481,7 +497,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
     __shared__ double sh[kBlock];
     const Blk bk = eblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
-    const InstDev& in = *ins;
+    const InstDev in = *ins;
     if (in.stopped) return;
     // PCG: the direction is built from the preconditioned residual z (w = z + beta w)
     const VT* __restrict__ r = (in.pcg && z) ? z : r_;
@@ -495,7 +511,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
         if (it > 1) load3(p_old, nid[n], po[n][0], po[n][1], po[n][2]);
     }
     double beta_d = 0.0;
-    if (it > 1 && !cg_next(ins, it, cg_dot(prr, ins, kDotRR, ready, sh), false, beta_d)) return;
+    if (it > 1 && !cg_next(ins, in, it, cg_dot(prr, in, kDotRR, ready, sh), false, beta_d)) return;
     if ((int64_t)bk.begin + threadIdx.x >= bk.end) return;
     const VT beta = (VT)beta_d;
     R u[12];
@@ -528,7 +544,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict_
     __shared__ double sh[kBlock], pr[kNodeThreads];
     const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
-    const InstDev& in = *ins;
+    const InstDev in = *ins;
     if (in.stopped) return;
     const VT* __restrict__ r = (in.pcg && z) ? z : r_;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
@@ -538,8 +554,10 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict_
     const VT rc = r[o], pc = p_old[o];
     const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
     const bool fixed = na.fixed[n] != 0;
+    Contributions<VT> g;    // the first 8 in flight while the scene's scalars are summed
+    g.load(na.inc, s0, s1, ef + c);
     double beta_d = 0.0;
-    if (it > 1 && !cg_next(ins, it, cg_dot(prr, ins, kDotRR, ready, sh), in.nblk_begin == bk.pad, beta_d)) return;
+    if (it > 1 && !cg_next(ins, in, it, cg_dot(prr, in, kDotRR, ready, sh), in.nblk_begin == bk.pad, beta_d)) return;
     const VT beta = (VT)beta_d;
     // p = r (first iteration) or p *= beta; p += r (cgstep_beta), from the previous p
     VT pn = rc;
@@ -556,7 +574,10 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict_
                 if (it > 1) { VT t = p_old[w] * beta; t += d[0]; d[0] = t; }
             }, &qn);
     }
-    gather_contributions<true, 1>(na.inc, s0, s1, ef + c, &qn);
+    for (int s = s0; s < s1; s += 8) {
+        if (s > s0) g.load(na.inc, s, s1, ef + c);
+        g.subtract(s, s1, qn);
+    }
     if (in.plane_on) {
         pr[threadIdx.x] = (double)pn;
         __syncthreads();
@@ -588,24 +609,25 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
     __shared__ double sh[kBlock], pr[kNodeThreads];
     const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
-    if (ins->stopped) return;
+    const InstDev in = *ins;
+    if (in.stopped) return;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
     const int n = min(bk.begin + j, bk.end - 1);
     const bool live = bk.begin + j < bk.end;
     const int64_t o = 3 * (int64_t)n + c;
     const VT pc = p[o], qc = q[o], xc = xcg[o], rc = r[o];
-    const bool pcg = ins->pcg && pinv;
-    const double den = cg_dot(ppq, ins, kDotPQ, ready, sh);
-    const bool record = ins->nblk_begin == bk.pad && threadIdx.x == 0;
-    if (!ins->pcg) {
-        const bool exempt = it == 1 && ins->first_solve;
-        const int stop = den == 0.0 ? 3 : fabs(den) <= ins->thr && !exempt ? 2 : 0;
+    const bool pcg = in.pcg && pinv;
+    const double den = cg_dot(ppq, in, kDotPQ, ready, sh);
+    const bool record = in.nblk_begin == bk.pad && threadIdx.x == 0;
+    if (!in.pcg) {
+        const bool exempt = it == 1 && in.first_solve;
+        const int stop = den == 0.0 ? 3 : fabs(den) <= in.thr && !exempt ? 2 : 0;
         if (stop) {
             if (record) { ins->den = den; ins->stopped = 1; ins->end_reason = stop; ins->last_iters = it; }
             return;
         }
     }
-    const double alpha = ins->rho_slot[it & 1] / den;
+    const double alpha = (it & 1 ? in.rho_slot[1] : in.rho_slot[0]) / den;
     if (record) { ins->den = den; ins->alpha = alpha; }
     const VT a = (VT)alpha, ma = (VT)(-alpha);
     const VT rn = rc + qc * ma;
@@ -619,7 +641,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
         __syncthreads();
         const VT rv[3] = {(VT)pr[3 * j], (VT)pr[3 * j + 1], (VT)pr[3 * j + 2]};
         VT zn[3];
-        precond_apply(ins->pcg, pinv + 9 * (int64_t)n, rv, zn);
+        precond_apply(in.pcg, pinv + 9 * (int64_t)n, rv, zn);
         const VT zc = c == 0 ? zn[0] : c == 1 ? zn[1] : zn[2];
         if (live) z[o] = zc;
         w = (double)zc;
@@ -667,7 +689,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const int* __restrict__ sce
     InstDev* in = &inst[scenes[blockIdx.x]];
     const bool open = !in->stopped, pcg = in->pcg && in->max_iter > 0;
     double rho = 0.0;
-    if (open && pcg) rho = cg_dot(prr, in, kDotRR, ready, sh);
+    if (open && pcg) rho = cg_dot(prr, *in, kDotRR, ready, sh);
     if (threadIdx.x != 0) return;
     if (open) {
         in->stopped = 1;

@@ -31,7 +31,8 @@ static __global__ __launch_bounds__(kBlock) void k_ir_residual(const NodeBlk* __
                                                                 float* __restrict__ zbuf) {
     __shared__ double sh[kBlock / 64];
     const NodeBlk nb = nb_[xcd_item()];
-    if (inst[nb.scene].stopped) return;
+    const InstDev in = inst[nb.scene];
+    if (in.stopped) return;
     double rr = 0.0, rr32 = 0.0;
 #pragma unroll
     for (int k = 0; k < kNodesPerThread; k++) {
@@ -52,7 +53,7 @@ static __global__ __launch_bounds__(kBlock) void k_ir_residual(const NodeBlk* __
             rr += dot3d(rn, rn);
             if (zbuf) {
                 float zf[3];
-                precond_z(inst[nb.scene].pcg, dinv, binv, n, rf, zf);
+                precond_z(in.pcg, dinv, binv, n, rf, zf);
                 st3(zbuf, n, zf);
                 rr32 += dot3d(rf, zf);
             } else {
@@ -80,7 +81,7 @@ static __global__ __launch_bounds__(kBlock) void k_ir_control(const int* __restr
         return;
     }
     const Ranges rg = ranges[si];
-    const double rr = reduce2(prr, rg.b0, rg.nb, 0, 0, sh);
+    const double rr = reduce2(prr, rg.b0, rg.nb, sh);
     if (threadIdx.x != 0) return;
     if (sweep == 1) o->normb = sqrt(rr);
     const double normb = o->normb;

@@ -110,12 +110,31 @@ __device__ __forceinline__ double wave_sum(double v) {
                             __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
+// acc + buf[a0 + k] + buf[a0 + k + STRIDE] + ... below a0 + na, B terms, all loads in flight
+template <int STRIDE, int B>
+__device__ __forceinline__ double strided_terms(const double* __restrict__ buf, int a0, int na, int k, double acc) {
+    double v[B];
+#pragma unroll
+    for (int j = 0; j < B; j++) v[j] = buf[a0 + min(k + j * STRIDE, na - 1)];
+#pragma unroll
+    for (int j = 0; j < B; j++) acc = k + j * STRIDE < na ? acc + v[j] : acc;
+    return acc;
+}
+// buf[a0 + t] + buf[a0 + t + STRIDE] + ... below a0 + na, in that order: eight loads in flight, two
+// where two are all (one after the other each waited for memory)
+template <int STRIDE>
+__device__ __forceinline__ double strided_sum(const double* __restrict__ buf, int a0, int na, int t) {
+    if (na <= 0) return 0.0;
+    if (na <= 2 * STRIDE) return strided_terms<STRIDE, 2>(buf, a0, na, t, 0.0);
+    double acc = 0.0;
+    for (int k = t; k < na; k += 8 * STRIDE) acc = strided_terms<STRIDE, 8>(buf, a0, na, k, acc);
+    return acc;
+}
+
 // every wave of the block: the sum of buf[a0 .. a0 + na) (lane-strided partial sums, then
 // wave_sum) -- no LDS and no barrier, and the same bits in every wave and every block
 __device__ __forceinline__ double wave_reduce(const double* __restrict__ buf, int a0, int na) {
-    double acc = 0.0;
-    for (int k = (int)(threadIdx.x & 63); k < na; k += 64) acc = acc + buf[a0 + k];
-    return wave_sum(acc);
+    return wave_sum(strided_sum<64>(buf, a0, na, (int)(threadIdx.x & 63)));
 }
 
 // fixed-order block sum of the tiled kernels (TB threads): wave_sum within each wave, then the
@@ -132,13 +151,10 @@ __device__ __forceinline__ double wave_block_sum(double v, double* sh) {
     return r;
 }
 
-// fixed-order sum of buf[a0 .. a0+na) then buf[c0 .. c0+nc), all threads of the block
+// fixed-order sum of buf[a0 .. a0+na), all threads of the block
 template <int TB = kBlock>
-__device__ __forceinline__ double reduce2(const double* __restrict__ buf, int a0, int na, int c0, int nc, double* sh) {
-    double acc = 0.0;
-    for (int k = threadIdx.x; k < na; k += TB) acc = acc + buf[a0 + k];
-    for (int k = threadIdx.x; k < nc; k += TB) acc = acc + buf[c0 + k];
-    return wave_block_sum<TB>(acc, sh);
+__device__ __forceinline__ double reduce2(const double* __restrict__ buf, int a0, int na, double* sh) {
+    return wave_block_sum<TB>(strided_sum<TB>(buf, a0, na, (int)threadIdx.x), sh);
 }
 
 // a scene's sum of na partials, the same bits in every block of the scene: few partials are
@@ -148,7 +164,7 @@ constexpr int kWavePartials = 256;
 template <int TB, bool WIDE = true>
 __device__ __forceinline__ double scene_sum(const double* __restrict__ buf, int a0, int na, double* sh) {
     if (!WIDE || na <= kWavePartials) return wave_reduce(buf, a0, na);
-    return reduce2<TB>(buf, a0, na, 0, 0, sh);
+    return reduce2<TB>(buf, a0, na, sh);
 }
 
 template <typename VT>
@@ -180,9 +196,7 @@ __device__ __forceinline__ double fold_tiles(const double* __restrict__ buf, con
     const int chunk = (rg.nt + rg.nf - 1) / rg.nf;
     const int a0 = rg.t0 + bi * chunk;
     const int a1 = min(rg.t0 + rg.nt, a0 + chunk);
-    double acc = 0.0;
-    for (int k = a0; k < a1; k++) acc = acc + buf[k];
-    return acc;
+    return strided_sum<1>(buf, a0, a1 - a0, 0);
 }
 
 template <typename R, int NR>
@@ -318,7 +332,7 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
     __shared__ int lptr[kTileNodes + 1];
     __shared__ double sh[TB / 64];
     const TileDesc td = a.tiles[xcd_item()];
-    const InstDev& in = a.inst[td.scene];
+    const InstDev in = a.inst[td.scene];
     // element records of this thread's elements, in registers for both passes
     R rin[EPT][NR], kk[EPT][3], em[EPT], rot[EPT][9];
     uint2 lt[EPT];
@@ -503,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
                                                      double* __restrict__ nd = nullptr) {
     __shared__ double sh[kBlock / 64];
     const FinBlk fb = fb_[xcd_item()];
-    const InstDev& in = inst[fb.scene];
+    const InstDev in = inst[fb.scene];
     const int j = fb.begin + threadIdx.x;
     double bb = 0.0;
     if (j < fb.end) {
@@ -576,6 +590,9 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     __shared__ int lptr[kTileNodes + 1];
     __shared__ double sh[TB / 64];
     const TileDesc td = a.tiles[xcd_item()];
+    InstDev* ins = &a.inst[td.scene];
+    const InstDev in = *ins;
+    const Ranges rg = a.ranges[td.scene];
     const bool consistent = (td.flags & kTileConsistent) != 0;
     const bool kvol = GEO == 2 && (td.flags & kTileOneMaterial) != 0;   // K recomputed, not loaded
     // ---- 1. issue every load that depends on the tile descriptor only: the element records of
@@ -617,9 +634,23 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         psl[m] = a.tn.pslot[li];
         lead[m] = EXACT ? a.tn.lead[li] : 0;
     }
-    InstDev* ins = &a.inst[td.scene];
     // a refinement sweep that keeps the previous search direction continues CG at its iteration 1
-    const bool cont = iter == 1 && ins->keep_dir && ins->sweep > 1;
+    const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
+    // the partials of |b|^2 (iteration 1) or r.r: node blocks, or finalize blocks, or the tiles of a
+    // scene without shared nodes
+    const bool by_node = cont || iter > 1 || pin_nodes;
+    const int pa = by_node ? rg.b0 : rg.nf > 0 ? rg.f0 : rg.t0, pn = by_node ? rg.nb : rg.nf > 0 ? rg.nf : rg.nt;
+    constexpr bool kEarly = !EXACT && !WIDE;    // up to kWavePartials of them: in flight with the gathers
+    const int lane = threadIdx.x & 63;
+    double part[kWavePartials / 64] = {0.0, 0.0, 0.0, 0.0};
+    static_assert(kWavePartials == 256, "four partials per lane");
+    if (kEarly && iter > 0) {
+        part[0] = pin[pa + min(lane, max(pn - 1, 0))];
+        if (pn > 64) {
+#pragma unroll
+            for (int k = 1; k < kWavePartials / 64; k++) part[k] = pin[pa + min(lane + 64 * k, pn - 1)];
+        }
+    }
     // the incidence tables into registers first: their loads are in flight while the node ids
     // arrive and the node gathers below are issued; they go to LDS after those
     const int ninc = 4 * td.e_count;
@@ -644,7 +675,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     // p is read from iteration 2 on (or continuing a direction); without a p (a plain operator
     // application) the loads read r instead, unused
     const VT* __restrict__ pl = p ? p : r;
-    const bool plane = PLANE && ins->plane_on;
+    const bool plane = PLANE && in.plane_on;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
         ld3(r, gid[m], rr_[m]);
@@ -670,40 +701,48 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         const int j = threadIdx.x + k * TB;
         if (j <= td.ln_count) lptr[j] = ptr_r[k];
     }
-    if (ins->stopped) return;
-    const Ranges rg = a.ranges[td.scene];
+    if (in.stopped) return;
     const bool first = (td.flags & kTileFirst) != 0;
     // ---- 3. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
+    double total = 0.0;      // |b|^2 or r.r
+    if (!EXACT && iter > 0) {
+        if constexpr (kEarly) {
+#pragma unroll
+            for (int k = 0; k < kWavePartials / 64; k++)
+                total = lane + 64 * k < pn ? total + part[k] : total;
+            total = wave_sum(total);
+        } else {
+            total = scene_sum<TB, WIDE>(pin, pa, pn, sh);
+        }
+    }
     double beta = 0.0;
     if (cont) {
         // the refinement replaced r by the true residual: beta from its r.r and the r.r that
         // built p; the tolerance is relative to the first sweep's |r|
-        const double rho = scene_sum<TB, WIDE>(pin, rg.b0, rg.nb, sh);
-        const double err = sqrt(rho) / ins->normb;
-        if (rho == 0.0 || err <= ins->tol) { record_stop(ins, first, 1, 1, err); return; }
-        beta = rho / ins->rho_last;
+        const double rho = total;
+        const double err = sqrt(rho) / in.normb;
+        if (rho == 0.0 || err <= in.tol) { record_stop(ins, first, 1, 1, err); return; }
+        beta = rho / in.rho_last;
         if (first && threadIdx.x == 0) {
             ins->rho_slot[1] = rho; ins->beta = beta; ins->iter = 1; ins->err = err;
         }
     } else if (iter == 1) {
-        const double bb = EXACT ? ins->dots[kDotBB]
-                          : pin_nodes ? scene_sum<TB, WIDE>(pin, rg.b0, rg.nb, sh)
-                          : rg.nf > 0 ? scene_sum<TB, WIDE>(pin, rg.f0, rg.nf, sh) : scene_sum<TB, WIDE>(pin, rg.t0, rg.nt, sh);
+        const double bb = EXACT ? in.dots[kDotBB] : total;
         const double normb = sqrt(bb);
         if (normb == 0.0) { record_stop(ins, first, 4, 0, 1.0); return; }
         // rho = r.r: b.b from a cold start; warmStart (reference order): the r.r of r = b - A x
-        const double rho = EXACT && ins->warm_start ? ins->dots[kDotRR] : bb;
+        const double rho = EXACT && in.warm_start ? in.dots[kDotRR] : bb;
         const double err = sqrt(rho) / normb;
-        if (err <= ins->tol && !ins->first_solve) { record_stop(ins, first, 1, 1, err); return; }
+        if (err <= in.tol && !in.first_solve) { record_stop(ins, first, 1, 1, err); return; }
         if (first && threadIdx.x == 0) {
             ins->normb = normb; ins->rho_slot[1] = rho; ins->iter = 1; ins->err = err;
         }
     } else if (iter > 1) {
-        if (iter > ins->max_iter) { record_stop(ins, first, 0, ins->max_iter, ins->err); return; }
-        const double rho = EXACT ? ins->dots[kDotRR] : scene_sum<TB, WIDE>(pin, rg.b0, rg.nb, sh);
-        const double err = sqrt(rho) / ins->normb;
-        if (err <= ins->tol) { record_stop(ins, first, 1, iter, err); return; }
-        const double rho_1 = ins->rho_slot[(iter - 1) & 1];
+        if (iter > in.max_iter) { record_stop(ins, first, 0, in.max_iter, in.err); return; }
+        const double rho = EXACT ? in.dots[kDotRR] : total;
+        const double err = sqrt(rho) / in.normb;
+        if (err <= in.tol) { record_stop(ins, first, 1, iter, err); return; }
+        const double rho_1 = (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
         beta = rho / rho_1;
         if (first && threadIdx.x == 0) {
             ins->rho_slot[iter & 1] = rho; ins->beta = beta; ins->iter = iter; ins->err = err;
@@ -760,15 +799,15 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
 #pragma unroll
                         for (int i = 0; i < 3; i++) p0[v][i] = lx0[3 * l[v] + i];
                     rest_frame<R, NR>(p0, rin[m]);
-                    if (kvol) stiffness_from_volume(p0, ins->ks, kk[m]);
+                    if (kvol) stiffness_from_volume(p0, in.ks, kk[m]);
                 }
             }
         }
         __syncthreads();
     }
     // ---- 5. element K p into LDS
-    const R kcg = (R)ins->k_cg;
-    const R mcg = (R)ins->m_cg;
+    const R kcg = (R)in.k_cg;
+    const R mcg = (R)in.m_cg;
 #pragma unroll
     for (int m = 0; m < EPT; m++) {
         const int k = threadIdx.x + m * TB;
@@ -788,7 +827,6 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     }
     __syncthreads();
     // ---- 6. per-node sums in ascending element id, from LDS only
-    const InstDev& in = *ins;
     double pq = 0.0;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
@@ -857,7 +895,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_exact(const FinBlk* __restrict__
                                                        VT* __restrict__ q, const VT* __restrict__ sp,
                                                        double* __restrict__ nd, const int8_t* __restrict__ contact) {
     const FinBlk fb = fb_[xcd_item()];
-    const InstDev& in = inst[fb.scene];
+    const InstDev in = inst[fb.scene];
     if (in.stopped) return;
     const int j = fb.begin + threadIdx.x;
     if (j >= fb.end) return;
@@ -893,7 +931,7 @@ __global__ __launch_bounds__(kBlock) void k_warm_begin_exact(const NodeBlk* __re
                                                               const VT* __restrict__ b, const VT* __restrict__ q,
                                                               VT* __restrict__ r, double* __restrict__ nd) {
     const NodeBlk nb = nb_[xcd_item()];
-    const InstDev& in = inst[nb.scene];
+    const InstDev in = inst[nb.scene];
     if (!in.warm_start || in.stopped) return;
     const VT m1 = (VT)(-1.0);
 #pragma unroll
@@ -922,7 +960,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_apply(const FinBlk* __restrict__
                                                        const int8_t* __restrict__ contact) {
     __shared__ double sh[kBlock / 64];
     const FinBlk fb = fb_[xcd_item()];
-    const InstDev& in = inst[fb.scene];
+    const InstDev in = inst[fb.scene];
     if (in.stopped) return;
     const int j = fb.begin + threadIdx.x;
     double pq = 0.0;
@@ -998,6 +1036,8 @@ __global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ n
     __shared__ double sh[kBlock / 64];
     const NodeBlk nb = nb_[xcd_item()];
     InstDev* ins = &inst[nb.scene];
+    const InstDev in = *ins;
+    const Ranges rg = ranges[nb.scene];
     // node data first (registers), then the reduction
     VT pv[kNodesPerThread][3], qv[kNodesPerThread][3], xv[kNodesPerThread][3], rv[kNodesPerThread][3];
     VT zv[kNodesPerThread][3];
@@ -1015,21 +1055,19 @@ __global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ n
         ld3(p, n, pv[k]);
         ld3(q, n, qv[k]);
     }
-    if (ins->stopped) return;
-    const bool cont = iter == 1 && ins->keep_dir && ins->sweep > 1;
-    const Ranges rg = ranges[nb.scene];
+    if (in.stopped) return;
+    const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
     const bool first = nb.first != 0;
-    const double den = EXACT ? ins->dots[kDotPQ] : scene_sum<kBlock>(pden, rg.t0, rg.nt, sh);
-    const bool exempt = (iter == 1 && ins->first_solve);
-    if (den == 0.0) { record_stop(ins, first, 3, iter, ins->err); if (first && threadIdx.x == 0) ins->den = den; return; }
-    if (fabs(den) <= ins->thr && !exempt) {
-        record_stop(ins, first, 2, iter, ins->err);
+    const double den = EXACT ? in.dots[kDotPQ] : scene_sum<kBlock>(pden, rg.t0, rg.nt, sh);
+    const bool exempt = (iter == 1 && in.first_solve);
+    if (den == 0.0) { record_stop(ins, first, 3, iter, in.err); if (first && threadIdx.x == 0) ins->den = den; return; }
+    if (fabs(den) <= in.thr && !exempt) {
+        record_stop(ins, first, 2, iter, in.err);
         if (first && threadIdx.x == 0) ins->den = den;
         return;
     }
-    const double alpha = ins->rho_slot[iter & 1] / den;
+    const double alpha = (iter & 1 ? in.rho_slot[1] : in.rho_slot[0]) / den;
     if (first && threadIdx.x == 0) { ins->den = den; ins->alpha = alpha; }
-    const InstDev& in = *ins;
     const VT vb = (VT)in.beta;
     const VT va = (VT)alpha, vma = (VT)(-alpha);
     double rr = 0.0;
@@ -1069,7 +1107,7 @@ __global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ n
                 nd[n] = dot3d(rn, rn);
             } else if (zbuf) {   // z = P^-1 r for the next iteration, and r.z
                 VT zn[3];
-                precond_z(ins->pcg, dinv, binv, n, rn, zn);
+                precond_z(in.pcg, dinv, binv, n, rn, zn);
                 st3(zbuf, n, zn);
                 rr += dot3d(rn, zn);
             } else {
@@ -1118,7 +1156,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate(const NodeBlk* __restrict_
                                                        const VT* __restrict__ xcg, VT* __restrict__ v,
                                                        VT* __restrict__ x) {
     const NodeBlk nb = nb_[xcd_item()];
-    const InstDev& in = inst[nb.scene];
+    const InstDev in = inst[nb.scene];
     const VT h = (VT)in.dt;
     // v += dv (firstOrder: v = dv), x += v h, then vdamping's v *= exp(-h d)
     // (EulerImplicitSolver.cpp:246-299)
