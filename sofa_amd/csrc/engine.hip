@@ -1346,7 +1346,7 @@ struct EngineT : EngineBase {
             // PCGLinearSolver: the preconditioner from this step's rotations, then r = b - A x from the
             // previous solution, z = P^-1 r (CG scenes of the set pass through untouched)
             if (cur->nb > 0)
-                k_pcg_diag<R, NR, Blk><<<cur->nb, kBlock, 0, s>>>(ev, nb, inst, na.inc_ptr, na.inc, mass, fixed, pinv);
+                k_pcg_diag<R, NR, Blk><<<dim3(cur->nb, kBlock / kQuadNodes), kBlock, 0, s>>>(ev, nb, inst, na.inc_ptr, na.inc, mass, fixed, pinv);
             if (cur->nl > 0) k_pcg_lm_identity<<<cur->nl, kBlock, 0, s>>>((const Blk*)cur->l, inst, pinv);
             k_pcg_open<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
             if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, xcg, p2, ef, 1, partial, 0);
@@ -1636,7 +1636,7 @@ struct EngineT : EngineBase {
         if (cur->nb > 0) k_fin_rhs<VT><<<cur->nb, kBlock, 0, s>>>(fb, inst, ranges_d, sn, mass, fixed, v, sp0, sp1, f, b, r, xcg, pbb, x, contact);
         if (cur->pcg) {   // the inner CG's Jacobi preconditioner from this step's rotations
             if (cur->nc > 0)
-                k_jacobi32<R, NR><<<cur->nc, kBlock, 0, s>>>(view(), nb, inst, inc_ptr, inc, mass, fixed, dinv32, binv32);
+                k_jacobi32<R, NR><<<dim3(cur->nc, kBlock * kNodesPerThread / kQuadNodes), kBlock, 0, s>>>(view(), nb, inst, inc_ptr, inc, mass, fixed, dinv32, binv32);
             if (cur->nl > 0) k_jacobi32_lm<<<cur->nl, kBlock, 0, s>>>((const Blk*)cur->l, inst, dinv32, binv32);
         }
         for (int sw = 1; sw <= cur->maxsw + 1; sw++) {

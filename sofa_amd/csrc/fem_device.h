@@ -682,6 +682,10 @@ __device__ __forceinline__ double dpp_row_from(double v) {
                             __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, true));
 }
 
+// v of lane K of the aligned quad
+template <int K>
+__device__ __forceinline__ double quad_lane(double v) { return dpp_row_from<K * 0x55>(v); }
+
 // returns true in every thread of the last-arriving block of scene `ins`; `total` then holds
 // the scene's sum over its node blocks
 __device__ __forceinline__ bool last_block_reduce(double blockval, double* partial, InstDev* ins,

@@ -147,18 +147,19 @@ __global__ __launch_bounds__(kBlock) void k_jacobi32(ElemView<R, NR> ev, const N
                                                       const int8_t* __restrict__ fixed, float* __restrict__ dinv,
                                                       float* __restrict__ binv) {
     const NodeBlk bk = nblk[xcd_item()];
-    const InstDev& in = inst[bk.scene];
+    const InstDev in = inst[bk.scene];
     if (!in.pcg) return;   // z = r: neither array is read
-    for (int n = bk.begin + threadIdx.x; n < bk.end; n += kBlock) {
-        double B[9];
-        pcg_block<R, NR>(in, ev, inc_ptr, inc, mass, fixed, n, B);
-        if (in.pcg == 1) {
-            const float d[3] = {(float)B[0], (float)B[4], (float)B[8]};
-            st3(dinv, n, d);
-        } else {
+    const int n = quad_node(bk.begin);
+    if (n >= bk.end) return;
+    double B[9];
+    pcg_block<R, NR>(in, ev, inc_ptr, inc, mass, fixed, n, B);
+    if ((threadIdx.x & 3) != 0) return;
+    if (in.pcg == 1) {
+        const float d[3] = {(float)B[0], (float)B[4], (float)B[8]};
+        st3(dinv, n, d);
+    } else {
 #pragma unroll
-            for (int i = 0; i < 9; i++) binv[9 * (int64_t)n + i] = (float)B[i];
-        }
+        for (int i = 0; i < 9; i++) binv[9 * (int64_t)n + i] = (float)B[i];
     }
 }
 
