@@ -297,11 +297,13 @@ int sofa_amd_engine_set_dot_segments(sofa_amd_engine eng, int segments, int wind
  * and then refuses a consistent MeshMatrixMass (SOFA_AMD_EINVAL at commit). */
 int sofa_amd_engine_set_dot_order(sofa_amd_engine eng, int order);
 
-/* Tiled engines: the CG operator kernel's variant -- threads per element and how much element
- * geometry it recomputes from positions: 0: 1 thread per element (512 per tile), rotation and
- * rest coordinates recomputed (the default); 1: 512 threads, rotation only; 2: 256 threads (2
- * elements each), rotation and rest coordinates; 3: 256 threads, rotation only.  Variants differ
- * in rounding only (the order of block sums, geometry recomputed in the engine's precision).
+/* Tiled engines: the CG operator kernel's variant -- threads per element and where an element's
+ * geometry comes from: 0: 1 thread per element (512 per tile), rest shape and K from the rest
+ * positions in the engine's precision (the default); 1: 512 threads, rest shape and K as set up in
+ * double and rounded; 2, 3: as 0 and 1 with 256 threads (2 elements each).  In the reference
+ * order 0 and 2 recompute rotation and rest shape in the kernel, 1 and 3 the rotation only, all
+ * four with the same bits; otherwise variants differ in rounding only (the order of block sums,
+ * float geometry).
  * sofa_amd_engine_autotune times all of them on the committed scenes (`reps` launches each, one
  * launch over every scene) and keeps the fastest, a later variant replacing an earlier one only
  * when faster by 1 % or more; it must run before the first step.  `chosen`

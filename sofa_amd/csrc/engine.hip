@@ -372,7 +372,6 @@ struct InnerCg {
     float *r, *p, *q, *d, *sp;
     float* z;                       // with a preconditioner: z = P^-1 r, staged by the operator
     const float *dinv, *binv;       // ... the inverted diagonal (3 per node) / 3x3 blocks (9)
-    const float *x, *x0;            // float positions and rest positions (geometry recomputed)
     double *pden, *prho;            // prho: |r|^2 partials per node block (iteration 1 included)
 };
 void launch_inner_cg(const InnerCg& c, hipStream_t s);
@@ -425,8 +424,9 @@ struct EngineT : EngineBase {
     VT *sp0 = nullptr, *sp1 = nullptr;
     double *pbb = nullptr, *pden = nullptr, *prho = nullptr;
     // MIXED: float element record and inner CG vectors, inner scene records, |r|^2 partials
-    float *kmat32 = nullptr, *emass32 = nullptr;   // MIXED: float K entries and edge masses
-    float *x32 = nullptr, *x0_32 = nullptr;   // MIXED: float positions (per step) and rest positions
+    // the float operator's record (FP32, SPLIT, MIXED's inner CG): rest shape and K in float (k_rest_float)
+    float *restf = nullptr, *kmatf = nullptr;
+    float *rot32 = nullptr, *emass32 = nullptr;    // MIXED: float rotations (per step) and edge masses
     float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *d32 = nullptr, *sp32 = nullptr;
     double *pden32 = nullptr, *prho32 = nullptr, *prr = nullptr;
     InstDev* inst_in = nullptr;
@@ -486,8 +486,8 @@ struct EngineT : EngineBase {
         void* ptrs[] = {x, v, f, b, r, p, q, xcg, mass, fixed, inc_ptr, inc, tet, rot, rest, kmat, ef, ef2,
                         inst, partial, partial2, tiles_d, ranges_d, ltet, ln_gid, ln_inc_ptr, ln_pslot, sh_gid, sh_ptr,
                         ln_inc, sp0, sp1, pbb, pden, prho, p2, em_ptr, em_nbr, em_val, emass, osc_node,
-                        osc_mean, osc_amp, osc_w, osc_phase, kmat32, emass32, r32, p32, q32,
-                        d32, sp32, pden32, prho32, prr, inst_in, sh_of, nd, x0, x32, x0_32, contact, inc_rank, pinv, zv,
+                        osc_mean, osc_amp, osc_w, osc_phase, restf, kmatf, rot32, emass32, r32, p32, q32,
+                        d32, sp32, pden32, prho32, prr, inst_in, sh_of, nd, x0, contact, inc_rank, pinv, zv,
                         inc_arank, sh_acnt, ln_lead, dinv32, binv32, z32};
         for (void* ptr : ptrs)
             if (ptr) (void)hipFree(ptr);
@@ -565,7 +565,8 @@ struct EngineT : EngineBase {
         int nE = 0;
         std::vector<int4> tet;                       // placement order, scene-local node ids
         std::vector<R> rot, rest, kmat, emass;       // SoA with stride nE
-        std::vector<float> k_lo, em_lo;     // MIXED
+        std::vector<float> k_lo;            // the float operator's K
+        std::vector<float> em_lo;           // MIXED
         std::vector<double> mass;                    // per node (DiagonalMass / MeshMatrixMass)
         std::vector<int> inc_ptr, inc;               // n + 1, 4 nE: position * 4 + vertex
         std::vector<int8_t> fixed;
@@ -582,7 +583,8 @@ struct EngineT : EngineBase {
         h.tet.resize(nE);
         h.rot.assign(9 * (size_t)nE, (R)0); h.rest.assign(NR * (size_t)nE, (R)0); h.kmat.assign(3 * (size_t)nE, (R)0);
         h.emass.assign(nE, (R)0);
-        if (mixed) { h.k_lo.assign(3 * (size_t)nE, 0.f); h.em_lo.assign(nE, 0.f); }
+        if (float_operator()) h.k_lo.assign(3 * (size_t)nE, 0.f);
+        if (mixed) h.em_lo.assign(nE, 0.f);
         h.mass.assign(n, 0.0);
         std::vector<int> cnt(n + 1, 0);
         double mass_sum = 0.0;                       // DiagonalMass computeVertexMass total
@@ -605,7 +607,7 @@ struct EngineT : EngineBase {
                 for (int k = 0; k < 6; k++) h.rest[k * (size_t)nE + pe] = (R)ei.rest[pick[k]];
             }
             for (int k = 0; k < 3; k++) h.kmat[k * (size_t)nE + pe] = (R)ei.k[k];
-            if (mixed)
+            if (float_operator())
                 for (int k = 0; k < 3; k++) h.k_lo[k * (size_t)nE + pe] = (float)ei.k[k];
             for (int k = 0; k < 4; k++) cnt[t[k] + 1]++;
             if (s.mass_kind == SOFA_AMD_MASS_DIAGONAL) {
@@ -959,7 +961,7 @@ struct EngineT : EngineBase {
         em_val = nullptr; emass = nullptr; osc_node = nullptr; osc_mean = osc_amp = osc_w = osc_phase = nullptr;
         inst = nullptr; partial = partial2 = nullptr; tiles_d = nullptr; ranges_d = nullptr; ltet = nullptr;
         ln_gid = ln_inc_ptr = ln_pslot = sh_gid = sh_ptr = nullptr; ln_inc = nullptr; sp0 = sp1 = nullptr;
-        pbb = pden = prho = nullptr; kmat32 = emass32 = nullptr; x32 = x0_32 = nullptr;
+        pbb = pden = prho = nullptr; restf = kmatf = rot32 = emass32 = nullptr;
         r32 = p32 = q32 = d32 = sp32 = nullptr; pden32 = prho32 = prr = nullptr; inst_in = nullptr; sh_of = nullptr; inc_rank = nullptr;
         pinv = nullptr; zv = nullptr; inc_arank = nullptr; sh_acnt = nullptr; ln_lead = nullptr; dinv32 = nullptr;
         binv32 = z32 = nullptr;
@@ -989,6 +991,7 @@ struct EngineT : EngineBase {
         contact = dalloc<int8_t>(N);
         HIPCHK(hipMemset(contact, 0, std::max<int64_t>(1, N)));
         tet = dalloc<int4>(E); rot = dalloc<R>(9 * E); rest = dalloc<R>(NR * E); kmat = dalloc<R>(3 * E);
+        if (float_operator()) { restf = dalloc<float>(6 * E); kmatf = dalloc<float>(3 * E); }
         emass = dalloc<R>(E); ltet = dalloc<uint2>(E); ef = dalloc<VT>(12 * E);
         inc = dalloc<int>(cap.inc); ln_inc = dalloc<uint16_t>(cap.inc);
         tiles_d = dalloc<TileDesc>(cap.tile);
@@ -1004,9 +1007,9 @@ struct EngineT : EngineBase {
         for (double* pb : {pbb, pden}) HIPCHK(hipMemset(pb, 0, std::max<size_t>(1, np) * sizeof(double)));
         HIPCHK(hipMemset(prho, 0, std::max<int64_t>(1, cap.nblk) * sizeof(double)));
         if (mixed) {
-            kmat32 = dalloc<float>(3 * E);
+            rot32 = dalloc<float>(9 * E);
             emass32 = dalloc<float>(E);
-            for (float** vec : {&r32, &p32, &q32, &d32, &x32, &x0_32}) {
+            for (float** vec : {&r32, &p32, &q32, &d32}) {
                 *vec = dalloc<float>(3 * N);
                 HIPCHK(hipMemset(*vec, 0, 3 * N * sizeof(float)));
             }
@@ -1077,15 +1080,25 @@ struct EngineT : EngineBase {
         for (int k = 0; k < NR; k++) put_at(rest, k * Etot + eb0, th.eh.rest.data() + k * (size_t)nE, nE);
         for (int k = 0; k < 3; k++) put_at(kmat, k * Etot + eb0, th.eh.kmat.data() + k * (size_t)nE, nE);
         put_at(emass, eb0, th.eh.emass);
+        if (float_operator() && nE > 0) {
+            for (int k = 0; k < 3; k++) put_at(kmatf, k * Etot + eb0, th.eh.k_lo.data() + k * (size_t)nE, nE);
+            const bool one = one_material(s);
+            double ks[3] = {0, 0, 0};
+            if (one) host::material_factors(s.young[0], s.poisson[0], ks);
+            const double* xd = nullptr;
+            const float* xf = nullptr;
+            if constexpr (std::is_same<VT, double>::value) xd = x0;
+            else xf = x0;
+            // on the stream of the copies around it
+            k_rest_float<<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, nullptr>>>(
+                tet, eb0, eb0 + nE, Etot, xd, xf, one, ks[0], ks[1], ks[2], restf, kmatf);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipStreamSynchronize(nullptr));
+        }
         put_at(ltet, eb0, P.ltet);
         put_at(ln_inc, ib0, P.ln_inc);
         if (mixed) {
-            for (int k = 0; k < 3; k++) put_at(kmat32, k * Etot + eb0, th.eh.k_lo.data() + k * (size_t)nE, nE);
             put_at(emass32, eb0, th.eh.em_lo);
-            std::vector<float> xf(3 * (size_t)(n + 1), 0.0f);
-            for (int i = 0; i < 3 * n; i++) xf[i] = (float)s.rest[i];
-            put_at(x32, 3 * (int64_t)nb0, xf);
-            put_at(x0_32, 3 * (int64_t)nb0, xf);
         }
         // tiles and their local nodes (each tile's list keeps one extra entry for its end)
         const int T = (int)P.t_ebegin.size();
@@ -1402,6 +1415,8 @@ struct EngineT : EngineBase {
     // the scenes are placed): shared nodes summed incidence by incidence in element order, every
     // CG dot product node after node (k_seqdot); the trajectories are then the FP64 parity
     // path's in its sequential dot order, bit for bit
+    // the CG operator computes elements in float
+    bool float_operator() const { return tiled && (mixed || std::is_same<R, float>::value); }
     bool exact_tiled() const { return tiled && !mixed && seq_dots && std::is_same<R, double>::value; }
 
     // one step in the reference's summation order (FP64 tiled engines): per CG iteration the tile
@@ -1476,19 +1491,18 @@ struct EngineT : EngineBase {
         k_step_end_tiled<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
     }
 
-    // the tile operator's launch shape and how much geometry it recomputes (results of the
-    // variants differ in rounding only: block sums and geometry recomputed in R instead of
-    // rounded from the host's double); picked by sofa_amd_engine_autotune or set explicitly
+    // the tile operator's launch shape and where its geometry comes from (results of the variants
+    // differ in rounding only: block sums, float rest shapes); picked by
+    // sofa_amd_engine_autotune or set explicitly
     static constexpr int kApplyVariants = 4;
     static int variant_threads(int v) { return v < 2 ? 512 : 256; }
-    static int variant_geometry(int v) { return (v & 1) ? 1 : 2; }
     int apply_variant = 0;
     void launch_apply(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp,
                       const double* pin, double* pd, int pin_nodes) {
         if constexpr (std::is_same<R, double>::value) {
-            if (exact_tiled()) {   // scalars from k_seqdot: no partial sums reduced
-                if (cur->plane) launch_apply_t<false, true, true>(na, s, ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
-                else launch_apply_t<false, false, true>(na, s, ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
+            if (exact_tiled()) {   // scalars from the dot-product kernels: no partial sums reduced
+                if (cur->plane) launch_exact_t<true>(na, s, ta, it, rr, pp, qq, sp);
+                else launch_exact_t<false>(na, s, ta, it, rr, pp, qq, sp);
                 return;
             }
         }
@@ -1501,14 +1515,21 @@ struct EngineT : EngineBase {
             else launch_apply_t<false, false>(na, s, ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
         }
     }
-    template <bool WIDE, bool PLANE, bool EXACT = false>
+    template <bool WIDE, bool PLANE>
     void launch_apply_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp,
                         const double* pin, double* pd, int pin_nodes) {
+        if (variant_threads(apply_variant) == 512)
+            k_tile_apply<R, NR, VT, 512, WIDE, PLANE><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
+        else
+            k_tile_apply<R, NR, VT, 256, WIDE, PLANE><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
+    }
+    template <bool PLANE>
+    void launch_exact_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp) {
         switch (apply_variant) {
-        case 1: k_tile_apply<R, NR, VT, 512, 1, WIDE, PLANE, EXACT><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0); break;
-        case 2: k_tile_apply<R, NR, VT, 256, 2, WIDE, PLANE, EXACT><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0); break;
-        case 3: k_tile_apply<R, NR, VT, 256, 1, WIDE, PLANE, EXACT><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0); break;
-        default: k_tile_apply<R, NR, VT, 512, 2, WIDE, PLANE, EXACT><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0); break;
+        case 1: k_tile_exact<R, NR, VT, 512, 1, PLANE><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, x, x0); break;
+        case 2: k_tile_exact<R, NR, VT, 256, 2, PLANE><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, x, x0); break;
+        case 3: k_tile_exact<R, NR, VT, 256, 1, PLANE><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, x, x0); break;
+        default: k_tile_exact<R, NR, VT, 512, 2, PLANE><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, x, x0); break;
         }
     }
     // times every variant on the engine's scenes (all of them in one launch, `reps` launches
@@ -1528,6 +1549,10 @@ struct EngineT : EngineBase {
         int best = 0;
         float best_us = 0;
         for (int v = 0; v < kApplyVariants; v++) {
+            if (!exact_tiled() && (v & 1)) {   // the kernel of v - 1 on another rest shape
+                if (us_out) us_out[v] = us_out[v - 1];
+                continue;
+            }
             apply_variant = v;
             for (int i = 0; i < 2; i++) launch_apply(cur->na, s, ta, 2, r, p, q, sp0, prho, pden, 0);
             HIPCHK(hipEventRecord(e0, s));
@@ -1567,9 +1592,13 @@ struct EngineT : EngineBase {
         ta.fixed = fixed;
         ta.contact = contact;
         ta.emass = emass;
-        ta.x_lo = nullptr;
         ta.nd = nd;
-        ta.dinv = nullptr;
+        ta.rot = rot;
+        ta.rest = rest;
+        ta.kmat = kmat;
+        if constexpr (std::is_same<R, float>::value)
+            if (!(apply_variant & 1)) { ta.rest = restf; ta.kmat = kmatf; }
+        ta.rot32 = rot32;
         return ta;
     }
 
@@ -1596,11 +1625,10 @@ struct EngineT : EngineBase {
         k_step_end_tiled<<<(n + 63) / 64, 64, 0, s>>>(cur->scenes, n, inst);
     }
 
-    // MIXED step: FP64 RHS (which also writes the float rotations), refinement sweeps with the
+    // MIXED step: FP64 RHS (which also writes the inner operator's float rotations), refinement sweeps with the
     // FP32 inner CG, FP64 update
     void launch_step_mixed(int n, hipStream_t s) {
-        TileArgs<R, NR> ta = tile_args();
-        ta.x_lo = x32;                 // the inner operator recomputes the rotations from these
+        const TileArgs<R, NR> ta = tile_args();
         const FinBlk* fb = (const FinBlk*)cur->b;
         const NodeBlk* nb = (const NodeBlk*)cur->c;
         const SharedNodes sn{sh_gid, sh_ptr, sh_of, sh_acnt};
@@ -1608,22 +1636,21 @@ struct EngineT : EngineBase {
         ic.ta.tiles = ta.tiles;
         ic.ta.inst = inst_in;
         ic.ta.ranges = ranges_d;
-        // rotations and rest coordinates are recomputed from x32 / x0_32: only K is read
-        ic.ta.ev = ElemView<float, 6>{tet, nullptr, nullptr, kmat32, Etot};
+        ic.ta.ev = ElemView<float, 6>{tet, nullptr, nullptr, nullptr, Etot};
         ic.ta.ltet = ltet;
         ic.ta.tn = ta.tn;
         ic.ta.mass = mass;
         ic.ta.fixed = fixed;
         ic.ta.contact = contact;
         ic.ta.emass = emass32;
-        ic.ta.x_lo = nullptr;
         ic.ta.nd = nullptr;
-        // PCGLinearSolver with a Jacobi preconditioner: the inner CG runs preconditioned
-        ic.ta.dinv = nullptr;   // the preconditioner acts in the node kernels (z), not in the operator
+        ic.ta.rot = rot32; ic.ta.rest = restf; ic.ta.kmat = kmatf;
+        ic.ta.rot32 = nullptr;
+        // PCGLinearSolver with a Jacobi preconditioner: the inner CG runs preconditioned (in the node
+        // kernels: the operator reads z)
         ic.z = cur->pcg ? z32 : nullptr;
         ic.dinv = dinv32;
         ic.binv = binv32;
-        ic.x = x32; ic.x0 = x0_32;
         ic.fb = fb; ic.nb = nb;
         ic.na = cur->na; ic.nfb = cur->nb; ic.nnb = cur->nc; ic.maxit = cur->maxit;
         ic.wide = cur->maxpart > kWavePartials;
@@ -2038,12 +2065,18 @@ struct EngineT : EngineBase {
             iterate_exact(ev, na, 1, s, nullptr, nullptr);
             k_finalize<false><<<1, kBlock, 0, s>>>(cur->scenes, inst, partial, exact_ready());
         } else {
-            const TileArgs<R, NR> ta = tile_args();
+            TileArgs<R, NR> ta = tile_args();
+            const int64_t nE = (int64_t)scenes[scene].tets.size() / 4, e0 = elem_begin(scene);
+            R* const rot_cg = reinterpret_cast<R*>(ef);   // scratch of the force calls: 12 VT per element
+            bool exact = false;
+            if constexpr (std::is_same<R, double>::value) exact = exact_tiled();
+            if (!exact && nE > 0) {   // the rotations of the engine's positions (ev.rot keeps addForce's)
+                k_rotations<R, VT><<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, s>>>(tet, e0, e0 + nE, x, rot_cg, Etot);
+                ta.rot = rot_cg;
+            }
             const FinBlk* fb = (const FinBlk*)cur->b;
             const NodeBlk* nbk = (const NodeBlk*)cur->c;
             const SharedNodes sn{sh_gid, sh_ptr, sh_of, sh_acnt};
-            bool exact = false;
-            if constexpr (std::is_same<R, double>::value) exact = exact_tiled();
             if (exact) {
                 if constexpr (std::is_same<R, double>::value) {
                     if (cur->nc > 0)
@@ -2281,20 +2314,12 @@ EngineBase* make_engine_split() {
 void launch_inner_cg(const InnerCg& c, hipStream_t s) {
     const float* rs = c.z ? c.z : c.r;   // the vector p is formed from (p = rs + beta p)
     for (int it = 1; it <= c.maxit; it++) {
-        if (c.na > 0)
-        {
-            if (c.wide && c.plane)
-                k_tile_apply<float, 6, float, kTileThreads, 2, true, true><<<c.na, kTileThreads, 0, s>>>(
-                    c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, c.x, c.x0);
-            else if (c.wide)
-                k_tile_apply<float, 6, float, kTileThreads, 2, true, false><<<c.na, kTileThreads, 0, s>>>(
-                    c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, c.x, c.x0);
-            else if (c.plane)
-                k_tile_apply<float, 6, float, kTileThreads, 2, false, true><<<c.na, kTileThreads, 0, s>>>(
-                    c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, c.x, c.x0);
-            else
-                k_tile_apply<float, 6, float, kTileThreads, 2, false, false><<<c.na, kTileThreads, 0, s>>>(
-                    c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, c.x, c.x0);
+        if (c.na > 0) {
+            const auto op = c.wide ? (c.plane ? k_tile_apply<float, 6, float, kTileThreads, true, true>
+                                              : k_tile_apply<float, 6, float, kTileThreads, true, false>)
+                                   : (c.plane ? k_tile_apply<float, 6, float, kTileThreads, false, true>
+                                              : k_tile_apply<float, 6, float, kTileThreads, false, false>);
+            op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1);
         }
         if (c.nnb > 0)
             k_update<float><<<c.nnb, kBlock, 0, s>>>(c.nb, c.ta.inst, c.ta.ranges, it, c.sn, c.sp, c.ta.mass, c.ta.fixed,

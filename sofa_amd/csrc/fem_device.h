@@ -227,6 +227,28 @@ __device__ __forceinline__ void normalize3(R& x, R& y, R& z) {
     if (n > Eps<R>::v) { x /= n; y /= n; z /= n; }
 }
 
+// a b - c d and a0 b0 + a1 b1 + a2 b2 of the element geometry.  double: every product and sum rounded,
+// as the reference computes them.  float: fused in this order, in every kernel and whatever the compiler
+// would choose around it, so that geometry computed in different kernels has the same bits.
+template <typename R>
+__device__ __forceinline__ R cross_r(R a, R b, R c, R d) {
+#pragma clang fp contract(off)
+    if constexpr (std::is_same<R, float>::value) return __builtin_fmaf(a, b, -(c * d));
+    else return a * b - c * d;
+}
+template <typename R>
+__device__ __forceinline__ R dot3_r(R a0, R a1, R a2, R b0, R b1, R b2) {
+#pragma clang fp contract(off)
+    if constexpr (std::is_same<R, float>::value) {
+        return __builtin_fmaf(a2, b2, __builtin_fmaf(a0, b0, a1 * b1));
+    } else {
+        R r = a0 * b0;
+        r += a1 * b1;
+        r += a2 * b2;
+        return r;
+    }
+}
+
 // FP32: one hardware reciprocal square root (v_rsq_f32, 1 ulp) and three multiplies instead of a
 // correctly rounded square root and three divisions.  The FP32 engine's error budget is far above
 // the ulp this costs; every FP32 kernel calls this same function, so a rotation recomputed from
@@ -234,9 +256,7 @@ __device__ __forceinline__ void normalize3(R& x, R& y, R& z) {
 template <>
 __device__ __forceinline__ void normalize3<float>(float& x, float& y, float& z) {
 #pragma clang fp contract(off)
-    float n2 = x * x;
-    n2 += y * y;
-    n2 += z * z;
+    const float n2 = dot3_r(x, y, z, x, y, z);
     if (n2 > Eps<float>::v * Eps<float>::v) {
         const float s = __builtin_amdgcn_rsqf(n2);
         x *= s; y *= s; z *= s;
@@ -418,11 +438,11 @@ __device__ __forceinline__ void rotation_large(const R p0[3], const R p1[3], con
     R ex0 = p1[0] - p0[0], ex1 = p1[1] - p0[1], ex2 = p1[2] - p0[2];
     normalize3(ex0, ex1, ex2);
     R ey0 = p2[0] - p0[0], ey1 = p2[1] - p0[1], ey2 = p2[2] - p0[2];
-    R ez0 = ex1 * ey2 - ex2 * ey1, ez1 = ex2 * ey0 - ex0 * ey2, ez2 = ex0 * ey1 - ex1 * ey0;
+    R ez0 = cross_r(ex1, ey2, ex2, ey1), ez1 = cross_r(ex2, ey0, ex0, ey2), ez2 = cross_r(ex0, ey1, ex1, ey0);
     normalize3(ez0, ez1, ez2);
-    ey0 = ez1 * ex2 - ez2 * ex1;
-    ey1 = ez2 * ex0 - ez0 * ex2;
-    ey2 = ez0 * ex1 - ez1 * ex0;
+    ey0 = cross_r(ez1, ex2, ez2, ex1);
+    ey1 = cross_r(ez2, ex0, ez0, ex2);
+    ey2 = cross_r(ez0, ex1, ez1, ex0);
     rot[0] = ex0; rot[1] = ey0; rot[2] = ez0;
     rot[3] = ex1; rot[4] = ey1; rot[5] = ez1;
     rot[6] = ex2; rot[7] = ey2; rot[8] = ez2;
@@ -441,12 +461,7 @@ __device__ __forceinline__ void rest_frame(const R p0[4][3], R* out) {
 #pragma unroll
     for (int k = 0; k < 4; k++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-            R r = rot[i] * p0[k][0];
-            r += rot[3 + i] * p0[k][1];
-            r += rot[6 + i] * p0[k][2];
-            ri[k][i] = r;
-        }
+        for (int i = 0; i < 3; i++) ri[k][i] = dot3_r(rot[i], rot[3 + i], rot[6 + i], p0[k][0], p0[k][1], p0[k][2]);
 #pragma unroll
     for (int k = 1; k < 4; k++)
 #pragma unroll
@@ -471,10 +486,8 @@ __device__ __forceinline__ void stiffness_from_volume(const R p0[4][3], const do
     const R a0 = p0[1][0] - p0[0][0], a1 = p0[1][1] - p0[0][1], a2 = p0[1][2] - p0[0][2];
     const R b0 = p0[2][0] - p0[0][0], b1 = p0[2][1] - p0[0][1], b2 = p0[2][2] - p0[0][2];
     const R c0 = p0[3][0] - p0[0][0], c1 = p0[3][1] - p0[0][1], c2 = p0[3][2] - p0[0][2];
-    const R x0 = a1 * b2 - a2 * b1, x1 = a2 * b0 - a0 * b2, x2 = a0 * b1 - a1 * b0;
-    R d = x0 * c0;
-    d += x1 * c1;
-    d += x2 * c2;
+    const R x0 = cross_r(a1, b2, a2, b1), x1 = cross_r(a2, b0, a0, b2), x2 = cross_r(a0, b1, a1, b0);
+    const R d = dot3_r(x0, x1, x2, c0, c1, c2);
     if constexpr (std::is_same<R, float>::value) {
         // FP32: 36 V = 6 |d|, one hardware reciprocal (1 ulp) for the three entries
         const float inv = __builtin_amdgcn_rcpf(fabsf(d) * 6.0f);
@@ -627,8 +640,22 @@ __device__ __forceinline__ void elem_force_r(const R p[4][3], const R* rin, cons
     elem_force_core<R, NR>(p, rc, g, k3, rot, c);
 }
 
+// k_mul with its products fused in a fixed order in float, whatever the compiler would choose around it (a
+// solve that stops before it converges shows the choice); DIAG: which product of the second is rounded first
+template <bool DIAG, typename R>
+__device__ __forceinline__ void k_mul_fixed(const R k[3], const R JtD[6], R KJ[6]) {
+    k_mul(k, JtD, KJ);
+    if constexpr (std::is_same<R, float>::value) {
+        const float K00 = k[0], K01 = k[1], a = K01 * JtD[1];
+        KJ[0] = __builtin_fmaf(K01, JtD[2], __builtin_fmaf(K00, JtD[0], a));
+        KJ[1] = __builtin_fmaf(K01, JtD[2], DIAG ? __builtin_fmaf(K01, JtD[0], K00 * JtD[1])
+                                                 : __builtin_fmaf(K00, JtD[1], K01 * JtD[0]));
+        KJ[2] = __builtin_fmaf(K00, JtD[2], __builtin_fmaf(K01, JtD[0], a));
+    }
+}
+
 // applyStiffnessCorotational with the element record in registers
-template <typename R, int NR>
+template <typename R, int NR, bool DIAG = false>
 __device__ __forceinline__ void elem_dforce_r(const R rot[9], const R* rin, const R k3[3], const R u[12],
                                               R fact, R c[12]) {
     R X[12];
@@ -642,7 +669,7 @@ __device__ __forceinline__ void elem_dforce_r(const R rot[9], const R* rin, cons
     jgroups_r<R, NR>(rin, g);
     R JtD[6], KJ[6], F[12];
     jt_mul<R, NR>(g, X, JtD);
-    k_mul(k3, JtD, KJ);
+    k_mul_fixed<DIAG>(k3, JtD, KJ);
 #pragma unroll
     for (int k = 0; k < 6; k++) KJ[k] *= fact;
     j_mul(g, KJ, F);

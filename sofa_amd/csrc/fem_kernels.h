@@ -40,28 +40,55 @@ struct NodeArrays {
 constexpr int kMassUniform = 0, kMassDiagonal = 1, kMassMatrix = 2, kMassMatrixLumped = 3;
 constexpr double kLumpTet = 2.5;   // MeshMatrixMass lumping coefficient of tetrahedra (MeshMatrixMass.inl:1476-1489)
 
-// vertex part of addMDx: UniformMass.inl:403-419, DiagonalMass.inl:536-559, MeshMatrixMass.inl:1987-2030
+// one component of mass_mdx, m the node's mass (uniform: the scene's).  FUSE: the product and the sum
+// rounded once, in float (left to the compiler, its contraction would depend on the code around it)
+template <bool FUSE, typename VT>
+__device__ __forceinline__ VT mass_add(VT a, VT b, VT c) {
+#pragma clang fp contract(off)
+    if constexpr (std::is_same<VT, float>::value) {
+        if constexpr (FUSE) return __builtin_fmaf(a, b, c);
+        float t = a * b;
+        asm("" : "+v"(t));
+        return c + t;
+    } else {
+        return c + a * b;
+    }
+}
 template <typename VT>
+__device__ __forceinline__ void mass_term(const InstDev& in, VT m, double factor, VT d, VT& out) {
+    const VT fct = (VT)factor;
+    if (in.mass_kind == kMassUniform) {
+        if (factor != 1.0) m *= fct;
+        out = mass_add<true>(d, m, out);
+    } else if (in.mass_kind == kMassDiagonal && factor == 1.0) {
+        out = mass_add<true>(d, m, out);
+    } else if (in.mass_kind == kMassMatrixLumped) {
+        out = mass_add<true>((d * m) * (VT)kLumpTet, fct, out);
+    } else {
+        out = mass_add<true>(d * m, fct, out);
+    }
+}
+
+// vertex part of addMDx: UniformMass.inl:403-419, DiagonalMass.inl:536-559, MeshMatrixMass.inl:1987-2030
+// SPLIT_Z: onto a sum (the right-hand side) z is rounded twice in float too
+template <bool SPLIT_Z = false, typename VT>
 __device__ __forceinline__ void mass_mdx(const InstDev& in, const NodeArrays& na, int n, double factor,
                                          const VT d[3], VT out[3]) {
+    const auto add = [&](VT a0, VT a1, VT a2, VT f) {
+        out[0] = mass_add<true>(a0, f, out[0]);
+        out[1] = mass_add<true>(a1, f, out[1]);
+        out[2] = mass_add<!SPLIT_Z>(a2, f, out[2]);
+    };
+    const VT fct = (VT)factor;
     if (in.mass_kind == kMassUniform) {
         VT m = (VT)in.vertex_mass;
-        if (factor != 1.0) m *= (VT)factor;
-        out[0] += d[0] * m; out[1] += d[1] * m; out[2] += d[2] * m;
-    } else if (in.mass_kind == kMassDiagonal) {
-        const VT m = (VT)na.mass[n];
-        if (factor == 1.0) {
-            out[0] += d[0] * m; out[1] += d[1] * m; out[2] += d[2] * m;
-        } else {
-            const VT fct = (VT)factor;
-            out[0] += (d[0] * m) * fct; out[1] += (d[1] * m) * fct; out[2] += (d[2] * m) * fct;
-        }
-    } else if (in.mass_kind == kMassMatrix) {
-        const VT m = (VT)na.mass[n], fct = (VT)factor;
-        out[0] += (d[0] * m) * fct; out[1] += (d[1] * m) * fct; out[2] += (d[2] * m) * fct;
+        if (factor != 1.0) m *= fct;
+        add(d[0], d[1], d[2], m);
     } else {
-        const VT m = (VT)na.mass[n], fct = (VT)factor, lc = (VT)kLumpTet;
-        out[0] += ((d[0] * m) * lc) * fct; out[1] += ((d[1] * m) * lc) * fct; out[2] += ((d[2] * m) * lc) * fct;
+        const VT m = (VT)na.mass[n], lc = (VT)kLumpTet;
+        if (in.mass_kind == kMassDiagonal && factor == 1.0) add(d[0], d[1], d[2], m);
+        else if (in.mass_kind == kMassMatrixLumped) add((d[0] * m) * lc, (d[1] * m) * lc, (d[2] * m) * lc, fct);
+        else add(d[0] * m, d[1] * m, d[2] * m, fct);
     }
 }
 
@@ -188,16 +215,7 @@ __device__ __forceinline__ void precond_apply(int kind, const double* __restrict
 template <typename VT>
 __device__ __forceinline__ void mass_mdx_1(const InstDev& in, const double* __restrict__ mass, int n, double factor,
                                            VT d, VT& out) {
-    if (in.mass_kind == kMassUniform) {
-        VT m = (VT)in.vertex_mass;
-        if (factor != 1.0) m *= (VT)factor;
-        out += d * m;
-    } else {
-        const VT m = (VT)mass[n], fct = (VT)factor;
-        if (in.mass_kind == kMassDiagonal && factor == 1.0) out += d * m;
-        else if (in.mass_kind == kMassMatrixLumped) out += ((d * m) * (VT)kLumpTet) * fct;
-        else out += (d * m) * fct;
-    }
+    mass_term(in, in.mass_kind == kMassUniform ? (VT)in.vertex_mass : (VT)mass[n], factor, d, out);
 }
 
 // the end of a node kernel of three threads per node: each node's three products added in dot3d's

@@ -19,6 +19,7 @@
 #pragma once
 
 #include "fem_device.h"
+#include "tiling.h"
 
 namespace sofa_amd {
 
@@ -27,8 +28,9 @@ namespace sofa_amd {
 #endif
 constexpr int kTileElems = SOFA_AMD_TILE_ELEMS;   // max elements per tile
 constexpr int kTileNodes = SOFA_AMD_TILE_ELEMS;   // max distinct nodes per tile
-// incidences are uint16 contribution slots (row 3 v + c of 12 rows of kTileElems)
-static_assert(12 * kTileElems <= 65536, "contribution slots must fit in 16 bits");
+constexpr int kTileRow = slot_row(kTileElems);    // a row of contributions in LDS
+// incidences are uint16 contribution slots (row 3 v + c of 12 rows of kTileRow)
+static_assert(12 * kTileRow <= 65536, "contribution slots must fit in 16 bits");
 #ifndef SOFA_AMD_NODES_PER_THREAD
 #define SOFA_AMD_NODES_PER_THREAD 2
 #endif
@@ -211,10 +213,10 @@ struct TileArgs {
     const int8_t* __restrict__ fixed;
     int8_t* __restrict__ contact;        // PlaneForceField contacts of the step (per node)
     const R* __restrict__ emass;        // per element rho V / 20 (consistent MeshMatrixMass), else unused
-    float* __restrict__ x_lo;           // MIXED engines: float copy of the positions (written by the RHS)
-    double* __restrict__ nd;            // reference order: per-node dot terms for k_seqdot
-    const float* __restrict__ dinv;     // MIXED inner CG with a Jacobi preconditioner: the inverted
-                                        // diagonal per node (z = dinv r); null: plain CG
+    double* __restrict__ nd;            // reference order: per-node dot terms
+    // the operator's element record, SoA: rotations (written by the step's force pass), rest shape, K
+    const R *rot, *rest, *kmat;
+    float* rot32;                       // MIXED: the inner operator's rotations, written by the force pass
 };
 
 // consistent-mass edge terms of one element, folded into its nodal contributions (which the
@@ -230,7 +232,7 @@ __device__ __forceinline__ void add_edge_mass(R mf, const R u[12], R c[12]) {
     }
 }
 
-// acc (+|-)= the node's element contributions lc[slot + c kTileElems] in incidence-list order.
+// acc (+|-)= the node's element contributions lc[slot + c kTileRow] in incidence-list order.
 // Four incidences per round: their slots are read together, then their values, so a round
 // waits on LDS twice instead of eight times; the adds keep the list order (same bits).
 template <bool SUB, typename R, typename VT>
@@ -244,7 +246,7 @@ __device__ __forceinline__ void sum_incidences(const uint16_t* linc, int s0, int
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
-            for (int i = 0; i < 3; i++) v[t][i] = lc[sl[t] + i * kTileElems];
+            for (int i = 0; i < 3; i++) v[t][i] = lc[sl[t] + i * kTileRow];
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -257,13 +259,27 @@ __device__ __forceinline__ void sum_incidences(const uint16_t* linc, int s0, int
         const int sl = linc[s];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            if (SUB) acc[i] -= (VT)lc[sl + i * kTileElems];
-            else acc[i] += (VT)lc[sl + i * kTileElems];
+            if (SUB) acc[i] -= (VT)lc[sl + i * kTileRow];
+            else acc[i] += (VT)lc[sl + i * kTileRow];
         }
     }
 }
 
-// reference order: each incidence's contribution lc[slot + c kTileElems] to its own global slot
+// one component of sum_incidences<true> (row: lc + c kTileRow)
+template <typename R, typename VT>
+__device__ __forceinline__ void sum_component(const uint16_t* linc, int s0, int s1, const R* row, VT& acc) {
+    int s = s0;
+    for (; s + 4 <= s1; s += 4) {
+        R v[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) v[t] = row[linc[s + t]];
+#pragma unroll
+        for (int t = 0; t < 4; t++) acc -= (VT)v[t];
+    }
+    for (; s < s1; s++) acc -= (VT)row[linc[s]];
+}
+
+// reference order: each incidence's contribution lc[slot + c kTileRow] to its own global slot
 // base + rank (the node's slots run in ascending element id, the order its finalize adds them);
 // rank: the tile's incidence ranks, indexed like linc
 template <typename R, typename VT>
@@ -273,7 +289,7 @@ __device__ __forceinline__ void store_incidences(const uint16_t* linc, const uin
         const int sl = linc[s];
         VT* o = sp + 3 * (int64_t)(base + rank[s]);
 #pragma unroll
-        for (int i = 0; i < 3; i++) o[i] = (VT)lc[sl + i * kTileElems];
+        for (int i = 0; i < 3; i++) o[i] = (VT)lc[sl + i * kTileRow];
     }
 }
 
@@ -327,7 +343,7 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
     constexpr int NPT = (kTileNodes + TB - 1) / TB;
     __shared__ R lx[kTileNodes * 3];
     __shared__ R lv[kTileNodes * 3];
-    __shared__ R lc[kTileElems * 12];
+    __shared__ R lc[kTileRow * 12];
     __shared__ uint16_t linc[kTileElems * 4];
     __shared__ int lptr[kTileNodes + 1];
     __shared__ double sh[TB / 64];
@@ -379,10 +395,6 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
         const int j = threadIdx.x + m * TB;
         if (j < td.ln_count) {
             lx[3 * j] = (R)xt[m][0]; lx[3 * j + 1] = (R)xt[m][1]; lx[3 * j + 2] = (R)xt[m][2];
-            if (a.x_lo) {   // every tile of a shared node writes the same value
-                const float xf[3] = {(float)xt[m][0], (float)xt[m][1], (float)xt[m][2]};
-                st3(a.x_lo, gid[m], xf);
-            }
             lv[3 * j] = (R)vt[m][0]; lv[3 * j + 1] = (R)vt[m][1]; lv[3 * j + 2] = (R)vt[m][2];
         }
     }
@@ -413,8 +425,18 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
             elem_force_r<R, NR>(p, rin[m], kk[m], rot[m], c);
 #pragma unroll
             for (int i = 0; i < 9; i++) a.ev.rot[i * a.ev.E + e] = rot[m][i];
+            if (a.rot32) {   // from the positions in float, as a force pass in float has them
+                float pf[3][3], rf[9];
 #pragma unroll
-            for (int i = 0; i < 12; i++) lc[i * kTileElems + k] = c[i];
+                for (int n = 0; n < 3; n++)
+#pragma unroll
+                    for (int i = 0; i < 3; i++) pf[n][i] = (float)p[n][i];
+                rotation_large(pf[0], pf[1], pf[2], rf);
+#pragma unroll
+                for (int i = 0; i < 9; i++) a.rot32[i * a.ev.E + e] = rf[i];
+            }
+#pragma unroll
+            for (int i = 0; i < 12; i++) lc[i * kTileRow + k] = c[i];
         }
     }
     __syncthreads();
@@ -447,14 +469,14 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
 #pragma unroll
                 for (int i = 0; i < 3; i++) u[3 * n + i] = lv[3 * l[n] + i];
             if (in.k_rhs != 0.0) {
-                elem_dforce_r<R, NR>(rot[m], rin[m], kk[m], u, krhs, c);
+                elem_dforce_r<R, NR, std::is_same<VT, double>::value>(rot[m], rin[m], kk[m], u, krhs, c);
             } else {
 #pragma unroll
                 for (int i = 0; i < 12; i++) c[i] = 0;
             }
             if (edge) add_edge_mass((R)in.m_rhs * em[m], u, c);
 #pragma unroll
-            for (int i = 0; i < 12; i++) lc[i * kTileElems + k] = c[i];
+            for (int i = 0; i < 12; i++) lc[i * kTileRow + k] = c[i];
         }
     }
     __syncthreads();
@@ -478,7 +500,7 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
                 }
                 st3(f, g, fn[m]);
                 VT bn[3] = {fn[m][0], fn[m][1], fn[m][2]};
-                if (in.m_rhs != 0.0) mass_mdx(in, NodeArrays{nullptr, nullptr, a.mass, a.fixed}, g, in.m_rhs, vn, bn);
+                if (in.m_rhs != 0.0) mass_mdx<true>(in, NodeArrays{nullptr, nullptr, a.mass, a.fixed}, g, in.m_rhs, vn, bn);
                 sum_incidences<true>(linc, s0, s1, lc, bn);
                 if (touch && in.k_rhs != 0.0) plane_dforce(in, in.k_rhs, vn, bn);
                 bn[0] *= h; bn[1] *= h; bn[2] *= h;
@@ -537,7 +559,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
         }
         st3(f, g, fn);
         VT bn[3] = {fn[0], fn[1], fn[2]};
-        if (in.m_rhs != 0.0) mass_mdx(in, NodeArrays{nullptr, nullptr, mass, fixed}, g, in.m_rhs, vn, bn);
+        if (in.m_rhs != 0.0) mass_mdx<true>(in, NodeArrays{nullptr, nullptr, mass, fixed}, g, in.m_rhs, vn, bn);
         sum_slots<true>(spv, s0, s1, bn);
         if (touch && in.k_rhs != 0.0) plane_dforce(in, in.k_rhs, vn, bn);
         const VT h = (VT)in.b_scale;   // h (firstOrder: 1, b = f)
@@ -556,49 +578,286 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
 }
 
 // ---------------------------------------------------------------------------------------
-// CG iteration `iter` (1-based): K1 tile apply, K2 shared finalize, K3 update.
-// iter = 0 is a plain operator application q = A r (no CG scalars, p untouched), used for
-// the FP64 residual of iterative refinement.
+// CG iteration `iter` (1-based): the operator, then k_update (reference order: k_fin_exact between).
+// iter = 0 is a plain operator application q = A r (no CG scalars, p untouched).
 // ---------------------------------------------------------------------------------------
-// PLANE = false: no scene of the launch has a PlaneForceField (its per-node terms compiled out).
-// GEO: how much element geometry is recomputed from node positions instead of read back, with
-// the functions and operation order of the element set-up and no fused multiply-adds (so the
-// same bits).  0: none (rotation, rest coordinates, K loaded).  1: the rotation, from the
-// current positions x (the ones the force pass used: x changes only after the solve) -- 9 reals
-// less per element, 3 more per tile-local node.  2: also the rotated rest coordinates from the
-// rest positions x0 (initLarge, TetrahedronFEMForceField.inl:835-868) and, for a scene of one
-// material, K from the rest volume -- NR (+ 3) reals less per element, 3 more per local node.
-// EXACT: the reference's summation order -- |b|^2 and r.r come from k_seqdot (InstDev::dots),
-// interior nodes write their p.q term to nd; a shared node's leading run (its first incidences in
-// ascending element id, when they lie in this tile) is summed here after the mass term into the
-// node's first slot, every later incidence goes to a slot of its own (finished by k_fin_exact);
-// no tile partial of p.q is formed.
-template <typename R, int NR, typename VT, int TB = kBlock, int GEO = 0, bool WIDE = true, bool PLANE = true,
-          bool EXACT = false>
+// The operator: one workgroup per tile, TB threads.
+//   1. loads: the elements' records into registers; a thread per tile-local node reads its tables, r, p;
+//   2. by the waves that have nodes: the scalars (rho, the tolerance test, beta), then p = r + beta p and
+//      what the node sums need of each node, staged in LDS;
+//   3. each element's contributions into LDS, 12 rows of kTileRow;
+//   4. a thread per (node, component): the contributions in ascending element id;
+//   5. by the waves that have nodes: interior nodes finished (q), a shared node's sum left as the tile's
+//      partial, p.q as one partial per tile.
+// The element's rotation, rest shape and K are read back (18 floats, 21 doubles), not recomputed from the
+// positions: 460 instead of 610 vector instructions per wave in float.  What bounds it: on a large mesh
+// VALU issue (half of the time), LDS (a third) and the latency of the phases of the four tiles that a CU
+// holds (FP64: two, by registers and LDS); on a small one that latency alone.  Measured, before (geometry
+// recomputed, a thread per node for staging and sums) and after: FP32 1.31M tetrahedra 32.2 -> 29.9 us, 24
+// beams of 0.6M 24.9 -> 22.6, 18,954 7.2 -> 6.6; SPLIT 150k 11.1 -> 10.2; FP64 360k 24.9 -> 22.8.
+// PLANE = false: no scene of the launch has a PlaneForceField; WIDE = false: no scene has more than
+// kWavePartials partials of r.r, which are then in flight with the gathers.
+constexpr int kNodeMass = 1 << 12;   // the node's sum starts from the mass term
+static_assert(4 * kTileElems <= kNodeMass, "a node's first incidence and the flag share 16 bits");
+template <typename R, int NR, typename VT, int TB, bool WIDE, bool PLANE>
 __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, const VT* __restrict__ r,
                                                     VT* __restrict__ p, VT* __restrict__ q, VT* __restrict__ sp,
                                                     const double* __restrict__ pin,   // |b|^2 (iter 1) or r.r partials
                                                     double* __restrict__ pden,
-                                                    int pin_nodes,     // 1: iter-1 |b|^2 partials per node block
-                                                    const VT* __restrict__ x, const VT* __restrict__ x0) {
+                                                    int pin_nodes) {   // 1: iter-1 |b|^2 partials per node block
     constexpr int EPT = kTileElems / TB;                   // elements per thread
     constexpr int NPT = (kTileNodes + TB - 1) / TB;        // tile-local nodes per thread
-    static_assert(kTileElems * 12 >= kTileNodes * 6, "positions are staged in the contribution buffer");
-    __shared__ R lu[kTileNodes * 3];
-    __shared__ R lc[kTileElems * 12];
-    __shared__ uint16_t linc[kTileElems * 4];
-    __shared__ int lptr[kTileNodes + 1];
+    __shared__ VT lu[kTileNodes * 3];        // p (in R), then the nodes' sums
+    __shared__ R lc[kTileRow * 12];
+    __shared__ __align__(8) uint16_t linc[kTileElems * 4];
+    __shared__ VT lmass[kTileNodes];
+    __shared__ uint16_t lnode[kTileNodes];   // first incidence and flags
     __shared__ double sh[TB / 64];
+    __shared__ int halt;
     const TileDesc td = a.tiles[xcd_item()];
     InstDev* ins = &a.inst[td.scene];
     const InstDev in = *ins;
     const Ranges rg = a.ranges[td.scene];
     const bool consistent = (td.flags & kTileConsistent) != 0;
+    const int ninc = 4 * td.e_count;
+    // a refinement sweep that keeps the previous search direction continues CG at its iteration 1
+    const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
+    // p is read from iteration 2 on (or continuing a direction)
+    const bool second = iter > 1 || cont;
+    const int w0 = __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63);   // the wave's first thread
+    // ---- 1. the nodes' tables, the partials, the element records, the incidence table
+    int gid[NPT], psl[NPT], s0[NPT];
+#pragma unroll
+    for (int m = 0; m < NPT; m++)
+        if (w0 + m * TB < td.ln_count) {
+            const unsigned j = min((int)threadIdx.x + m * TB, td.ln_count - 1);
+            gid[m] = (a.tn.gid + td.ln_begin)[j];
+            psl[m] = (a.tn.pslot + td.ln_begin)[j];
+            s0[m] = (a.tn.inc_ptr + td.ln_begin)[j] - td.inc_begin;
+        }
+    // the partials of |b|^2 (iteration 1) or r.r: node blocks, or finalize blocks, or the tiles of a
+    // scene without shared nodes
+    const bool by_node = second || pin_nodes;
+    const int pa = by_node ? rg.b0 : rg.nf > 0 ? rg.f0 : rg.t0, pn = by_node ? rg.nb : rg.nf > 0 ? rg.nf : rg.nt;
+    const int lane = threadIdx.x & 63;
+    double part[kWavePartials / 64] = {0.0, 0.0, 0.0, 0.0};
+    static_assert(kWavePartials == 256, "four partials per lane");
+    if (!WIDE && iter > 0 && w0 < td.ln_count) {
+        part[0] = (pin + pa)[(unsigned)min(lane, max(pn - 1, 0))];
+        if (pn > 64) {
+#pragma unroll
+            for (int k = 1; k < kWavePartials / 64; k++) part[k] = (pin + pa)[(unsigned)min(lane + 64 * k, pn - 1)];
+        }
+    }
+    R rot[EPT][9], rin[EPT][NR], kk[EPT][3], em[EPT];
+    uint2 lt[EPT], inc[EPT];
+#pragma unroll
+    for (int m = 0; m < EPT; m++) {
+        const unsigned k = threadIdx.x + m * TB;
+        if ((int)k < td.e_count) {
+            lt[m] = (a.ltet + td.e_begin)[k];
+            inc[m] = reinterpret_cast<const uint2*>(a.tn.inc + td.inc_begin)[k];   // four incidences
+#pragma unroll
+            for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.ev.E + td.e_begin))[k];
+#pragma unroll
+            for (int i = 0; i < NR; i++) rin[m][i] = (a.rest + (i * a.ev.E + td.e_begin))[k];
+#pragma unroll
+            for (int i = 0; i < 3; i++) kk[m][i] = (a.kmat + (i * a.ev.E + td.e_begin))[k];
+            em[m] = consistent ? (a.emass + td.e_begin)[k] : (R)0;
+        }
+    }
+    VT pv[NPT][3], po[NPT][3], ms[NPT];
+    int8_t fx[NPT], ct[NPT];
+    const bool plane = PLANE && in.plane_on, table = in.mass_kind != kMassUniform;
+#pragma unroll
+    for (int m = 0; m < NPT; m++)
+        if (w0 + m * TB < td.ln_count) {
+            ld3(r, gid[m], pv[m]);
+            if (second) ld3(p, gid[m], po[m]);
+            ms[m] = table ? (VT)a.mass[gid[m]] : (VT)in.vertex_mass;
+            fx[m] = a.fixed[gid[m]];
+            ct[m] = plane ? a.contact[gid[m]] : 0;
+        }
+#pragma unroll
+    for (int m = 0; m < EPT; m++) {
+        const int k = threadIdx.x + m * TB;
+        if (k < td.e_count) *reinterpret_cast<uint2*>(linc + 4 * k) = inc[m];
+    }
+    if (in.stopped) return;
+    const bool first = (td.flags & kTileFirst) != 0;
+    // ---- 2. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
+    double total = 0.0, beta = 0.0;      // |b|^2 or r.r
+    bool go = true;
+    if (WIDE && iter > 0) total = scene_sum<TB, WIDE>(pin, pa, pn, sh);
+    if (w0 < td.ln_count) {
+        if (!WIDE && iter > 0) {
+#pragma unroll
+            for (int k = 0; k < kWavePartials / 64; k++) total = lane + 64 * k < pn ? total + part[k] : total;
+            total = wave_sum(total);
+        }
+        double err = 0.0;
+        if (cont) {
+            // the refinement replaced r by the true residual: beta from its r.r and the r.r that
+            // built p; the tolerance is relative to the first sweep's |r|
+            err = sqrt(total) / in.normb;
+            if (total == 0.0 || err <= in.tol) { record_stop(ins, first, 1, 1, err); go = false; }
+            beta = total / in.rho_last;
+            if (go && first && threadIdx.x == 0) {
+                ins->rho_slot[1] = total; ins->beta = beta; ins->iter = 1; ins->err = err;
+            }
+        } else if (iter == 1) {
+            const double normb = sqrt(total);
+            err = sqrt(total) / normb;
+            if (normb == 0.0) { record_stop(ins, first, 4, 0, 1.0); go = false; }
+            else if (err <= in.tol && !in.first_solve) { record_stop(ins, first, 1, 1, err); go = false; }
+            if (go && first && threadIdx.x == 0) {
+                ins->normb = normb; ins->rho_slot[1] = total; ins->iter = 1; ins->err = err;
+            }
+        } else if (iter > 1) {
+            err = sqrt(total) / in.normb;
+            if (iter > in.max_iter) { record_stop(ins, first, 0, in.max_iter, in.err); go = false; }
+            else if (err <= in.tol) { record_stop(ins, first, 1, iter, err); go = false; }
+            beta = total / (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
+            if (go && first && threadIdx.x == 0) {
+                ins->rho_slot[iter & 1] = total; ins->beta = beta; ins->iter = iter; ins->err = err;
+            }
+        }
+        if (go) {   // p = r + beta p (interior nodes: this tile owns p and writes it back)
+            const VT vb = (VT)beta;
+#pragma unroll
+            for (int m = 0; m < NPT; m++) {
+                const int j = threadIdx.x + m * TB;
+                if (j < td.ln_count) {
+                    const bool interior = psl[m] < 0;
+                    if (second) {
+#pragma unroll
+                        for (int i = 0; i < 3; i++) { VT t = po[m][i] * vb; t += pv[m][i]; pv[m][i] = t; }
+                    }
+                    if (iter > 0 && interior) st3(p, gid[m], pv[m]);
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
+                        pv[m][i] = (VT)(R)pv[m][i];
+                        lu[3 * j + i] = pv[m][i];
+                    }
+                    lmass[j] = ms[m];
+                    lnode[j] = (uint16_t)(s0[m] | (in.m_cg != 0.0 && interior ? kNodeMass : 0));
+                }
+            }
+        }
+    }
+    if (threadIdx.x == 0) halt = !go;
+    __syncthreads();
+    if (halt) return;
+    // ---- 3. element K p into LDS
+    const R kcg = (R)in.k_cg, mcg = (R)in.m_cg;
+#pragma unroll
+    for (int m = 0; m < EPT; m++) {
+        const int k = threadIdx.x + m * TB;
+        if (k < td.e_count) {
+            int l[4];
+            unpack_ltet(lt[m], l);
+            R u[12], c[12];
+#pragma unroll
+            for (int n = 0; n < 4; n++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) u[3 * n + i] = (R)lu[3 * l[n] + i];
+            elem_dforce_r<R, NR>(rot[m], rin[m], kk[m], u, kcg, c);
+            if (consistent) add_edge_mass(mcg * em[m], u, c);
+#pragma unroll
+            for (int i = 0; i < 12; i++) lc[i * kTileRow + k] = c[i];
+        }
+    }
+    __syncthreads();
+    // ---- 4. per-node sums in ascending element id, from LDS only
+    const int n3 = 3 * td.ln_count;
+#pragma unroll 1
+    for (int j = threadIdx.x; j < n3; j += TB) {
+        const int n = j / 3, c = j - 3 * n;
+        const int nf = lnode[n], i0 = nf & (kNodeMass - 1);
+        const int i1 = n + 1 < td.ln_count ? (int)(lnode[n + 1] & (kNodeMass - 1)) : ninc;
+        VT acc = 0;
+        if (nf & kNodeMass) mass_term(in, lmass[n], in.m_cg, lu[j], acc);
+        sum_component(linc, i0, i1, lc + c * kTileRow, acc);
+        lu[j] = acc;
+    }
+    __syncthreads();
+    // ---- 5. the nodes' results
+    double pq = 0.0;
+#pragma unroll
+    for (int m = 0; m < NPT; m++) {
+        const int j = threadIdx.x + m * TB;
+        if (w0 + m * TB < td.ln_count && j < td.ln_count) {
+            VT qn[3] = {lu[3 * j], lu[3 * j + 1], lu[3 * j + 2]};
+            if (psl[m] < 0) {
+                if (PLANE && ct[m]) plane_dforce(in, in.k_cg, pv[m], qn);
+                if (fx[m]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
+                st3(q, gid[m], qn);
+                pq += dot3d(pv[m], qn);
+            } else {
+                st3(sp, psl[m] & (kSlotOwner - 1), qn);
+                // p.q is linear in q: a shared node's term is split over its tiles (p . this
+                // tile's partial), its mass and plane terms added by its first tile, so that the
+                // tile partials hold all of p.q and no later kernel has to add to it
+                if (!fx[m]) {
+                    pq += dot3d(pv[m], qn);
+                    if ((psl[m] & kSlotOwner) && (in.m_cg != 0.0 || (PLANE && ct[m]))) {
+                        VT mq[3] = {0, 0, 0};
+                        if (in.m_cg != 0.0)
+#pragma unroll
+                            for (int i = 0; i < 3; i++) mass_term(in, ms[m], in.m_cg, pv[m][i], mq[i]);
+                        if (PLANE && ct[m]) plane_dforce(in, in.k_cg, pv[m], mq);
+                        pq += dot3d(pv[m], mq);
+                    }
+                }
+            }
+        }
+    }
+    if (w0 < td.ln_count) pq = wave_sum(pq);
+    if (lane == 0) sh[threadIdx.x >> 6] = pq;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = sh[0];
+#pragma unroll
+        for (int k = 1; k < TB / 64; k++) t = t + sh[k];
+        pden[td.pslot] = t;
+    }
+}
+
+// The operator in the reference's summation order, the arithmetic of applyStiffnessCorotational in its
+// own order.  |b|^2 and r.r come from InstDev::dots; interior nodes write their p.q term to nd; a
+// shared node's leading run (its first incidences in ascending element id, when they lie in this
+// tile) is summed here after the mass term into the node's first slot, every later incidence goes to
+// a slot of its own (finished by k_fin_exact).
+// GEO: how much element geometry is recomputed from node positions instead of read back, with
+// the functions and operation order of the element set-up and no fused multiply-adds (so the
+// same bits).  1: the rotation, from the current positions x (the ones the force pass used: x changes
+// only after the solve) -- 9 reals less per element, 3 more per tile-local node.  2: also the rotated
+// rest coordinates from the rest positions x0 (initLarge, TetrahedronFEMForceField.inl:835-868) and,
+// for a scene of one material, K from the rest volume -- NR (+ 3) reals less per element, 3 more per
+// local node.  Reading all of it back and summing by component, as k_tile_apply does, took 39.2 us against
+// 37.4 on 16 beams of 0.56M tetrahedra in double, and 4 % more of the step: the 168 bytes per element
+// push the vectors and slots out of L2, and its sums are stored incidence by incidence anyway.
+// PLANE = false: no scene of the launch has a PlaneForceField (its per-node terms compiled out).
+template <typename R, int NR, typename VT, int TB, int GEO, bool PLANE>
+__global__ __launch_bounds__(TB) void k_tile_exact(TileArgs<R, NR> a, int iter, const VT* __restrict__ r,
+                                                    VT* __restrict__ p, VT* __restrict__ q, VT* __restrict__ sp,
+                                                    const VT* __restrict__ x, const VT* __restrict__ x0) {
+    constexpr int EPT = kTileElems / TB;                   // elements per thread
+    constexpr int NPT = (kTileNodes + TB - 1) / TB;        // tile-local nodes per thread
+    static_assert(GEO == 1 || GEO == 2, "the rotation is recomputed from the positions");
+    static_assert(kTileElems * 12 >= kTileNodes * 6, "positions are staged in the contribution buffer");
+    __shared__ R lu[kTileNodes * 3];
+    __shared__ R lc[kTileRow * 12];
+    __shared__ uint16_t linc[kTileElems * 4];
+    __shared__ int lptr[kTileNodes + 1];
+    const TileDesc td = a.tiles[xcd_item()];
+    InstDev* ins = &a.inst[td.scene];
+    const InstDev in = *ins;
     const bool kvol = GEO == 2 && (td.flags & kTileOneMaterial) != 0;   // K recomputed, not loaded
     // ---- 1. issue every load that depends on the tile descriptor only: the element records of
     //         this thread (kept in registers), the tile-local node ids / slots / masks, the
     //         incidence tables, the scene record
-    R rot[EPT][9], rin[EPT][NR], kk[EPT][3], em[EPT];
+    R rot[EPT][9], rin[EPT][NR], kk[EPT][3];
     uint2 lt[EPT];
 #pragma unroll
     for (int m = 0; m < EPT; m++) {
@@ -606,10 +865,6 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         if (k < td.e_count) {
             const int64_t e = (int64_t)td.e_begin + k;
             lt[m] = a.ltet[e];
-            if (GEO == 0) {
-#pragma unroll
-                for (int i = 0; i < 9; i++) rot[m][i] = a.ev.rot[i * a.ev.E + e];
-            }
             if (GEO < 2) {
 #pragma unroll
                 for (int i = 0; i < NR; i++) rin[m][i] = a.ev.rest[i * a.ev.E + e];
@@ -618,7 +873,6 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
 #pragma unroll
                 for (int i = 0; i < 3; i++) kk[m][i] = a.ev.kmat[i * a.ev.E + e];
             }
-            em[m] = consistent ? a.emass[e] : (R)0;
         }
     }
     // tile-local node tables: every thread loads, at its node or (past the tile's count) at the
@@ -632,24 +886,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         const int li = td.ln_begin + j;
         gid[m] = a.tn.gid[li];
         psl[m] = a.tn.pslot[li];
-        lead[m] = EXACT ? a.tn.lead[li] : 0;
-    }
-    // a refinement sweep that keeps the previous search direction continues CG at its iteration 1
-    const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
-    // the partials of |b|^2 (iteration 1) or r.r: node blocks, or finalize blocks, or the tiles of a
-    // scene without shared nodes
-    const bool by_node = cont || iter > 1 || pin_nodes;
-    const int pa = by_node ? rg.b0 : rg.nf > 0 ? rg.f0 : rg.t0, pn = by_node ? rg.nb : rg.nf > 0 ? rg.nf : rg.nt;
-    constexpr bool kEarly = !EXACT && !WIDE;    // up to kWavePartials of them: in flight with the gathers
-    const int lane = threadIdx.x & 63;
-    double part[kWavePartials / 64] = {0.0, 0.0, 0.0, 0.0};
-    static_assert(kWavePartials == 256, "four partials per lane");
-    if (kEarly && iter > 0) {
-        part[0] = pin[pa + min(lane, max(pn - 1, 0))];
-        if (pn > 64) {
-#pragma unroll
-            for (int k = 1; k < kWavePartials / 64; k++) part[k] = pin[pa + min(lane + 64 * k, pn - 1)];
-        }
+        lead[m] = a.tn.lead[li];
     }
     // the incidence tables into registers first: their loads are in flight while the node ids
     // arrive and the node gathers below are issued; they go to LDS after those
@@ -671,17 +908,15 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     // ---- 2. the tile's nodes: r and p (dependent on the node ids), masks; issued before the
     //         scene's stop flag is tested (in-bounds loads, unused for a stopped scene)
     VT rr_[NPT][3], po_[NPT][3], xx_[NPT][3], x0_[NPT][3];
-    float dv_[NPT][3];
-    // p is read from iteration 2 on (or continuing a direction); without a p (a plain operator
-    // application) the loads read r instead, unused
+    // p is read from iteration 2 on; without a p (a plain operator application) the loads read r
+    // instead, unused
     const VT* __restrict__ pl = p ? p : r;
     const bool plane = PLANE && in.plane_on;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
         ld3(r, gid[m], rr_[m]);
-        if (a.dinv) ld3(a.dinv, gid[m], dv_[m]);
         ld3(pl, gid[m], po_[m]);
-        if (GEO >= 1) ld3(x, gid[m], xx_[m]);
+        ld3(x, gid[m], xx_[m]);
         if (GEO == 2) ld3(x0, gid[m], x0_[m]);
         fx[m] = a.fixed[gid[m]];
         if (PLANE) {
@@ -704,34 +939,13 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     if (in.stopped) return;
     const bool first = (td.flags & kTileFirst) != 0;
     // ---- 3. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
-    double total = 0.0;      // |b|^2 or r.r
-    if (!EXACT && iter > 0) {
-        if constexpr (kEarly) {
-#pragma unroll
-            for (int k = 0; k < kWavePartials / 64; k++)
-                total = lane + 64 * k < pn ? total + part[k] : total;
-            total = wave_sum(total);
-        } else {
-            total = scene_sum<TB, WIDE>(pin, pa, pn, sh);
-        }
-    }
     double beta = 0.0;
-    if (cont) {
-        // the refinement replaced r by the true residual: beta from its r.r and the r.r that
-        // built p; the tolerance is relative to the first sweep's |r|
-        const double rho = total;
-        const double err = sqrt(rho) / in.normb;
-        if (rho == 0.0 || err <= in.tol) { record_stop(ins, first, 1, 1, err); return; }
-        beta = rho / in.rho_last;
-        if (first && threadIdx.x == 0) {
-            ins->rho_slot[1] = rho; ins->beta = beta; ins->iter = 1; ins->err = err;
-        }
-    } else if (iter == 1) {
-        const double bb = EXACT ? in.dots[kDotBB] : total;
+    if (iter == 1) {
+        const double bb = in.dots[kDotBB];
         const double normb = sqrt(bb);
         if (normb == 0.0) { record_stop(ins, first, 4, 0, 1.0); return; }
-        // rho = r.r: b.b from a cold start; warmStart (reference order): the r.r of r = b - A x
-        const double rho = EXACT && in.warm_start ? in.dots[kDotRR] : bb;
+        // rho = r.r: b.b from a cold start; warmStart: the r.r of r = b - A x
+        const double rho = in.warm_start ? in.dots[kDotRR] : bb;
         const double err = sqrt(rho) / normb;
         if (err <= in.tol && !in.first_solve) { record_stop(ins, first, 1, 1, err); return; }
         if (first && threadIdx.x == 0) {
@@ -739,37 +953,29 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         }
     } else if (iter > 1) {
         if (iter > in.max_iter) { record_stop(ins, first, 0, in.max_iter, in.err); return; }
-        const double rho = EXACT ? in.dots[kDotRR] : total;
+        const double rho = in.dots[kDotRR];
         const double err = sqrt(rho) / in.normb;
         if (err <= in.tol) { record_stop(ins, first, 1, iter, err); return; }
-        const double rho_1 = (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
-        beta = rho / rho_1;
+        beta = rho / (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
         if (first && threadIdx.x == 0) {
             ins->rho_slot[iter & 1] = rho; ins->beta = beta; ins->iter = iter; ins->err = err;
         }
     }
-    // ---- 4. stage p = r + beta p, or z + beta p with z = dinv r (interior nodes: this tile owns
-    //         p and writes it back)
+    // ---- 4. stage p = r + beta p (interior nodes: this tile owns p and writes it back)
     const VT vb = (VT)beta;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
         const int j = threadIdx.x + m * TB;
         if (j < td.ln_count) {
             VT pp[3] = {rr_[m][0], rr_[m][1], rr_[m][2]};
-            if (a.dinv) {
-#pragma unroll
-                for (int i = 0; i < 3; i++) pp[i] = pp[i] * (VT)dv_[m][i];
-            }
-            if (iter > 1 || cont) {
+            if (iter > 1) {
 #pragma unroll
                 for (int i = 0; i < 3; i++) { VT t = po_[m][i] * vb; t += pp[i]; pp[i] = t; }
             }
             if (iter > 0 && psl[m] < 0) st3(p, gid[m], pp);
             lu[3 * j] = (R)pp[0]; lu[3 * j + 1] = (R)pp[1]; lu[3 * j + 2] = (R)pp[2];
-            if (GEO >= 1) {
 #pragma unroll
-                for (int i = 0; i < 3; i++) lc[3 * j + i] = (R)xx_[m][i];
-            }
+            for (int i = 0; i < 3; i++) lc[3 * j + i] = (R)xx_[m][i];
             if (GEO == 2) {
 #pragma unroll
                 for (int i = 0; i < 3; i++) lc[3 * kTileNodes + 3 * j + i] = (R)x0_[m][i];
@@ -777,7 +983,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         }
     }
     __syncthreads();
-    if (GEO >= 1) {   // geometry from the staged positions, then the buffer is free again
+    {   // geometry from the staged positions, then the buffer is free again
         const R* lx = lc;
         const R* lx0 = lc + 3 * kTileNodes;
 #pragma unroll
@@ -807,7 +1013,6 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     }
     // ---- 5. element K p into LDS
     const R kcg = (R)in.k_cg;
-    const R mcg = (R)in.m_cg;
 #pragma unroll
     for (int m = 0; m < EPT; m++) {
         const int k = threadIdx.x + m * TB;
@@ -820,14 +1025,12 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
 #pragma unroll
                 for (int i = 0; i < 3; i++) u[3 * n + i] = lu[3 * l[n] + i];
             elem_dforce_r<R, NR>(rot[m], rin[m], kk[m], u, kcg, c);
-            if (consistent) add_edge_mass(mcg * em[m], u, c);
 #pragma unroll
-            for (int i = 0; i < 12; i++) lc[i * kTileElems + k] = c[i];
+            for (int i = 0; i < 12; i++) lc[i * kTileRow + k] = c[i];
         }
     }
     __syncthreads();
     // ---- 6. per-node sums in ascending element id, from LDS only
-    double pq = 0.0;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
         const int j = threadIdx.x + m * TB;
@@ -841,9 +1044,8 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
                 if (PLANE && ct[m]) plane_dforce(in, in.k_cg, pp, qn);
                 if (fx[m]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
                 st3(q, gid[m], qn);
-                if (EXACT) a.nd[gid[m]] = dot3d(pp, qn);
-                else pq += dot3d(pp, qn);
-            } else if (EXACT) {
+                a.nd[gid[m]] = dot3d(pp, qn);
+            } else {
                 int s = s0;
                 if (lead[m] > 0) {
                     // this tile holds the node's leading run: the node's sum starts here (the mass
@@ -856,31 +1058,59 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
                     st3(sp, psl[m], acc);
                 }
                 store_incidences(linc, a.tn.arank + td.inc_begin, s, s1, lc, sp, psl[m]);
-            } else {
-                VT acc[3] = {0, 0, 0};
-                sum_incidences<true>(linc, s0, s1, lc, acc);
-                st3(sp, psl[m] & (kSlotOwner - 1), acc);
-                // p.q is linear in q: a shared node's term is split over its tiles (p . this
-                // tile's partial), its mass and plane terms added by its first tile, so that the
-                // tile partials hold all of p.q and no later kernel has to add to it
-                if (!fx[m]) {
-                    const VT pp[3] = {(VT)lu[3 * j], (VT)lu[3 * j + 1], (VT)lu[3 * j + 2]};
-                    pq += dot3d(pp, acc);
-                    if ((psl[m] & kSlotOwner) && (in.m_cg != 0.0 || (PLANE && ct[m]))) {
-                        VT mq[3] = {0, 0, 0};
-                        if (in.m_cg != 0.0)
-                            mass_mdx(in, NodeArrays{nullptr, nullptr, a.mass, a.fixed}, gid[m], in.m_cg, pp, mq);
-                        if (PLANE && ct[m]) plane_dforce(in, in.k_cg, pp, mq);
-                        pq += dot3d(pp, mq);
-                    }
-                }
             }
         }
     }
-    if (!EXACT) {
-        const double tot = wave_block_sum<TB>(pq, sh);
-        if (threadIdx.x == 0) pden[td.pslot] = tot;
+}
+
+// The float record's rest shape and (a scene of one material) K from the rest positions in float, with
+// the functions and operation order of the element set-up (initLarge, TetrahedronFEMForceField.inl:835-868)
+// and no fused multiply-adds: an operator in float throughout, not one rounded from the host's double.
+static __global__ __launch_bounds__(kBlock) void k_rest_float(const int4* __restrict__ tet, int64_t e0, int64_t e1, int64_t E,
+                                                               const double* __restrict__ xd, const float* __restrict__ xf,
+                                                               bool one_material, double ks0, double ks1, double ks2,
+                                                               float* __restrict__ rest, float* __restrict__ kmat) {
+    const int64_t e = e0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= e1) return;
+    const int4 t = tet[e];
+    const int v[4] = {t.x, t.y, t.z, t.w};
+    float p[4][3], rin[6];
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int64_t o = 3 * (int64_t)v[n] + i;
+            p[n][i] = xd ? (float)xd[o] : xf[o];
+        }
+    rest_frame<float, 6>(p, rin);
+#pragma unroll
+    for (int i = 0; i < 6; i++) rest[i * E + e] = rin[i];
+    if (one_material) {
+        const double ks[3] = {ks0, ks1, ks2};
+        float k3[3];
+        stiffness_from_volume(p, ks, k3);
+#pragma unroll
+        for (int i = 0; i < 3; i++) kmat[i * E + e] = k3[i];
     }
+}
+
+// the rotations of the elements [e0, e1) from the engine's current positions, for a solve that does not
+// follow a force pass (component-level CG)
+template <typename R, typename VT>
+__global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ tet, int64_t e0, int64_t e1,
+                                                       const VT* __restrict__ x, R* __restrict__ rot, int64_t E) {
+    const int64_t e = e0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= e1) return;
+    const int4 t = tet[e];
+    const int v[3] = {t.x, t.y, t.z};
+    R p[3][3], ro[9];
+#pragma unroll
+    for (int n = 0; n < 3; n++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) p[n][i] = (R)x[3 * (int64_t)v[n] + i];
+    rotation_large(p[0], p[1], p[2], ro);
+#pragma unroll
+    for (int i = 0; i < 9; i++) rot[i * E + e] = ro[i];
 }
 
 // reference order, after the tile apply: the shared nodes' p = r + beta p, q = (1 + h rm) M p

@@ -8,9 +8,9 @@
 // each tile-local node the incidence list is sorted by ORIGINAL element id: the order in which
 // the reference's element loop accumulates into that node (TetrahedronFEMForceField.inl:
 // 1630-1634).  An incidence is the LDS slot of the element's contribution to the node: the
-// kernels keep the 12 contribution components of a tile's elements as 12 rows of max_elems
+// kernels keep the 12 contribution components of a tile's elements as 12 rows of slot_row
 // (row 3 v + c, column = tile-local element), so vertex v of local element k is the slot
-// 3 v max_elems + k and its component c sits c max_elems further.
+// 3 v slot_row + k and its component c sits c slot_row further.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -30,7 +30,7 @@ struct TilePlan {
     std::vector<uint2> ltet;        // per permuted element: 4 x uint16 tile-local node index
     std::vector<int> ln_gid;        // tile-local node -> scene-local node id
     std::vector<int> ln_inc_ptr;    // size(ln_gid) + 1
-    std::vector<uint16_t> ln_inc;   // contribution slot: 3 max_elems vertex + local element
+    std::vector<uint16_t> ln_inc;   // contribution slot: 3 slot_row vertex + local element
     std::vector<int> ln_pslot;      // -1 interior, else scene-local shared-partial slot
     std::vector<int> sh_gid;        // nodes finished by the finalize kernel (ascending)
     std::vector<int> sh_ptr;        // size(sh_gid) + 1
@@ -56,6 +56,10 @@ static inline uint64_t spread3(uint64_t v) {   // 21 bits -> every third bit
     v = (v | (v << 2)) & 0x1249249249249249ULL;
     return v;
 }
+
+// the length of a contribution row: eight more than the elements of a full tile, so that a node's three
+// components, read by neighbouring lanes from three rows, lie in different LDS banks
+constexpr int slot_row(int max_elems) { return max_elems + 8; }
 
 enum TileOrder { kOrderMorton = 0, kOrderElementId = 1 };
 static inline TilePlan plan_tiles(int n_nodes, const double* rest, const int32_t* tets, int E, int max_elems,
@@ -193,7 +197,7 @@ static inline TilePlan plan_tiles(int n_nodes, const double* rest, const int32_t
             uint32_t l[4];
             for (int v = 0; v < 4; v++) {
                 l[v] = (uint32_t)loc[tets[4 * e + v]];
-                per[l[v]].push_back({e, v * 3 * max_elems + k});
+                per[l[v]].push_back({e, v * 3 * slot_row(max_elems) + k});
             }
             P.ltet[e0 + k] = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
         }
@@ -274,7 +278,7 @@ static inline void plan_exact(TilePlan& P, int n_nodes, int max_elems) {
             const int k = shidx[P.ln_gid[li]];
             if (k < 0) continue;
             for (int c = P.ln_inc_ptr[li]; c < P.ln_inc_ptr[li + 1]; c++) {
-                const int local_elem = (int)P.ln_inc[c] % max_elems;   // slot = 3 max_elems v + element
+                const int local_elem = (int)P.ln_inc[c] % slot_row(max_elems);   // slot = 3 row v + element
                 lists[k].push_back({P.perm[P.t_ebegin[ti] + local_elem], c, ti, li});
             }
         }

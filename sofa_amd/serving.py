@@ -40,10 +40,12 @@ def footprint_bytes(precision, nodes, tets, reference_order=False, scenes=1):
     nr = 6 if precision == capi.FP32 else 9
     per_node = 8 * 3 * pv + 8 + 1 + 4 + 16 + 12 + 6 * pv
     per_tet = 24 + (9 + nr + 3 + 1) * pe + 12 * pv + 24
+    if precision in (capi.FP32, capi.SPLIT, capi.MIXED):
+        per_tet += (6 + 3) * 4                 # the operator's rest shape and K in float
     if precision == capi.MIXED:
-        # float r, p, q, d, x, x0 and shared partials; float K entries and edge masses
-        per_node += 6 * 3 * 4 + 3 * 4
-        per_tet += (3 + 1) * 4
+        # float r, p, q, d and shared partials; float rotations and edge masses
+        per_node += 4 * 3 * 4 + 3 * 4
+        per_tet += (9 + 1) * 4
     per_scene = 0
     if reference_order:
         per_tet += 4 * 2 * 3 * pv + 4 * 2

@@ -1,0 +1,81 @@
+"""The tiled CG operator (k_tile_apply): tiles with few elements, a full tile and a remainder, many tiles;
+one material and a material per element with a consistent mass; with and without a plane.  The
+engines that run it in one CG against the oracle's step (MIXED, which refines with the FP32 engine's operator,
+is compared with converged solutions elsewhere).  Bars: FP64_TILED sums shared nodes tile by tile and p.q by
+blocks, a few ulp (1e-16) of the vectors per operation, amplified by at most the 10 iterations of a solve
+that is far from converged: 1e-10, on x and v.  The single precision elements: 2e-5 on x, the bar of every
+FP32 trajectory test; their v after two steps is the small difference that the float force pass leaves of
+positions of order one, which says nothing about the operator, and is not compared."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BARS = {"FP64_TILED": 1e-10, "FP32": 2e-5, "SPLIT": 2e-5}
+
+
+def _capi():
+    from sofa_amd import capi
+    return capi
+
+
+def _spec(n, kind):
+    from sofa_amd import workloads
+    s = workloads._beam_spec(n, (1.0, 1.0, 4.0), 1e5, 0.45, 0.01, 10)
+    if kind == "materials":
+        rng = np.random.default_rng(7)
+        s["E"] = rng.uniform(0.7e5, 1.4e5, len(s["tets"]))
+        s["nu"] = rng.uniform(0.3, 0.45, len(s["tets"]))
+        s["mass"] = ("meshmatrix", 1000.0)
+    elif kind == "plane":
+        s["plane"] = dict(normal=(0.0, 1.0, 0.0), d=0.05, stiffness=500.0, damping=1.0)
+    return s
+
+
+@pytest.mark.parametrize("kind", ["one", "materials", "plane"])
+@pytest.mark.parametrize("n", [(2, 2, 2), (3, 3, 27), (2, 3, 53), (9, 8, 30)])
+@pytest.mark.parametrize("prec", ["FP64_TILED", "FP32", "SPLIT"])
+def test_tile_operator(prec, n, kind):
+    from specs import oracle_from_spec
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: tile operator {prec} {n} {kind}", flush=True)
+    spec = _spec(n, kind)
+    o = oracle_from_spec(spec, 0)
+    o.step(spec["dt"], 2)
+    for variant in (0, 2):
+        eng = capi.Engine(0, getattr(capi, prec))
+        sid = workloads.add_to_engine(eng, spec)
+        eng.commit()
+        eng.set_apply_variant(variant)
+        eng.step([sid], 2)
+        x, v, _ = eng.read(sid)
+        eng.close()
+        for a, b in ((x, o.get("x")), (v, o.get("v")))[:2 if prec == "FP64_TILED" else 1]:
+            e = float(np.linalg.norm(a - b) / np.linalg.norm(b))
+            assert e <= BARS[prec], (variant, e)
+
+
+@pytest.mark.parametrize("prec", ["FP64_TILED", "FP32"])
+def test_cg_solve_keeps_the_force_calls_rotations(prec):
+    """cg_solve computes the rotations of the engine's own positions; addDForce after it still uses the last
+    addForce's, so its result has the same bits before and after."""
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: cg_solve between addDForce calls, {prec}", flush=True)
+    dt = np.float32 if prec == "FP32" else np.float64
+    spec = _spec((3, 3, 27), "one")
+    eng = capi.Engine(0, getattr(capi, prec))
+    sid = workloads.add_to_engine(eng, spec)
+    eng.commit()
+    rng = np.random.default_rng(3)
+    dev = lambda a: capi.DeviceArray(np.ascontiguousarray(a, dtype=dt))
+    x, dx = dev(spec["pos"] + 0.02 * rng.standard_normal(spec["pos"].shape)), dev(rng.standard_normal(spec["pos"].shape))
+    f, before, after, sol = (dev(np.zeros(spec["pos"].shape)) for _ in range(4))
+    eng.fem_add_force(sid, x.ptr, f.ptr)
+    eng.fem_add_dforce(sid, dx.ptr, before.ptr, 1.0)
+    eng.cg_solve(sid, 1.0, 0.0, -1e-3, dx.ptr, sol.ptr)
+    eng.fem_add_dforce(sid, dx.ptr, after.ptr, 1.0)
+    a, b = before.numpy(), after.numpy()
+    eng.close()
+    assert np.any(a) and np.array_equal(a, b)
