@@ -1469,7 +1469,7 @@ struct EngineT : EngineBase {
         const SharedNodes sn{sh_gid, sh_ptr, sh_of, sh_acnt};
         launch_seqdot(n, s, kDotPQ);
         if (cur->nc > 0)
-            k_update<VT, true><<<cur->nc, kBlock, 0, s>>>(nb, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r,
+            k_update<VT, true><<<cur->nc, kUpdateThreads, 0, s>>>(nb, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r,
                                                           pden, prho, contact, nd);
         launch_seqdot(n, s, kDotRR);
     }
@@ -1617,7 +1617,7 @@ struct EngineT : EngineBase {
             if (cur->na > 0)
                 launch_apply(cur->na, s, ta, it, r, p, q, sp0, it == 1 ? pbb : prho, pden, 0);
             if (cur->nc > 0)
-                k_update<VT><<<cur->nc, kBlock, 0, s>>>(nb, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r, pden, prho, contact);
+                k_update<VT><<<cur->nc, kUpdateThreads, 0, s>>>(nb, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r, pden, prho, contact);
         }
         if (cur->nc > 0) k_integrate<VT><<<cur->nc, kBlock, 0, s>>>(nb, inst, fixed, xcg, v, x);
         if (cur->no > 0) k_oscillate<VT><<<cur->no, kBlock, 0, s>>>((const Blk*)cur->o, inst, oscillators(), x, v);
@@ -2088,7 +2088,7 @@ struct EngineT : EngineBase {
                             k_fin_exact<VT><<<cur->nb, kBlock, 0, s>>>(fb, inst, sn, mass, fixed, it, r, p, q, sp0, nd, contact);
                         launch_seqdot(1, s, kDotPQ, false);
                         if (cur->nc > 0)
-                            k_update<VT, true><<<cur->nc, kBlock, 0, s>>>(nbk, inst, ranges_d, it, sn, sp0, mass, fixed, p, q,
+                            k_update<VT, true><<<cur->nc, kUpdateThreads, 0, s>>>(nbk, inst, ranges_d, it, sn, sp0, mass, fixed, p, q,
                                                                           xcg, r, pden, prho, contact, nd);
                         launch_seqdot(1, s, kDotRR, false);
                     }
@@ -2099,7 +2099,7 @@ struct EngineT : EngineBase {
                 for (int it = 1; it <= cur->maxit; it++) {
                     if (cur->na > 0) launch_apply(cur->na, s, ta, it, r, p, q, sp0, prho, pden, it == 1 ? 1 : 0);
                     if (cur->nc > 0)
-                        k_update<VT><<<cur->nc, kBlock, 0, s>>>(nbk, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r,
+                        k_update<VT><<<cur->nc, kUpdateThreads, 0, s>>>(nbk, inst, ranges_d, it, sn, sp0, mass, fixed, p, q, xcg, r,
                                                                 pden, prho, contact);
                 }
             }
@@ -2322,7 +2322,7 @@ void launch_inner_cg(const InnerCg& c, hipStream_t s) {
             op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1);
         }
         if (c.nnb > 0)
-            k_update<float><<<c.nnb, kBlock, 0, s>>>(c.nb, c.ta.inst, c.ta.ranges, it, c.sn, c.sp, c.ta.mass, c.ta.fixed,
+            k_update<float><<<c.nnb, kUpdateThreads, 0, s>>>(c.nb, c.ta.inst, c.ta.ranges, it, c.sn, c.sp, c.ta.mass, c.ta.fixed,
                                                       c.p, c.q, c.d, c.r, c.pden, c.prho, c.ta.contact, nullptr,
                                                       c.dinv, c.binv, c.z);
     }

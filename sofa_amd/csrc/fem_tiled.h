@@ -169,6 +169,57 @@ __device__ __forceinline__ double scene_sum(const double* __restrict__ buf, int 
     return reduce2<TB>(buf, a0, na, sh);
 }
 
+// scene_sum in two parts: the loads at the head of a kernel, the sum where it is needed.  TB threads add
+// (a larger block's others only take part in the barrier); sh holds TB / 64 doubles
+constexpr int kSumBatch = 8;
+struct SceneTerms {
+    double v[kSumBatch];
+};
+template <int TB, bool WIDE>
+__device__ __forceinline__ void load_terms(const double* __restrict__ buf, int na, SceneTerms& s) {
+    const int lane = threadIdx.x & 63;
+    static_assert(kWavePartials == 256, "four partials per lane");
+#pragma unroll
+    for (int k = 0; k < kSumBatch; k++) s.v[k] = 0.0;
+    if (na <= 0) return;
+    if (!WIDE || na <= kWavePartials) {
+        s.v[0] = buf[(unsigned)min(lane, na - 1)];
+        if (na > 64) {
+#pragma unroll
+            for (int k = 1; k < kWavePartials / 64; k++) s.v[k] = buf[(unsigned)min(lane + 64 * k, na - 1)];
+        }
+    } else if ((int)threadIdx.x < TB) {
+        s.v[0] = buf[(unsigned)min((int)threadIdx.x, na - 1)];
+        s.v[1] = buf[(unsigned)min((int)threadIdx.x + TB, na - 1)];
+        if (na > 2 * TB) {
+#pragma unroll
+            for (int k = 2; k < kSumBatch; k++) s.v[k] = buf[(unsigned)min((int)threadIdx.x + k * TB, na - 1)];
+        }
+    }
+}
+template <int TB, bool WIDE>
+__device__ __forceinline__ double sum_terms(const double* __restrict__ buf, int na, const SceneTerms& s, double* sh) {
+    const int lane = threadIdx.x & 63, t = threadIdx.x;
+    double acc = 0.0;
+    if (!WIDE || na <= kWavePartials) {
+#pragma unroll
+        for (int k = 0; k < kWavePartials / 64; k++) acc = lane + 64 * k < na ? acc + s.v[k] : acc;
+        return wave_sum(acc);
+    }
+    if (t < TB) {
+#pragma unroll
+        for (int k = 0; k < kSumBatch; k++) acc = t + k * TB < na ? acc + s.v[k] : acc;
+        for (int k = t + kSumBatch * TB; k < na; k += 8 * TB) acc = strided_terms<TB, 8>(buf, 0, na, k, acc);
+        acc = wave_sum(acc);
+        if (lane == 0) sh[t >> 6] = acc;
+    }
+    __syncthreads();
+    acc = sh[0];
+#pragma unroll
+    for (int k = 1; k < TB / 64; k++) acc = acc + sh[k];
+    return acc;
+}
+
 template <typename VT>
 __device__ __forceinline__ void ld3(const VT* __restrict__ v, int n, VT o[3]) {
     const VT* q = v + 3 * (int64_t)n;
@@ -640,15 +691,8 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     const bool by_node = second || pin_nodes;
     const int pa = by_node ? rg.b0 : rg.nf > 0 ? rg.f0 : rg.t0, pn = by_node ? rg.nb : rg.nf > 0 ? rg.nf : rg.nt;
     const int lane = threadIdx.x & 63;
-    double part[kWavePartials / 64] = {0.0, 0.0, 0.0, 0.0};
-    static_assert(kWavePartials == 256, "four partials per lane");
-    if (!WIDE && iter > 0 && w0 < td.ln_count) {
-        part[0] = (pin + pa)[(unsigned)min(lane, max(pn - 1, 0))];
-        if (pn > 64) {
-#pragma unroll
-            for (int k = 1; k < kWavePartials / 64; k++) part[k] = (pin + pa)[(unsigned)min(lane + 64 * k, pn - 1)];
-        }
-    }
+    SceneTerms part;
+    if (!WIDE && iter > 0 && w0 < td.ln_count) load_terms<TB, WIDE>(pin + pa, pn, part);
     R rot[EPT][9], rin[EPT][NR], kk[EPT][3], em[EPT];
     uint2 lt[EPT], inc[EPT];
 #pragma unroll
@@ -688,13 +732,9 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     // ---- 2. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
     double total = 0.0, beta = 0.0;      // |b|^2 or r.r
     bool go = true;
-    if (WIDE && iter > 0) total = scene_sum<TB, WIDE>(pin, pa, pn, sh);
+    if (WIDE && iter > 0) total = scene_sum<TB, WIDE>(pin, pa, pn, sh);   // (early, it costs a wave per SIMD)
     if (w0 < td.ln_count) {
-        if (!WIDE && iter > 0) {
-#pragma unroll
-            for (int k = 0; k < kWavePartials / 64; k++) total = lane + 64 * k < pn ? total + part[k] : total;
-            total = wave_sum(total);
-        }
+        if (!WIDE && iter > 0) total = sum_terms<TB, WIDE>(pin + pa, pn, part, sh);
         double err = 0.0;
         if (cont) {
             // the refinement replaced r by the true residual: beta from its r.r and the r.r that
@@ -1221,16 +1261,26 @@ __global__ __launch_bounds__(kBlock) void k_fin_apply(const FinBlk* __restrict__
 
 // z = P^-1 r of a MIXED inner CG's preconditioner (the scene's kind: 0 none, 1 the inverted
 // diagonal dinv, 3 per node, 2 the inverted 3x3 block binv, 9 per node, row-major), in float
-template <typename VT>
-__device__ __forceinline__ void precond_z(int kind, const float* __restrict__ dinv, const float* __restrict__ binv,
-                                          int n, const VT r[3], VT z[3]) {
-    if (kind == 1) {
-        float dv[3];
-        ld3(dinv, n, dv);
+__device__ __forceinline__ void precond_load(int kind, const float* __restrict__ dinv, const float* __restrict__ binv,
+                                             int n, float B[9]) {
+    const float* p = kind == 2 ? binv + 9 * (int64_t)n : dinv + 3 * (int64_t)n;
 #pragma unroll
-        for (int i = 0; i < 3; i++) z[i] = r[i] * (VT)dv[i];
+    for (int i = 0; i < 9; i++) B[i] = 0.0f;
+    if (kind != 0) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) B[i] = p[i];
+    }
+    if (kind == 2) {
+#pragma unroll
+        for (int i = 3; i < 9; i++) B[i] = p[i];
+    }
+}
+template <typename VT>
+__device__ __forceinline__ void precond_mul(int kind, const float B[9], const VT r[3], VT z[3]) {
+    if (kind == 1) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) z[i] = r[i] * (VT)B[i];
     } else if (kind == 2) {
-        const float* B = binv + 9 * (int64_t)n;
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             VT t = r[0] * (VT)B[3 * i];
@@ -1243,6 +1293,13 @@ __device__ __forceinline__ void precond_z(int kind, const float* __restrict__ di
         for (int i = 0; i < 3; i++) z[i] = r[i];
     }
 }
+template <typename VT>
+__device__ __forceinline__ void precond_z(int kind, const float* __restrict__ dinv, const float* __restrict__ binv,
+                                          int n, const VT r[3], VT z[3]) {
+    float B[9];
+    precond_load(kind, dinv, binv, n, B);
+    precond_mul(kind, B, r, z);
+}
 
 // CG iteration `iter` after the tile apply.  Nodes shared by several tiles are finished here:
 // p = r + beta p, q = (1 + h rm) M p + their tile partials in tile order, projection (the work
@@ -1253,8 +1310,16 @@ __device__ __forceinline__ void precond_z(int kind, const float* __restrict__ di
 // reference-order p.q of k_seqdot, and each node's r.r term goes to nd.  zbuf (MIXED inner CG
 // with a preconditioner): it holds z = P^-1 r of the previous residual (shared nodes' p = z +
 // beta p); each node's new z (precond_z with dinv / binv) replaces it, r.z partials in place of r.r
+// One thread per node, and everything that a node may need -- a shared node's slot range and its first
+// kSlotBatch partials, mass, masks, the preconditioner's block -- on its way before the sum of the tile
+// partials: what bounds it is that chain of dependent loads (node block, scene and ranges, partials; node,
+// its slots, their partials), not bytes.  Two nodes per thread, and the shared nodes' loads after the sum,
+// took: FP32 4,000 nodes 6.3 us, now 4.8 (a launch that waits for the one before costs 4 by itself); MIXED
+// with block-Jacobi 40k nodes 8.3, now 5.5; FP64 60k nodes 9.6, now 7.0; FP32 280k nodes 11.2, now 10.8.
+constexpr int kUpdateThreads = kBlock * kNodesPerThread;   // a node block, as the partials of r.r are formed
+static_assert(kUpdateThreads <= 1024, "one thread per node of a node block");
 template <typename VT, bool EXACT = false>
-__global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ nb_, InstDev* __restrict__ inst,
+__global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __restrict__ nb_, InstDev* __restrict__ inst,
                                                     const Ranges* __restrict__ ranges, int iter, SharedNodes sn,
                                                     const VT* __restrict__ sp, const double* __restrict__ mass,
                                                     const int8_t* __restrict__ fixed, VT* __restrict__ p,
@@ -1263,91 +1328,126 @@ __global__ __launch_bounds__(kBlock) void k_update(const NodeBlk* __restrict__ n
                                                     const int8_t* __restrict__ contact, double* __restrict__ nd = nullptr,
                                                     const float* __restrict__ dinv = nullptr,
                                                     const float* __restrict__ binv = nullptr, VT* __restrict__ zbuf = nullptr) {
-    __shared__ double sh[kBlock / 64];
+    constexpr int kSlotBatch = 4;
+    __shared__ double sh[2][kBlock / 64];
+    __shared__ double upper[EXACT ? 1 : kUpdateThreads - kBlock + 1];
     const NodeBlk nb = nb_[xcd_item()];
     InstDev* ins = &inst[nb.scene];
     const InstDev in = *ins;
     const Ranges rg = ranges[nb.scene];
-    // node data first (registers), then the reduction
-    VT pv[kNodesPerThread][3], qv[kNodesPerThread][3], xv[kNodesPerThread][3], rv[kNodesPerThread][3];
-    VT zv[kNodesPerThread][3];
-    int shk[kNodesPerThread];
-    // every load at a clamped node index (no branch: all in flight together; a node past the
-    // block's end repeats its last node, unused), p and q also where the shared-node path below
-    // replaces them
+    const int t = threadIdx.x, lane = t & 63;
+    // node data first (registers), then the reduction: every load at a clamped node index (a node past
+    // the block's end repeats its last node, unused), p and q also where the shared-node path replaces them
+    const bool mine = nb.begin + t < nb.end;
+    const int n = min(nb.begin + t, nb.end - 1);
+    const int of = EXACT ? -1 : sn.of[n];
+    SceneTerms part;
+    if (!EXACT) load_terms<kBlock, true>(pden + rg.t0, rg.nt, part);
+    VT pv[3], qv[3], xv[3], rv[3], zv[3];
+    ld3(xcg, n, xv);
+    ld3(r, n, rv);
+    if (zbuf) ld3(zbuf, n, zv);
+    ld3(p, n, pv);
+    ld3(q, n, qv);
+    VT m = 0;
+    int8_t fx = 0, ct = 0;
+    float B[9];
+    int s0 = 0, s1 = 0;
+    VT sv[kSlotBatch][3];
+    if (!EXACT) {
+        m = in.mass_kind == kMassUniform ? (VT)in.vertex_mass : (VT)mass[n];
+        fx = fixed[n];
+        if (in.plane_on) ct = contact[n];
+        if (zbuf) precond_load(in.pcg, dinv, binv, n, B);
+        if (of >= 0) {
+            s0 = sn.ptr[of];
+            s1 = sn.ptr[of + 1];
 #pragma unroll
-    for (int k = 0; k < kNodesPerThread; k++) {
-        const int n = min(nb.begin + k * kBlock + (int)threadIdx.x, nb.end - 1);
-        shk[k] = EXACT ? -1 : sn.of[n];
-        ld3(xcg, n, xv[k]);
-        ld3(r, n, rv[k]);
-        if (zbuf) ld3(zbuf, n, zv[k]);
-        ld3(p, n, pv[k]);
-        ld3(q, n, qv[k]);
+            for (int k = 0; k < kSlotBatch; k++) ld3(sp, min(s0 + k, s1 - 1), sv[k]);
+        }
     }
     if (in.stopped) return;
     const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
     const bool first = nb.first != 0;
-    const double den = EXACT ? in.dots[kDotPQ] : scene_sum<kBlock>(pden, rg.t0, rg.nt, sh);
+    double den;
+    if constexpr (EXACT) den = in.dots[kDotPQ];
+    else den = sum_terms<kBlock, true>(pden + rg.t0, rg.nt, part, sh[0]);
     const bool exempt = (iter == 1 && in.first_solve);
-    if (den == 0.0) { record_stop(ins, first, 3, iter, in.err); if (first && threadIdx.x == 0) ins->den = den; return; }
+    if (den == 0.0) { record_stop(ins, first, 3, iter, in.err); if (first && t == 0) ins->den = den; return; }
     if (fabs(den) <= in.thr && !exempt) {
         record_stop(ins, first, 2, iter, in.err);
-        if (first && threadIdx.x == 0) ins->den = den;
+        if (first && t == 0) ins->den = den;
         return;
     }
     const double alpha = (iter & 1 ? in.rho_slot[1] : in.rho_slot[0]) / den;
-    if (first && threadIdx.x == 0) { ins->den = den; ins->alpha = alpha; }
+    if (first && t == 0) { ins->den = den; ins->alpha = alpha; }
     const VT vb = (VT)in.beta;
     const VT va = (VT)alpha, vma = (VT)(-alpha);
     double rr = 0.0;
+    if (mine) {
+        if (of >= 0) {
+            VT pp[3] = {rv[0], rv[1], rv[2]};
+            if (zbuf) {
 #pragma unroll
-    for (int k = 0; k < kNodesPerThread; k++) {
-        const int n = nb.begin + k * kBlock + threadIdx.x;
-        if (n < nb.end) {
-            if (shk[k] >= 0) {
-                VT pp[3] = {rv[k][0], rv[k][1], rv[k][2]};
-                if (zbuf) {
-#pragma unroll
-                    for (int i = 0; i < 3; i++) pp[i] = zv[k][i];
-                }
-                if (iter > 1 || cont) {
-#pragma unroll
-                    for (int i = 0; i < 3; i++) { VT t = pv[k][i] * vb; t += pp[i]; pp[i] = t; }
-                }
-                st3(p, n, pp);
-                VT qn[3] = {0, 0, 0};
-                if (in.m_cg != 0.0) mass_mdx(in, NodeArrays{nullptr, nullptr, mass, fixed}, n, in.m_cg, pp, qn);
-                const int s0 = sn.ptr[shk[k]], s1 = sn.ptr[shk[k] + 1];
-                sum_slots<false>(sp, s0, s1, qn);
-                if (in.plane_on && contact[n]) plane_dforce(in, in.k_cg, pp, qn);
-                if (fixed[n]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
-#pragma unroll
-                for (int i = 0; i < 3; i++) { pv[k][i] = pp[i]; qv[k][i] = qn[i]; }
+                for (int i = 0; i < 3; i++) pp[i] = zv[i];
             }
-            VT xn[3], rn[3];
+            if (iter > 1 || cont) {
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
-                xn[i] = xv[k][i] + pv[k][i] * va;
-                rn[i] = rv[k][i] + qv[k][i] * vma;
+                for (int i = 0; i < 3; i++) { VT w = pv[i] * vb; w += pp[i]; pp[i] = w; }
             }
-            st3(xcg, n, xn);
-            st3(r, n, rn);
-            if (EXACT) {
-                nd[n] = dot3d(rn, rn);
-            } else if (zbuf) {   // z = P^-1 r for the next iteration, and r.z
-                VT zn[3];
-                precond_z(in.pcg, dinv, binv, n, rn, zn);
-                st3(zbuf, n, zn);
-                rr += dot3d(rn, zn);
-            } else {
-                rr += dot3d(rn, rn);
+            st3(p, n, pp);
+            VT qn[3] = {0, 0, 0};
+            if (in.m_cg != 0.0) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) mass_term(in, m, in.m_cg, pp[i], qn[i]);
             }
+#pragma unroll
+            for (int k = 0; k < kSlotBatch; k++) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) qn[i] = s0 + k < s1 ? qn[i] + sv[k][i] : qn[i];
+            }
+            sum_slots<false>(sp, s0 + kSlotBatch, s1, qn);
+            if (ct) plane_dforce(in, in.k_cg, pp, qn);
+            if (fx) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
+#pragma unroll
+            for (int i = 0; i < 3; i++) { pv[i] = pp[i]; qv[i] = qn[i]; }
+        }
+        VT xn[3], rn[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            xn[i] = xv[i] + pv[i] * va;
+            rn[i] = rv[i] + qv[i] * vma;
+        }
+        st3(xcg, n, xn);
+        st3(r, n, rn);
+        if (EXACT) {
+            nd[n] = dot3d(rn, rn);
+        } else if (zbuf) {   // z = P^-1 r for the next iteration, and r.z
+            VT zn[3];
+            precond_mul(in.pcg, B, rn, zn);
+            st3(zbuf, n, zn);
+            rr = dot3d(rn, zn);
+        } else {
+            rr = dot3d(rn, rn);
         }
     }
     if (EXACT) return;
-    const double tot = wave_block_sum<kBlock>(rr, sh);
-    if (threadIdx.x == 0) prho[nb.pslot] = tot;
+    // the partial of r.r: nodes t, t + kBlock, ... of each of the first kBlock threads, then their tree
+    if (t >= kBlock) upper[t - kBlock] = rr;
+    __syncthreads();
+    if (t < kBlock) {
+#pragma unroll
+        for (int k = 0; k + 1 < kNodesPerThread; k++) rr += upper[k * kBlock + t];
+        rr = wave_sum(rr);
+        if (lane == 0) sh[1][t >> 6] = rr;
+    }
+    __syncthreads();
+    if (t == 0) {
+        double v = sh[1][0];
+#pragma unroll
+        for (int k = 1; k < kBlock / 64; k++) v = v + sh[1][k];
+        prho[nb.pslot] = v;
+    }
 }
 
 // start of a component-level CG solve on the tiled kernels: r = b = the caller's right-hand side,

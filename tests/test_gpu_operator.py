@@ -57,6 +57,47 @@ def test_tile_operator(prec, n, kind):
 
 
 @pytest.mark.parametrize("prec", ["FP64_TILED", "FP32"])
+def test_many_tiles(prec):
+    """More than 256 tiles: the scene's partial sums are added by the block, in the operator and in the update.  Bars
+    as above."""
+    from specs import oracle_from_spec
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: many tiles {prec}", flush=True)
+    spec = _spec((21, 21, 81), "one")
+    o = oracle_from_spec(spec, 0)
+    o.step(spec["dt"], 1)
+    eng = capi.Engine(0, getattr(capi, prec))
+    sid = workloads.add_to_engine(eng, spec)
+    eng.commit()
+    assert eng.tiling(sid)["tiles"] > 256
+    eng.step([sid], 1)
+    x = eng.read(sid)[0]
+    eng.close()
+    assert float(np.linalg.norm(x - o.get("x")) / np.linalg.norm(o.get("x"))) <= BARS[prec]
+
+
+def test_many_node_blocks():
+    """The untiled FP64 engine above 512 node blocks (131,072 nodes), where a scene's partials of p.q and r.r are
+    added by a kernel of its own: the oracle's blocked sums, bit for bit."""
+    from specs import oracle_from_spec
+    from sofa_amd import workloads
+    capi = _capi()
+    print("case: many node blocks", flush=True)
+    spec = dict(_spec((52, 52, 49), "one"), iters=4)
+    assert len(spec["pos"]) > 512 * 256
+    o = oracle_from_spec(spec, 1)
+    o.step(spec["dt"], 1)
+    eng = capi.Engine(0, capi.FP64)
+    sid = workloads.add_to_engine(eng, spec)
+    eng.commit()
+    eng.step([sid], 1)
+    x, v, _ = eng.read(sid)
+    eng.close()
+    assert np.array_equal(x, o.get("x")) and np.array_equal(v, o.get("v"))
+
+
+@pytest.mark.parametrize("prec", ["FP64_TILED", "FP32"])
 def test_cg_solve_keeps_the_force_calls_rotations(prec):
     """cg_solve computes the rotations of the engine's own positions; addDForce after it still uses the last
     addForce's, so its result has the same bits before and after."""
