@@ -109,6 +109,21 @@ static void material_factors(double E, double nu, double ks[3]) {
     ks[2] = k33 * s;
 }
 
+// out = the n values in double; whether all of them are finite (an exponent of ones is not)
+template <typename VT>
+static bool widen(const VT* __restrict__ in, double* __restrict__ out, int64_t n) {
+    typedef typename std::conditional<sizeof(VT) == 4, uint32_t, uint64_t>::type U;
+    const U ones = sizeof(VT) == 4 ? (U)0x7f800000u : (U)0x7ff0000000000000ull;
+    U bad = 0;
+    for (int64_t i = 0; i < n; i++) {
+        U u;
+        std::memcpy(&u, in + i, sizeof(U));
+        bad |= (U)((u & ones) == ones);
+        out[i] = (double)in[i];
+    }
+    return bad == 0;
+}
+
 static bool init_element(const std::vector<V3>& P, const int32_t* t, double E, double nu, ElemInit& out) {
 #pragma clang fp contract(off)
     const V3 &pa = P[t[0]], &pb = P[t[1]], &pc = P[t[2]], &pd = P[t[3]];
@@ -309,7 +324,7 @@ struct EngineBase {
     }
     virtual void commit() = 0;
     virtual void step(const int32_t* ids, int n, int nsteps, hipStream_t s) = 0;
-    virtual void read(int scene, double* x, double* v, double* f) = 0;
+    virtual bool read(int scene, double* x, double* v, double* f) = 0;   // whether every value is finite
     virtual void write(int scene, const double* x, const double* v) = 0;
     virtual void stats(int scene, sofa_amd_cg_stats* out) = 0;
     virtual void element(int scene, int e, double* rot9, double* k3, double* rest12) = 0;
@@ -391,6 +406,27 @@ struct EngineT : EngineBase {
     // element record (SoA, in tile order on the tiled path, else in element order)
     int4* tet = nullptr;
     R *rot = nullptr, *rest = nullptr, *kmat = nullptr;
+    // read-back: two halves of pinned memory, made at commit, a half as large as the largest scene's state
+    // but at most kStageMost (8 MiB of it took 250 us to make, as much as a small scene's whole set-up)
+    static constexpr int64_t kStageMost = 2 << 20;
+    int64_t stage_half = 0;
+    char* stage = nullptr;
+    hipEvent_t stage_ev[2] = {};
+    std::mutex stage_lock;
+    void ensure_stage() {
+        int64_t need = live_mode ? kStageMost : 0;
+        for (const SceneHost& sc : scenes) need = std::max<int64_t>(need, 9 * (int64_t)sc.n_nodes * (int64_t)sizeof(VT));
+        need = std::min<int64_t>(kStageMost, (need + 4095) / 4096 * 4096);
+        if (need <= stage_half) return;
+        if (stage) HIPCHK(hipHostFree(stage));
+        stage = nullptr;
+        stage_half = 0;
+        if (need == kStageMost)   // some scene takes several chunks
+            for (hipEvent_t& e : stage_ev)
+                if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPCHK(hipHostMalloc((void**)&stage, 2 * need));
+        stage_half = need;
+    }
     VT *ef = nullptr, *ef2 = nullptr;
     std::vector<std::vector<int>> iperm;           // per scene: original element -> position
     VT* p2 = nullptr;                              // previous CG direction (exact path)
@@ -477,6 +513,9 @@ struct EngineT : EngineBase {
         for (hipEvent_t e : turn_ev)
             if (e) (void)hipEventDestroy(e);
         if (fork_ev) (void)hipEventDestroy(fork_ev);
+        for (hipEvent_t e : stage_ev)
+            if (e) (void)hipEventDestroy(e);
+        if (stage) (void)hipHostFree(stage);
         while (!vmd.empty()) free_vm(vmd.begin()->first);
         while (!kd.empty()) free_k(kd.begin()->first);
         while (!lmd.empty()) free_lm(lmd.begin()->first);
@@ -784,6 +823,7 @@ struct EngineT : EngineBase {
         HIPCHK(hipSetDevice(device));
         if (tiled) commit_tiled();
         else commit_exact();
+        ensure_stage();
         committed = true;
     }
 
@@ -1020,6 +1060,7 @@ struct EngineT : EngineBase {
             HIPCHK(hipMemset(prr, 0, std::max<int64_t>(1, cap.nblk) * sizeof(double)));
             inst_in = dalloc<InstDev>(cap.sid);
         }
+        ensure_stage();
         place.assign(scenes.size(), Place());
         iperm.resize(scenes.size());
         HIPCHK(hipDeviceSynchronize());
@@ -1873,17 +1914,49 @@ struct EngineT : EngineBase {
         out[4] = 4 * out[5];
     }
 
-    void read_vec(const VT* src, int scene, double* out) {
-        const SceneHost& sc = scenes[scene];
-        std::vector<VT> tmp(3 * (size_t)sc.n_nodes);
-        HIPCHK(hipMemcpy(tmp.data(), src + 3 * (int64_t)node_begin(scene), tmp.size() * sizeof(VT), hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < tmp.size(); i++) out[i] = (double)tmp[i];
-    }
-    void read(int scene, double* xo, double* vo, double* fo) override {
+    // the scene's state: one kernel per chunk of stage_half bytes writes it to pinned memory, the host widens and
+    // checks a chunk while the next one is on its way.  Three copies of a beam of 5,000 nodes to pageable
+    // memory took 3 x 25 us and the check as much again.  Measured, before and after: 525 nodes in double 91 -> 29
+    // us, 24 scenes of 7,000 in float 1.89 -> 1.12 ms, 280,000 nodes 1.66 -> 0.66 ms (half of which is the caller's
+    // fresh pages).
+    bool read(int scene, double* xo, double* vo, double* fo) override {
+        HIPCHK(hipSetDevice(device));
         HIPCHK(hipDeviceSynchronize());
-        if (xo) read_vec(x, scene, xo);
-        if (vo) read_vec(v, scene, vo);
-        if (fo) read_vec(f, scene, fo);
+        const SceneHost& sc = scenes[scene];
+        const int64_t n3 = 3 * (int64_t)sc.n_nodes, at = 3 * (int64_t)node_begin(scene);
+        const VT* src[3];
+        double* dst[3];
+        int na = 0;
+        for (auto& pr : {std::make_pair((const VT*)x, xo), std::make_pair((const VT*)v, vo), std::make_pair((const VT*)f, fo)})
+            if (pr.second) { src[na] = pr.first + at; dst[na++] = pr.second; }
+        if (na == 0 || n3 == 0) return true;
+        for (int k = na; k < 3; k++) { src[k] = src[0]; dst[k] = dst[0]; }
+        std::lock_guard<std::mutex> lock(stage_lock);
+        ensure_stage();
+        const int64_t per = stage_half / (int64_t)sizeof(VT), total = na * n3, chunks = (total + per - 1) / per;
+        const auto launch = [&](int64_t c) {
+            const int64_t at0 = c * per, count = std::min(per, total - at0);
+            k_read_state<VT><<<(unsigned)std::min<int64_t>((count + 255) / 256, 2048), 256, 0, stream>>>(
+                src[0], src[1], src[2], n3, at0, count, (VT*)(stage + (c & 1) * stage_half));
+            HIPCHK(hipGetLastError());
+            if (chunks > 1) HIPCHK(hipEventRecord(stage_ev[c & 1], stream));
+        };
+        launch(0);
+        bool finite = true;
+        for (int64_t c = 0; c < chunks; c++) {
+            if (c + 1 < chunks) launch(c + 1);
+            HIPCHK(chunks > 1 ? hipEventSynchronize(stage_ev[c & 1]) : hipStreamSynchronize(stream));
+            const VT* in = (const VT*)(stage + (c & 1) * stage_half);
+            int64_t i = c * per;
+            const int64_t end = std::min(total, i + per);
+            while (i < end) {
+                const int64_t k = i / n3, o = i - k * n3, len = std::min(end - i, n3 - o);
+                finite &= host::widen(in, dst[k] + o, len);
+                in += len;
+                i += len;
+            }
+        }
+        return finite;
     }
     void write(int scene, const double* xi, const double* vi) override {
         HIPCHK(hipDeviceSynchronize());
@@ -2733,11 +2806,8 @@ int sofa_amd_scene_read(sofa_amd_engine eng, int scene, double* x, double* v, do
     GUARD_BEGIN
     if (!scene_of(eng, scene)) return fail(SOFA_AMD_EINVAL, "invalid scene");
     if (!usable(eng, scene)) return fail(SOFA_AMD_ESTATE, "scene not committed");
-    eng->impl->read(scene, x, v, f);
     // the buffers are filled either way; a state that has left the finite numbers is reported
-    const size_t n3 = 3 * (size_t)scene_of(eng, scene)->n_nodes;
-    for (const double* a : {(const double*)x, (const double*)v, (const double*)f})
-        if (a && !all_finite(a, n3)) return fail(SOFA_AMD_ENAN, "non-finite state (NaN or Inf) in the scene read back");
+    if (!eng->impl->read(scene, x, v, f)) return fail(SOFA_AMD_ENAN, "non-finite state (NaN or Inf) in the scene read back");
     return SOFA_AMD_OK;
     GUARD_END
 }

@@ -69,6 +69,18 @@ __device__ __forceinline__ void mass_term(const InstDev& in, VT m, double factor
     }
 }
 
+// entries [first, first + count) of the three vectors a, b, c (n each) one after the other, to pinned host
+// memory: bounded by the host link
+template <typename VT>
+__global__ __launch_bounds__(256) void k_read_state(const VT* __restrict__ a, const VT* __restrict__ b,
+                                                    const VT* __restrict__ c, int64_t n, int64_t first, int64_t count,
+                                                    VT* __restrict__ out) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256) {
+        const int64_t k = first + i;
+        out[i] = k < n ? a[k] : k < 2 * n ? b[k - n] : c[k - 2 * n];
+    }
+}
+
 // vertex part of addMDx: UniformMass.inl:403-419, DiagonalMass.inl:536-559, MeshMatrixMass.inl:1987-2030
 // SPLIT_Z: onto a sum (the right-hand side) z is rounded twice in float too
 template <bool SPLIT_Z = false, typename VT>
