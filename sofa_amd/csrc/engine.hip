@@ -1436,17 +1436,27 @@ struct EngineT : EngineBase {
         const Blk* nb = (const Blk*)cur->b;
         double* ndp = seq_dots ? nd : nullptr;
         const int ready = exact_ready();
+        // few node blocks leave most of the chip idle: four workgroups for each
+        const bool spread = cur->nb <= kSpreadBlocks;
         for (int it = 1; it <= cur->maxit; it++) {
             // direction of iteration it in buffer it & 1, the previous one in the other
             VT* p_new = (it & 1) ? p : p2;
             const VT* p_old = (it & 1) ? p2 : p;
             if (cur->na > 0) k_cg_elem<R, NR, VT><<<cur->na, kBlock, 0, s>>>(ev, eb, inst, r, p_old, ef, it, partial, ready, zi);
             if (cur->nb > 0) {
-                k_cg_node<VT><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, na, ef, r, p_old, p_new, q, it, partial, ready,
-                                                               partial2, ndp, zi);
+                if (spread)
+                    k_cg_node<VT, kSpread><<<cur->nb * kSpread, kNodeThreads / kSpread, 0, s>>>(
+                        nb, inst, na, ef, r, p_old, p_new, q, it, partial, ready, partial2, nd, zi);
+                else
+                    k_cg_node<VT, 1><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, na, ef, r, p_old, p_new, q, it, partial,
+                                                                     ready, partial2, ndp, zi);
                 exact_total(n, s, partial2, kDotPQ);
-                k_cg_update<VT><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, p_new, q, xcg, r, it, partial2, ready, partial, ndp,
-                                                                 pi, zi);
+                if (spread && !ready)
+                    k_cg_update<VT, true><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, p_new, q, xcg, r, it, partial2, ready,
+                                                                           partial, ndp, nd, pi, zi);
+                else
+                    k_cg_update<VT, false><<<cur->nb, kNodeThreads, 0, s>>>(nb, inst, p_new, q, xcg, r, it, partial2, ready,
+                                                                            partial, ndp, nullptr, pi, zi);
                 exact_total(n, s, partial, kDotRR);
             }
         }

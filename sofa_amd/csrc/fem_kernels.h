@@ -129,7 +129,7 @@ template <int NC, typename VT, typename F>
 __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double factor, F dof, VT out[NC]) {
     const int s0 = na.em_ptr[n], s1 = na.em_ptr[n + 1];
     const VT fct = (VT)factor;
-    constexpr int B = NC == 1 ? 8 : 4;
+    constexpr int B = 4;
     for (int s = s0; s < s1; s += B) {
         int nbr[B];
         VT tm[B], d[B][NC];
@@ -150,27 +150,90 @@ __device__ __forceinline__ void mass_edges(const NodeArrays& na, int n, double f
     }
 }
 
+// mass_edges for one component of p = r + beta p_old, the loads of the first edges apart from their use
+template <typename VT>
+struct EdgeTerms {
+    static constexpr int B = 8;
+    int s0, s1;
+    VT val[B], rv[B], pv[B];
+    __device__ __forceinline__ void batch(const NodeArrays& na, int s, bool old, const VT* __restrict__ r,
+                                          const VT* __restrict__ p) {
+        int nbr[B];
+#pragma unroll
+        for (int t = 0; t < B; t++) {
+            const int i = max(min(s + t, s1 - 1), 0);
+            nbr[t] = na.em_nbr[i];
+            val[t] = (VT)na.em_val[i];
+        }
+#pragma unroll
+        for (int t = 0; t < B; t++) {
+            const int64_t w = 3 * (int64_t)nbr[t];
+            rv[t] = r[w];
+            pv[t] = old ? p[w] : (VT)0;
+        }
+    }
+    __device__ __forceinline__ void load(const NodeArrays& na, int n, bool old, const VT* __restrict__ r,
+                                         const VT* __restrict__ p) {
+        s0 = na.em_ptr[n];
+        s1 = na.em_ptr[n + 1];
+        if (s0 < s1) batch(na, s0, old, r, p);
+    }
+    __device__ __forceinline__ void add(const NodeArrays& na, double factor, bool old, VT beta, const VT* __restrict__ r,
+                                        const VT* __restrict__ p, VT& out) {
+        const VT fct = (VT)factor;
+        for (int s = s0; s < s1; s += B) {
+            if (s > s0) batch(na, s, old, r, p);
+#pragma unroll
+            for (int t = 0; t < B; t++)
+                if (s + t < s1) {
+                    VT d = rv[t];
+                    if (old) { d = pv[t] * beta; d += rv[t]; }
+                    out += d * (val[t] * fct);
+                }
+        }
+    }
+};
+
 // A node's element contributions ef[3 slot ..] over its incidence list, in list order, eight
 // incidences at a time: their slots, then their values, are loaded together (the tail at clamped
 // indices), so a node of 24 tetrahedra waits for memory 6 times instead of 48.  Latency is what
 // bounds the node kernels: the CG node kernel, a lane per node, went from 14.0 to 10.3 us on 525 nodes
 // and from 25.7 to 21.7 on 57,000.  Contributions: one component, the loads apart from the adds, so
-// that the first can be in flight while the scene's scalars are summed.
+// that the first can be in flight while the scene's scalars are summed, and each eight while the eight
+// before are added.
 template <typename VT>
 struct Contributions {
     static constexpr int B = 8;
+    int slot[B];
     VT c[B];
-    __device__ __forceinline__ void load(const int* __restrict__ inc, int s, int s1, const VT* __restrict__ ef) {
-        int slot[B];
+    __device__ __forceinline__ void slots(const int* __restrict__ inc, int s, int s1) {
 #pragma unroll
         for (int t = 0; t < B; t++) slot[t] = inc[max(min(s + t, s1 - 1), 0)];   // (an empty list: entry 0)
+    }
+    __device__ __forceinline__ void values(const VT* __restrict__ ef) {
 #pragma unroll
         for (int t = 0; t < B; t++) c[t] = ef[3 * (int64_t)slot[t]];
     }
-    __device__ __forceinline__ void subtract(int s, int s1, VT& acc) const {
+    // the first eight values, and the next eight slots, on their way
+    __device__ __forceinline__ void begin(const int* __restrict__ inc, int s0, int s1, const VT* __restrict__ ef) {
+        slots(inc, s0, s1);
+        values(ef);
+        if (s0 + B < s1) slots(inc, s0 + B, s1);
+    }
+    // acc -= all of them in list order, each eight while the next are on their way
+    __device__ __forceinline__ void subtract(const int* __restrict__ inc, int s0, int s1, const VT* __restrict__ ef, VT& acc) {
+        for (int s = s0; s < s1; s += B) {
+            VT now[B];
 #pragma unroll
-        for (int t = 0; t < B; t++)
-            if (s + t < s1) acc -= c[t];
+            for (int t = 0; t < B; t++) now[t] = c[t];
+            if (s + B < s1) {
+                values(ef);
+                if (s + 2 * B < s1) slots(inc, s + 2 * B, s1);
+            }
+#pragma unroll
+            for (int t = 0; t < B; t++)
+                if (s + t < s1) acc -= now[t];
+        }
     }
 };
 template <bool SUB, typename VT>
@@ -221,13 +284,6 @@ __device__ __forceinline__ void precond_apply(int kind, const double* __restrict
             z[j] = (VT)acc;
         }
     }
-}
-
-// mass_mdx for one component
-template <typename VT>
-__device__ __forceinline__ void mass_mdx_1(const InstDev& in, const double* __restrict__ mass, int n, double factor,
-                                           VT d, VT& out) {
-    mass_term(in, in.mass_kind == kMassUniform ? (VT)in.vertex_mass : (VT)mass[n], factor, d, out);
 }
 
 // the end of a node kernel of three threads per node: each node's three products added in dot3d's
@@ -442,9 +498,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_begin(const Blk* __restrict__ nbl
 constexpr int kNodeThreads = 3 * kBlock;
 
 // the tree of block_sum over sh[0 .. 255], by the first wave (lane 0 has the sum)
-__device__ __forceinline__ double tree_256(const double* sh) {
-    const int l = threadIdx.x;
-    double v = (sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]);
+__device__ __forceinline__ double tree_wave(double v) {
     v = v + __shfl_down(v, 32, 64);
     v = v + __shfl_down(v, 16, 64);
     v = v + dpp_row_from<0x108>(v);
@@ -452,14 +506,19 @@ __device__ __forceinline__ double tree_256(const double* sh) {
     v = v + dpp_row_from<0x102>(v);
     return v + dpp_row_from<0x101>(v);
 }
+__device__ __forceinline__ double tree_256(const double* sh) {
+    const int l = threadIdx.x;
+    return tree_wave((sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]));
+}
 // the scene's sum of its node blocks' partials, in every thread: each of 256 threads a strided sum,
 // then block_sum's tree (last_block_reduce's order)
+template <int TB>
 __device__ __forceinline__ double block_partials(const double* __restrict__ partial, const InstDev& in, double* sh) {
     const int nb = in.nblk_count, b0 = in.nblk_begin;
-    if (threadIdx.x < kBlock) {
+    for (int t = threadIdx.x; t < kBlock; t += TB) {
         double acc = 0.0;
-        for (int k = threadIdx.x; k < nb; k += kBlock) acc = acc + partial[b0 + k];
-        sh[threadIdx.x] = acc;
+        for (int k = t; k < nb; k += kBlock) acc = acc + partial[b0 + k];
+        sh[t] = acc;
     }
     __syncthreads();
     if (threadIdx.x < 64) {
@@ -469,11 +528,46 @@ __device__ __forceinline__ double block_partials(const double* __restrict__ part
     __syncthreads();
     return sh[0];
 }
+// the same from the nodes' terms (at most kSpreadBlocks node blocks, kNodeThreads threads): a wave forms a
+// block's partial.  A step of 25 iterations, spread and not: 7 blocks 372 and 457 us, 26 blocks 408 and
+// 484, 51 blocks 459 and 505, 64 blocks 503 and 529; beyond, adding the terms costs what the gathers gain
+constexpr int kSpreadBlocks = 64, kSpread = 4;
+__device__ __forceinline__ double node_partials(const double* __restrict__ nd, const InstDev& in, double* sh) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int W = kNodeThreads / 64, B = (kSpreadBlocks + W - 1) / W;
+    const double* d = nd + in.node_begin;
+    double v[B][4];
+#pragma unroll
+    for (int k = 0; k < B; k++)
+        if (wave + k * W < in.nblk_count) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int n = (wave + k * W) * kBlock + lane + 64 * i;
+                v[k][i] = n < in.node_count ? d[n] : 0.0;
+            }
+        }
+    if (threadIdx.x < kBlock) sh[threadIdx.x] = 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < B; k++)
+        if (wave + k * W < in.nblk_count) {
+            const double t = tree_wave((v[k][0] + v[k][2]) + (v[k][1] + v[k][3]));
+            if (lane == 0) sh[wave + k * W] = t;
+        }
+    __syncthreads();
+    double t = 0.0;
+    if (threadIdx.x < 64) t = tree_256(sh);
+    __syncthreads();
+    if (threadIdx.x == 0) sh[0] = t;
+    __syncthreads();
+    return sh[0];
+}
 // a dot product of the scene: already in its record (`ready`: summed in the reference's order, or
 // by k_cg_total), or from the partials
+template <int TB>
 __device__ __forceinline__ double cg_dot(const double* __restrict__ partial, const InstDev& in, int which, int ready,
                                          double* sh) {
-    return ready ? in.dots[which] : block_partials(partial, in, sh);
+    return ready ? in.dots[which] : block_partials<TB>(partial, in, sh);
 }
 // a scene of many node blocks: its partials added once, by one block per scene, instead of by every
 // block of the next kernel
@@ -482,7 +576,7 @@ static __global__ __launch_bounds__(kBlock) void k_cg_total(const int* __restric
     __shared__ double sh[kBlock];
     InstDev* ins = &inst[scenes[blockIdx.x]];
     if (ins->stopped) return;
-    const double v = block_partials(partial, *ins, sh);
+    const double v = block_partials<kBlock>(partial, *ins, sh);
     if (threadIdx.x == 0) ins->dots[which] = v;
 }
 
@@ -541,7 +635,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
         if (it > 1) load3(p_old, nid[n], po[n][0], po[n][1], po[n][2]);
     }
     double beta_d = 0.0;
-    if (it > 1 && !cg_next(ins, in, it, cg_dot(prr, in, kDotRR, ready, sh), false, beta_d)) return;
+    if (it > 1 && !cg_next(ins, in, it, cg_dot<kBlock>(prr, in, kDotRR, ready, sh), false, beta_d)) return;
     if ((int64_t)bk.begin + threadIdx.x >= bk.end) return;
     const VT beta = (VT)beta_d;
     R u[12];
@@ -562,32 +656,44 @@ __global__ __launch_bounds__(kBlock) void k_cg_elem(ElemView<R, NR> ev, const Bl
 }
 
 // p (owned node), q = (1 + h rm) M p - h(h + rs) K p, projected; p.q per 256-node block into ppq, or
-// per node into nd (reference order)
-template <typename VT>
-__global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
+// per node into nd (reference order).  S > 1: S workgroups per node block, p.q per node into nd, for the
+// update to form the blocks' partials (node_partials).  What bounds it: the gathers' latency, and on a
+// scene of few blocks the few CUs that issue them (525 nodes: 3, 9,000: 36).  With S = 4, 525 nodes took
+// 4.8 instead of 7.9 us and 9,000 nodes with edge masses 8.3 instead of 17.2, the update 4.8 and 6.3
+// instead of 4.7 and 4.8.
+template <typename VT, int S>
+__global__ __launch_bounds__(kNodeThreads / S) void k_cg_node(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
                                                            NodeArrays na, const VT* __restrict__ ef,
                                                            const VT* __restrict__ r_, const VT* __restrict__ p_old,
                                                            VT* __restrict__ p, VT* __restrict__ q, int it,
                                                            const double* __restrict__ prr, int ready,
                                                            double* __restrict__ ppq, double* __restrict__ nd,
                                                            const VT* __restrict__ z = nullptr) {
-    __shared__ double sh[kBlock], pr[kNodeThreads];
-    const Blk bk = nblk[xcd_item()];
+    constexpr int N = kBlock / S;
+    __shared__ double sh[kBlock], pr[3 * N];
+    const int item = xcd_item();
+    const Blk bk = nblk[item / S];
+    const int first = bk.begin + item % S * N;
     InstDev* ins = &inst[bk.inst];
     const InstDev in = *ins;
     if (in.stopped) return;
     const VT* __restrict__ r = (in.pcg && z) ? z : r_;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
-    const int n = min(bk.begin + j, bk.end - 1);
-    const bool live = bk.begin + j < bk.end;
+    const int n = min(first + j, bk.end - 1);
+    const bool live = first + j < bk.end;
     const int64_t o = 3 * (int64_t)n + c;
     const VT rc = r[o], pc = p_old[o];
     const int s0 = na.inc_ptr[n], s1 = na.inc_ptr[n + 1];
     const bool fixed = na.fixed[n] != 0;
-    Contributions<VT> g;    // the first 8 in flight while the scene's scalars are summed
-    g.load(na.inc, s0, s1, ef + c);
+    // the node's mass, its first edges and its first contributions in flight while the scene's scalars are summed
+    const VT m = in.mass_kind == kMassUniform ? (VT)in.vertex_mass : (VT)na.mass[n];
+    const bool edges = in.m_cg != 0.0 && in.mass_kind == kMassMatrix;
+    EdgeTerms<VT> e;
+    if (edges) e.load(na, n, it > 1, r + c, p_old + c);
+    Contributions<VT> g;
+    g.begin(na.inc, s0, s1, ef + c);
     double beta_d = 0.0;
-    if (it > 1 && !cg_next(ins, in, it, cg_dot(prr, in, kDotRR, ready, sh), in.nblk_begin == bk.pad, beta_d)) return;
+    if (it > 1 && !cg_next(ins, in, it, cg_dot<kNodeThreads / S>(prr, in, kDotRR, ready, sh), in.node_begin == first, beta_d)) return;
     const VT beta = (VT)beta_d;
     // p = r (first iteration) or p *= beta; p += r (cgstep_beta), from the previous p
     VT pn = rc;
@@ -596,18 +702,10 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict_
     // q = 0; mass addMDx(q, p, 1 + h rm); FEM addDForce(q, p, -h(h+rs)); projectResponse(q)
     VT qn = 0;
     if (in.m_cg != 0.0) {
-        mass_mdx_1(in, na.mass, n, in.m_cg, pn, qn);
-        if (in.mass_kind == kMassMatrix)
-            mass_edges<1>(na, n, in.m_cg, [&](int k, VT d[1]) {
-                const int64_t w = 3 * (int64_t)k + c;
-                d[0] = r[w];
-                if (it > 1) { VT t = p_old[w] * beta; t += d[0]; d[0] = t; }
-            }, &qn);
+        mass_term(in, m, in.m_cg, pn, qn);
+        if (edges) e.add(na, in.m_cg, it > 1, beta, r + c, p_old + c, qn);
     }
-    for (int s = s0; s < s1; s += 8) {
-        if (s > s0) g.load(na.inc, s, s1, ef + c);
-        g.subtract(s, s1, qn);
-    }
+    g.subtract(na.inc, s0, s1, ef + c, qn);
     if (in.plane_on) {
         pr[threadIdx.x] = (double)pn;
         __syncthreads();
@@ -622,18 +720,31 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_node(const Blk* __restrict_
     if (fixed) qn = 0;
     if (live) q[o] = qn;
     pr[threadIdx.x] = live ? (double)pn * (double)qn : 0.0;
-    node_partial(pr, sh, nd, bk, ppq);
+    if constexpr (S == 1) {
+        node_partial(pr, sh, nd, bk, ppq);
+    } else {
+        __syncthreads();
+        const int t = threadIdx.x;
+        if (t < N && first + t < bk.end) {
+            double v = pr[3 * t];
+            v += pr[3 * t + 1];
+            v += pr[3 * t + 2];
+            nd[first + t] = v;
+        }
+    }
 }
 
 // den = p.q, the threshold test and alpha (CGLinearSolver.inl:207-265; PCG: alpha = r.z / w.s,
 // PCGLinearSolver.inl:222-224), then x += p alpha; r += q (-alpha) (CGLinearSolver.cpp:46-64,
 // vOp_v_inc_bf) and the partials of r.r (PCG: s = P^-1 r, r.s, PCGLinearSolver.inl:229-244)
-template <typename VT>
+// TERMS: p.q is formed from the nodes' terms (k_cg_node with S > 1, not ready)
+template <typename VT, bool TERMS>
 __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restrict__ nblk, InstDev* __restrict__ inst,
                                                              const VT* __restrict__ p, const VT* __restrict__ q,
                                                              VT* __restrict__ xcg, VT* __restrict__ r, int it,
                                                              const double* __restrict__ ppq, int ready,
                                                              double* __restrict__ prr, double* __restrict__ nd,
+                                                             const double* __restrict__ terms = nullptr,
                                                              const double* __restrict__ pinv = nullptr,
                                                              VT* __restrict__ z = nullptr) {
     __shared__ double sh[kBlock], pr[kNodeThreads];
@@ -647,7 +758,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
     const int64_t o = 3 * (int64_t)n + c;
     const VT pc = p[o], qc = q[o], xc = xcg[o], rc = r[o];
     const bool pcg = in.pcg && pinv;
-    const double den = cg_dot(ppq, in, kDotPQ, ready, sh);
+    const double den = TERMS ? node_partials(terms, in, sh) : cg_dot<kNodeThreads>(ppq, in, kDotPQ, ready, sh);
     const bool record = in.nblk_begin == bk.pad && threadIdx.x == 0;
     if (!in.pcg) {
         const bool exempt = it == 1 && in.first_solve;
@@ -719,7 +830,7 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const int* __restrict__ sce
     InstDev* in = &inst[scenes[blockIdx.x]];
     const bool open = !in->stopped, pcg = in->pcg && in->max_iter > 0;
     double rho = 0.0;
-    if (open && pcg) rho = cg_dot(prr, *in, kDotRR, ready, sh);
+    if (open && pcg) rho = cg_dot<kBlock>(prr, *in, kDotRR, ready, sh);
     if (threadIdx.x != 0) return;
     if (open) {
         in->stopped = 1;

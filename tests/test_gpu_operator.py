@@ -97,6 +97,32 @@ def test_many_node_blocks():
     assert np.array_equal(x, o.get("x")) and np.array_equal(v, o.get("v"))
 
 
+@pytest.mark.parametrize("order", [0, 1])
+@pytest.mark.parametrize("n", [(2, 2, 2), (8, 8, 4), (8, 8, 5), (4, 5, 13), (16, 16, 64), (16, 16, 65)])
+def test_few_node_blocks(n, order):
+    """The untiled FP64 engine's node kernel with four workgroups per node block (up to 64 blocks, 16,384 nodes) and
+    above it: one node block partly and exactly filled and one node more, the last block of the rule and the
+    first beyond; both summation orders; two scenes, so that the second's nodes start inside a block of the
+    flattened arrays.  Bit for bit."""
+    from specs import oracle_from_spec
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: few node blocks {n} order {order}", flush=True)
+    spec = _spec(n, "one")
+    eng = capi.Engine(0, capi.FP64)
+    if order:
+        eng.set_dot_order(True)
+    workloads.add_to_engine(eng, _spec((3, 3, 4), "one"))
+    sid = workloads.add_to_engine(eng, spec)
+    eng.commit()
+    eng.step([0, sid], 2)
+    x, v, _ = eng.read(sid)
+    eng.close()
+    o = oracle_from_spec(spec, 0 if order else 1)
+    o.step(spec["dt"], 2)
+    assert np.array_equal(x, o.get("x")) and np.array_equal(v, o.get("v"))
+
+
 @pytest.mark.parametrize("prec", ["FP64_TILED", "FP32"])
 def test_cg_solve_keeps_the_force_calls_rotations(prec):
     """cg_solve computes the rotations of the engine's own positions; addDForce after it still uses the last
