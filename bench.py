@@ -116,11 +116,11 @@ def time_plain(eng, ids, steps, warmup):
 
 
 def apply_roofline(eng, reps, pe, pv, nrec, E, N, node_extra=0):
-    """The dominant kernel: the tiled CG operator apply k_tile_apply (p = r + beta p staged in LDS,
-    element rotations recomputed from the positions, element K p, per-node sums in LDS, q of
-    tile-owned nodes, partials of shared nodes) over every scene of the engine in one launch,
-    timed with HIP events on its stream.  The element geometry (rotation, rest coordinates) is
-    recomputed from the node positions.
+    """The dominant kernel: the tiled CG operator (p = r + beta p staged in LDS, element K p,
+    per-node sums in LDS, q of tile-owned nodes, partials of shared nodes) over every scene of the
+    engine in one launch, timed with HIP events on its stream.  k_tile_exact (reference order)
+    recomputes the element geometry (rotation, rest coordinates) from the node positions;
+    k_tile_apply reads it back, bytes that an operator can do without and that are not counted here.
     Algorithmic bytes per launch: E (16 + nrec p_e) + N 18 p_v
       per element: 16 B of indices (4 local node ids + 4 incidence slots, u16 each) and nrec
                    reals: the stiffness entries K00, K01, K33 (3) where elements have their own
@@ -639,7 +639,8 @@ def main():
     prec_of = {p[0]: (p[1], p[2]) for p in MIX_PATHS}
     roof = dict(hrow.get("roofline") or {})
     if roof:
-        roof["kernel"] = (f"k_tile_apply<{'float' if head in ('fp32', 'split') else 'double'}> over the 256-beam mix "
+        roof["kernel"] = (f"k_tile_{'exact' if 'exact' in head else 'apply'}"
+                          f"<{'float' if head in ('fp32', 'split') else 'double'}> over the 256-beam mix "
                           "(CG operator: addDForce + mass + projection + p update), path " + head)
         roof["autotuned_variant"] = {"chosen": hrow.get("variant"), "us_per_launch": hrow.get("variant_us")}
         tr = measured_traffic(f"profiles/k_tile_apply_beam_mix_{head}_traffic.md", hrow.get("variant"))

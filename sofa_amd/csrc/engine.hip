@@ -1464,7 +1464,7 @@ struct EngineT : EngineBase {
 
     // the reference's summation order on the tiled kernels (FP64 tiled engines, chosen before
     // the scenes are placed): shared nodes summed incidence by incidence in element order, every
-    // CG dot product node after node (k_seqdot); the trajectories are then the FP64 parity
+    // CG dot product node after node (k_scandot); the trajectories are then the FP64 parity
     // path's in its sequential dot order, bit for bit
     // the CG operator computes elements in float
     bool float_operator() const { return tiled && (mixed || std::is_same<R, float>::value); }

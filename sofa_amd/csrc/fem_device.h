@@ -101,7 +101,7 @@ struct alignas(64) InstDev {
     int dot_fallbacks, pad_fb;
 };
 
-// which entry of InstDev::dots a k_seqdot launch writes
+// which entry of InstDev::dots a dot-product launch (k_scandot, k_seqdot) writes
 constexpr int kDotBB = 0, kDotPQ = 1, kDotRR = 2;
 
 // MechanicalObject::vDot in the reference's order (MechanicalObject.inl:2334-2356): the scene's

@@ -1156,7 +1156,7 @@ __global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ t
 // reference order, after the tile apply: the shared nodes' p = r + beta p, q = (1 + h rm) M p
 // minus their element contributions one by one in ascending element id (continued from the sum
 // the leading run's tile left in the node's first slot), plane and projection, and their p.q
-// terms for k_seqdot (the work k_update does for them in tile order otherwise)
+// terms for k_scandot (the work k_update does for them in tile order otherwise)
 template <typename VT>
 __global__ __launch_bounds__(kBlock) void k_fin_exact(const FinBlk* __restrict__ fb_, InstDev* __restrict__ inst,
                                                        SharedNodes sn, const double* __restrict__ mass,
@@ -1194,7 +1194,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_exact(const FinBlk* __restrict__
 
 // CGLinearSolver warmStart in the reference order (CGLinearSolver.inl:95-99): after the operator
 // of iteration 0 on the previous solution (q = A x, shared nodes finished by k_fin_exact),
-// r.eq(b, q, -1.0): r = b + q (-1) per component, and each node's r.r term for k_seqdot
+// r.eq(b, q, -1.0): r = b + q (-1) per component, and each node's r.r term for k_scandot
 template <typename VT>
 __global__ __launch_bounds__(kBlock) void k_warm_begin_exact(const NodeBlk* __restrict__ nb_,
                                                               const InstDev* __restrict__ inst,
@@ -1307,7 +1307,7 @@ __device__ __forceinline__ void precond_z(int kind, const float* __restrict__ di
 // the tile partials (which already hold every node's term), the threshold test and alpha
 // (CGLinearSolver.inl:207-265), x += alpha p, r -= alpha q and the r.r partials.
 // EXACT: every node's p and q are final (k_fin_exact finished the shared ones), den is the
-// reference-order p.q of k_seqdot, and each node's r.r term goes to nd.  zbuf (MIXED inner CG
+// reference-order p.q of k_scandot, and each node's r.r term goes to nd.  zbuf (MIXED inner CG
 // with a preconditioner): it holds z = P^-1 r of the previous residual (shared nodes' p = z +
 // beta p); each node's new z (precond_z with dinv / binv) replaces it, r.z partials in place of r.r
 // One thread per node, and everything that a node may need -- a shared node's slot range and its first
@@ -1452,7 +1452,7 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
 
 // start of a component-level CG solve on the tiled kernels: r = b = the caller's right-hand side,
 // x = 0, and |b|^2 as per-node-block partials (read by the tile apply of iteration 1 with
-// pin_nodes = 1) or, in the reference order, as per-node terms for k_seqdot
+// pin_nodes = 1) or, in the reference order, as per-node terms for k_scandot
 template <typename VT, bool EXACT = false>
 __global__ __launch_bounds__(kBlock) void k_cg_begin_tiled(const NodeBlk* __restrict__ nb_, const VT* __restrict__ b_in,
                                                             int nb0, VT* __restrict__ b, VT* __restrict__ r,
