@@ -1569,11 +1569,19 @@ struct EngineT : EngineBase {
     template <bool WIDE, bool PLANE>
     void launch_apply_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp,
                         const double* pin, double* pd, int pin_nodes) {
-        if (variant_threads(apply_variant) == 512)
-            k_tile_apply<R, NR, VT, 512, WIDE, PLANE><<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
-        else
-            k_tile_apply<R, NR, VT, 256, WIDE, PLANE><<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes);
+        // (set_apply_variant 1 and 3 on a float engine: the host's rest shape, always read back)
+        const bool geo = ta.rot == rot && !(std::is_same<R, float>::value && (apply_variant & 1)) &&
+                         (int64_t)na * kTileElems * (12 + NR) * (int64_t)sizeof(R) > kRecordCached;
+        if (variant_threads(apply_variant) == 512) {
+            const auto op = geo ? k_tile_apply<R, NR, VT, 512, WIDE, PLANE, true> : k_tile_apply<R, NR, VT, 512, WIDE, PLANE>;
+            op<<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0);
+        } else {
+            const auto op = geo ? k_tile_apply<R, NR, VT, 256, WIDE, PLANE, true> : k_tile_apply<R, NR, VT, 256, WIDE, PLANE>;
+            op<<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0);
+        }
     }
+    // a launch set's record beyond this does not stay in the last-level cache (k_tile_apply's GEO)
+    static constexpr int64_t kRecordCached = 256 << 20;
     template <bool PLANE>
     void launch_exact_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp) {
         switch (apply_variant) {
@@ -2402,7 +2410,7 @@ void launch_inner_cg(const InnerCg& c, hipStream_t s) {
                                               : k_tile_apply<float, 6, float, kTileThreads, true, false>)
                                    : (c.plane ? k_tile_apply<float, 6, float, kTileThreads, false, true>
                                               : k_tile_apply<float, 6, float, kTileThreads, false, false>);
-            op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1);
+            op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, nullptr, nullptr);
         }
         if (c.nnb > 0)
             k_update<float><<<c.nnb, kUpdateThreads, 0, s>>>(c.nb, c.ta.inst, c.ta.ranges, it, c.sn, c.sp, c.ta.mass, c.ta.fixed,

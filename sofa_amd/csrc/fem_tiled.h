@@ -646,16 +646,21 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
 // holds (FP64: two, by registers and LDS); on a small one that latency alone.  Measured, before (geometry
 // recomputed, a thread per node for staging and sums) and after: FP32 1.31M tetrahedra 32.2 -> 29.9 us, 24
 // beams of 0.6M 24.9 -> 22.6, 18,954 7.2 -> 6.6; SPLIT 150k 11.1 -> 10.2; FP64 360k 24.9 -> 22.8.
+// GEO: the record recomputed from the positions all the same (same bits), for launch sets whose record does
+// not stay in the 256 MB last-level cache from one iteration to the next.  256 beams of 8.9M tetrahedra, recomputed
+// and read back: FP32 5.9 and 6.8 ms/step, SPLIT 7.7 and 9.2, FP64 12.0 and 13.9; at 1.31M tetrahedra (94 MB of
+// record) and below reading back is the faster one.
 // PLANE = false: no scene of the launch has a PlaneForceField; WIDE = false: no scene has more than
 // kWavePartials partials of r.r, which are then in flight with the gathers.
 constexpr int kNodeMass = 1 << 12;   // the node's sum starts from the mass term
 static_assert(4 * kTileElems <= kNodeMass, "a node's first incidence and the flag share 16 bits");
-template <typename R, int NR, typename VT, int TB, bool WIDE, bool PLANE>
+template <typename R, int NR, typename VT, int TB, bool WIDE, bool PLANE, bool GEO = false>
 __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, const VT* __restrict__ r,
                                                     VT* __restrict__ p, VT* __restrict__ q, VT* __restrict__ sp,
                                                     const double* __restrict__ pin,   // |b|^2 (iter 1) or r.r partials
                                                     double* __restrict__ pden,
-                                                    int pin_nodes) {   // 1: iter-1 |b|^2 partials per node block
+                                                    int pin_nodes,     // 1: iter-1 |b|^2 partials per node block
+                                                    const VT* __restrict__ x, const VT* __restrict__ x0) {   // GEO
     constexpr int EPT = kTileElems / TB;                   // elements per thread
     constexpr int NPT = (kTileNodes + TB - 1) / TB;        // tile-local nodes per thread
     __shared__ VT lu[kTileNodes * 3];        // p (in R), then the nodes' sums
@@ -669,7 +674,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     InstDev* ins = &a.inst[td.scene];
     const InstDev in = *ins;
     const Ranges rg = a.ranges[td.scene];
-    const bool consistent = (td.flags & kTileConsistent) != 0;
+    const bool consistent = (td.flags & kTileConsistent) != 0, one = (td.flags & kTileOneMaterial) != 0;
     const int ninc = 4 * td.e_count;
     // a refinement sweep that keeps the previous search direction continues CG at its iteration 1
     const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
@@ -701,16 +706,19 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         if ((int)k < td.e_count) {
             lt[m] = (a.ltet + td.e_begin)[k];
             inc[m] = reinterpret_cast<const uint2*>(a.tn.inc + td.inc_begin)[k];   // four incidences
+            if (!GEO) {
 #pragma unroll
-            for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.ev.E + td.e_begin))[k];
+                for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.ev.E + td.e_begin))[k];
 #pragma unroll
-            for (int i = 0; i < NR; i++) rin[m][i] = (a.rest + (i * a.ev.E + td.e_begin))[k];
+                for (int i = 0; i < NR; i++) rin[m][i] = (a.rest + (i * a.ev.E + td.e_begin))[k];
+            }
+            if (!GEO || !one)
 #pragma unroll
-            for (int i = 0; i < 3; i++) kk[m][i] = (a.kmat + (i * a.ev.E + td.e_begin))[k];
+                for (int i = 0; i < 3; i++) kk[m][i] = (a.kmat + (i * a.ev.E + td.e_begin))[k];
             em[m] = consistent ? (a.emass + td.e_begin)[k] : (R)0;
         }
     }
-    VT pv[NPT][3], po[NPT][3], ms[NPT];
+    VT pv[NPT][3], po[NPT][3], ms[NPT], xt[NPT][3], x0t[NPT][3];
     int8_t fx[NPT], ct[NPT];
     const bool plane = PLANE && in.plane_on, table = in.mass_kind != kMassUniform;
 #pragma unroll
@@ -718,6 +726,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         if (w0 + m * TB < td.ln_count) {
             ld3(r, gid[m], pv[m]);
             if (second) ld3(p, gid[m], po[m]);
+            if (GEO) { ld3(x, gid[m], xt[m]); ld3(x0, gid[m], x0t[m]); }
             ms[m] = table ? (VT)a.mass[gid[m]] : (VT)in.vertex_mass;
             fx[m] = a.fixed[gid[m]];
             ct[m] = plane ? a.contact[gid[m]] : 0;
@@ -778,6 +787,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
                     for (int i = 0; i < 3; i++) {
                         pv[m][i] = (VT)(R)pv[m][i];
                         lu[3 * j + i] = pv[m][i];
+                        if (GEO) { lc[3 * j + i] = (R)xt[m][i]; lc[3 * kTileNodes + 3 * j + i] = (R)x0t[m][i]; }
                     }
                     lmass[j] = ms[m];
                     lnode[j] = (uint16_t)(s0[m] | (in.m_cg != 0.0 && interior ? kNodeMass : 0));
@@ -788,6 +798,28 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     if (threadIdx.x == 0) halt = !go;
     __syncthreads();
     if (halt) return;
+    if constexpr (GEO) {   // the record from the staged positions, then their buffer is free
+#pragma unroll
+        for (int m = 0; m < EPT; m++) {
+            const int k = threadIdx.x + m * TB;
+            if (k < td.e_count) {
+                int l[4];
+                unpack_ltet(lt[m], l);
+                R xe[3][3], x0e[4][3];
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
+                        if (v < 3) xe[v][i] = lc[3 * l[v] + i];
+                        x0e[v][i] = lc[3 * kTileNodes + 3 * l[v] + i];
+                    }
+                rotation_large(xe[0], xe[1], xe[2], rot[m]);
+                rest_frame<R, NR>(x0e, rin[m]);
+                if (one) stiffness_from_volume(x0e, in.ks, kk[m]);
+            }
+        }
+        __syncthreads();
+    }
     // ---- 3. element K p into LDS
     const R kcg = (R)in.k_cg, mcg = (R)in.m_cg;
 #pragma unroll

@@ -97,6 +97,29 @@ def test_many_node_blocks():
     assert np.array_equal(x, o.get("x")) and np.array_equal(v, o.get("v"))
 
 
+@pytest.mark.parametrize("prec,copies", [("FP64_TILED", 6), ("FP32", 14)])
+def test_large_sets(prec, copies):
+    """A launch set whose element records exceed 256 MB (the operator recomputes them) against the same scenes
+    stepped one by one (it reads them back): the same bits, with materials per element and one material."""
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: large sets {prec}", flush=True)
+    specs = [_spec((33, 33, 65), "materials"), _spec((33, 33, 65), "one")]
+    out = []
+    for together in (True, False):
+        eng = capi.Engine(0, getattr(capi, prec))
+        ids = [workloads.add_to_engine(eng, specs[k % 2]) for k in range(copies)]
+        eng.commit()
+        per_tet = 72 if prec == "FP32" else 168
+        assert sum(eng.tiling(i)["tiles"] for i in ids) * 512 * per_tet > 256 << 20
+        for group in ([ids] if together else [[i] for i in ids[:2]]):
+            eng.step(group, 2)
+        out.append([eng.read(i)[:2] for i in ids[:2]])
+        eng.close()
+    for (x, v), (xs, vs) in zip(*out):
+        assert np.array_equal(x, xs) and np.array_equal(v, vs)
+
+
 @pytest.mark.parametrize("order", [0, 1])
 @pytest.mark.parametrize("n", [(2, 2, 2), (8, 8, 4), (8, 8, 5), (4, 5, 13), (16, 16, 64), (16, 16, 65)])
 def test_few_node_blocks(n, order):
