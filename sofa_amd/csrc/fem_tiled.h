@@ -648,8 +648,8 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
 // beams of 0.6M 24.9 -> 22.6, 18,954 7.2 -> 6.6; SPLIT 150k 11.1 -> 10.2; FP64 360k 24.9 -> 22.8.
 // GEO: the record recomputed from the positions all the same (same bits), for launch sets whose record does
 // not stay in the 256 MB last-level cache from one iteration to the next.  256 beams of 8.9M tetrahedra, recomputed
-// and read back: FP32 5.9 and 6.8 ms/step, SPLIT 7.7 and 9.2, FP64 12.0 and 13.9; at 1.31M tetrahedra (94 MB of
-// record) and below reading back is the faster one.
+// and read back: FP32 5.9 and 6.8 ms/step, SPLIT 7.7 and 9.2, FP64 12.0 and 13.9; the operator
+// of 1.31M tetrahedra in float (94 MB of record) 33.4 and 29.7 us, of 0.6M 25.6 and 22.7, of 360k in double 23.6 and 22.4.
 // PLANE = false: no scene of the launch has a PlaneForceField; WIDE = false: no scene has more than
 // kWavePartials partials of r.r, which are then in flight with the gathers.
 constexpr int kNodeMass = 1 << 12;   // the node's sum starts from the mass term
@@ -698,6 +698,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     const int lane = threadIdx.x & 63;
     SceneTerms part;
     if (!WIDE && iter > 0 && w0 < td.ln_count) load_terms<TB, WIDE>(pin + pa, pn, part);
+    if (in.stopped) return;   // before the record's loads: a converged scene's launches are many
     R rot[EPT][9], rin[EPT][NR], kk[EPT][3], em[EPT];
     uint2 lt[EPT], inc[EPT];
 #pragma unroll
@@ -736,7 +737,6 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         const int k = threadIdx.x + m * TB;
         if (k < td.e_count) *reinterpret_cast<uint2*>(linc + 4 * k) = inc[m];
     }
-    if (in.stopped) return;
     const bool first = (td.flags & kTileFirst) != 0;
     // ---- 2. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
     double total = 0.0, beta = 0.0;      // |b|^2 or r.r
@@ -1381,6 +1381,7 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
     if (zbuf) ld3(zbuf, n, zv);
     ld3(p, n, pv);
     ld3(q, n, qv);
+    if (in.stopped) return;
     VT m = 0;
     int8_t fx = 0, ct = 0;
     float B[9];
@@ -1398,7 +1399,6 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
             for (int k = 0; k < kSlotBatch; k++) ld3(sp, min(s0 + k, s1 - 1), sv[k]);
         }
     }
-    if (in.stopped) return;
     const bool cont = iter == 1 && in.keep_dir && in.sweep > 1;
     const bool first = nb.first != 0;
     double den;
