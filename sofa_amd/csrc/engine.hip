@@ -1653,6 +1653,7 @@ struct EngineT : EngineBase {
         ta.emass = emass;
         ta.nd = nd;
         ta.rot = rot;
+        ta.rot_row = Etot;
         ta.rest = rest;
         ta.kmat = kmat;
         if constexpr (std::is_same<R, float>::value)
@@ -1703,7 +1704,7 @@ struct EngineT : EngineBase {
         ic.ta.contact = contact;
         ic.ta.emass = emass32;
         ic.ta.nd = nullptr;
-        ic.ta.rot = rot32; ic.ta.rest = restf; ic.ta.kmat = kmatf;
+        ic.ta.rot = rot32; ic.ta.rot_row = Etot; ic.ta.rest = restf; ic.ta.kmat = kmatf;
         ic.ta.rot32 = nullptr;
         // PCGLinearSolver with a Jacobi preconditioner: the inner CG runs preconditioned (in the node
         // kernels: the operator reads z)
@@ -2158,12 +2159,16 @@ struct EngineT : EngineBase {
         } else {
             TileArgs<R, NR> ta = tile_args();
             const int64_t nE = (int64_t)scenes[scene].tets.size() / 4, e0 = elem_begin(scene);
-            R* const rot_cg = reinterpret_cast<R*>(ef);   // scratch of the force calls: 12 VT per element
             bool exact = false;
             if constexpr (std::is_same<R, double>::value) exact = exact_tiled();
-            if (!exact && nE > 0) {   // the rotations of the engine's positions (ev.rot keeps addForce's)
-                k_rotations<R, VT><<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, s>>>(tet, e0, e0 + nE, x, rot_cg, Etot);
+            if (!exact && nE > 0) {
+                // the rotations of the engine's positions (ev.rot keeps addForce's), in the scene's own share of
+                // the force calls' scratch (12 VT per element, from 12 e0): another scene's force call may be
+                // using its share on another stream.  Rows of nE; element e is at e - e0 of a row.
+                R* const rot_cg = reinterpret_cast<R*>(ef + 12 * e0) - e0;
+                k_rotations<R, VT><<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, s>>>(tet, e0, e0 + nE, x, rot_cg, nE);
                 ta.rot = rot_cg;
+                ta.rot_row = nE;
             }
             const FinBlk* fb = (const FinBlk*)cur->b;
             const NodeBlk* nbk = (const NodeBlk*)cur->c;

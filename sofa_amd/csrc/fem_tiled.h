@@ -267,6 +267,7 @@ struct TileArgs {
     double* __restrict__ nd;            // reference order: per-node dot terms
     // the operator's element record, SoA: rotations (written by the step's force pass), rest shape, K
     const R *rot, *rest, *kmat;
+    int64_t rot_row;                    // length of a row of rot (rest and kmat: ev.E)
     float* rot32;                       // MIXED: the inner operator's rotations, written by the force pass
 };
 
@@ -709,7 +710,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
             inc[m] = reinterpret_cast<const uint2*>(a.tn.inc + td.inc_begin)[k];   // four incidences
             if (!GEO) {
 #pragma unroll
-                for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.ev.E + td.e_begin))[k];
+                for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.rot_row + td.e_begin))[k];
 #pragma unroll
                 for (int i = 0; i < NR; i++) rin[m][i] = (a.rest + (i * a.ev.E + td.e_begin))[k];
             }
@@ -1170,7 +1171,7 @@ static __global__ __launch_bounds__(kBlock) void k_rest_float(const int4* __rest
 // follow a force pass (component-level CG)
 template <typename R, typename VT>
 __global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ tet, int64_t e0, int64_t e1,
-                                                       const VT* __restrict__ x, R* __restrict__ rot, int64_t E) {
+                                                       const VT* __restrict__ x, R* __restrict__ rot, int64_t row) {
     const int64_t e = e0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (e >= e1) return;
     const int4 t = tet[e];
@@ -1182,7 +1183,7 @@ __global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ t
         for (int i = 0; i < 3; i++) p[n][i] = (R)x[3 * (int64_t)v[n] + i];
     rotation_large(p[0], p[1], p[2], ro);
 #pragma unroll
-    for (int i = 0; i < 9; i++) rot[i * E + e] = ro[i];
+    for (int i = 0; i < 9; i++) rot[i * row + e] = ro[i];
 }
 
 // reference order, after the tile apply: the shared nodes' p = r + beta p, q = (1 + h rm) M p

@@ -169,3 +169,43 @@ def test_cg_solve_keeps_the_force_calls_rotations(prec):
     a, b = before.numpy(), after.numpy()
     eng.close()
     assert np.any(a) and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("first", [0, 1])
+@pytest.mark.parametrize("prec", ["FP64_TILED", "FP32", "SPLIT"])
+def test_cg_solve_beside_force_calls(prec, first):
+    """cg_solve of one scene on one stream while force calls of another scene of the same engine are in flight on
+    a second stream: scenes share no buffer, so each has the bits that it has alone."""
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: cg_solve of scene {first} beside force calls, {prec}", flush=True)
+    dt = np.float32 if prec == "FP32" else np.float64
+    specs = [_spec((9, 9, 40), "one"), _spec((8, 9, 33), "materials")]
+    eng = capi.Engine(0, getattr(capi, prec))
+    for s in specs:
+        workloads.add_to_engine(eng, s)
+    eng.commit()
+    a, b = first, 1 - first
+    rng = np.random.default_rng(5)
+    dev = lambda v: capi.DeviceArray(np.ascontiguousarray(v, dtype=dt))
+    shape = [s["pos"].shape for s in specs]
+    rhs, x, dx = (dev(rng.standard_normal(shape[a])), dev(specs[b]["pos"] + 0.01 * rng.standard_normal(shape[b])),
+                  dev(rng.standard_normal(shape[b])))
+    one, two = capi.Stream(), capi.Stream()
+    got = []
+    for beside in (False, True):
+        sol, f = dev(np.zeros(shape[a])), dev(np.zeros(shape[b]))
+        for _ in range(8):
+            for _ in range(40):
+                eng.fem_add_force(b, x.ptr, f.ptr, stream=two)
+                eng.fem_add_dforce(b, dx.ptr, f.ptr, -0.5, stream=two)
+            if not beside:
+                two.synchronize()
+            eng.cg_solve(a, 1.0, 0.0, -1e-3, rhs.ptr, sol.ptr, stream=one)
+        two.synchronize()
+        got.append((sol.numpy(), f.numpy()))
+        sol.close()
+        f.close()
+    eng.close()
+    assert np.any(got[0][0]) and np.any(got[0][1])
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
