@@ -24,6 +24,8 @@
 #include <float.h>
 #include <type_traits>
 
+#include "stop_mark.h"
+
 namespace sofa_amd {
 
 constexpr int kBlock = 256;   // threads per block for every kernel (4 wave64)
@@ -37,7 +39,7 @@ constexpr int kBlock = 256;   // threads per block for every kernel (4 wave64)
 // kernel).  Fields are written through the pointer.
 struct alignas(64) InstDev {
     // what the kernels of a CG iteration read: two cache lines (CGLinearSolver.inl:86-270)
-    int stopped;                      // 1 once the loop has exited
+    int stopped;                      // not 0 once the loop has exited: by which launch (stop_mark)
     int first_solve;                  // timeStepCount == 0
     int max_iter;
     int mass_kind;                    // 0 uniform, 1 diagonal

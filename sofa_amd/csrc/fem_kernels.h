@@ -492,8 +492,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_begin(const Blk* __restrict__ nbl
 // as one partial per 256-node block; whoever needs the sum adds the partials itself, in the order the
 // scalars of a solve have always been summed, so no block waits for or fences against another.  The
 // scene's record is written by its first node block only: every field that the other blocks of the
-// same kernel read (rho_slot of the other parity, limits) is left alone there, and a stop they may see
-// early is the one they reach themselves.
+// same kernel read (rho_slot of the other parity, limits) is left alone there, and a stop that it records
+// is passed over by them (stopped_before): they reach it themselves.
 // ---------------------------------------------------------------------------------------
 constexpr int kNodeThreads = 3 * kBlock;
 
@@ -599,7 +599,7 @@ __device__ __forceinline__ bool cg_next(InstDev* ins, const InstDev& in, int it,
     if (record) {
         if (in.pcg || !over) ins->err = err;
         if (stop) {
-            ins->stopped = 1;
+            ins->stopped = stop_mark(it, 0);
             ins->end_reason = over ? 0 : 1;
             ins->last_iters = over && !in.pcg ? in.max_iter : it;
         } else {
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(kNodeThreads / S) void k_cg_node(const Blk* __restr
     const int first = bk.begin + item % S * N;
     InstDev* ins = &inst[bk.inst];
     const InstDev in = *ins;
-    if (in.stopped) return;
+    if (stopped_before(in.stopped, stop_mark(it, 0))) return;
     const VT* __restrict__ r = (in.pcg && z) ? z : r_;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
     const int n = min(first + j, bk.end - 1);
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
     const Blk bk = nblk[xcd_item()];
     InstDev* ins = &inst[bk.inst];
     const InstDev in = *ins;
-    if (in.stopped) return;
+    if (stopped_before(in.stopped, stop_mark(it, 1))) return;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
     const int n = min(bk.begin + j, bk.end - 1);
     const bool live = bk.begin + j < bk.end;
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
         const bool exempt = it == 1 && in.first_solve;
         const int stop = den == 0.0 ? 3 : fabs(den) <= in.thr && !exempt ? 2 : 0;
         if (stop) {
-            if (record) { ins->den = den; ins->stopped = 1; ins->end_reason = stop; ins->last_iters = it; }
+            if (record) { ins->den = den; ins->stopped = stop_mark(it, 1); ins->end_reason = stop; ins->last_iters = it; }
             return;
         }
     }

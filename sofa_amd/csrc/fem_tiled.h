@@ -232,10 +232,10 @@ __device__ __forceinline__ void st3(VT* __restrict__ v, int n, const VT o[3]) {
 }
 
 // stop the scene's CG loop: every block of the kernel reaches the same decision; the first
-// block records it
-__device__ __forceinline__ void record_stop(InstDev* ins, bool first, int reason, int iters, double err) {
+// block records it, with the launch's mark
+__device__ __forceinline__ void record_stop(InstDev* ins, bool first, int mark, int reason, int iters, double err) {
     if (first && threadIdx.x == 0) {
-        ins->stopped = 1;
+        ins->stopped = mark;
         ins->end_reason = reason;
         ins->last_iters = iters;
         ins->err = err;
@@ -699,7 +699,8 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     const int lane = threadIdx.x & 63;
     SceneTerms part;
     if (!WIDE && iter > 0 && w0 < td.ln_count) load_terms<TB, WIDE>(pin + pa, pn, part);
-    if (in.stopped) return;   // before the record's loads: a converged scene's launches are many
+    const int mark = iter > 0 ? stop_mark(iter, 0) : 0;
+    if (stopped_before(in.stopped, mark)) return;   // before the record's loads: a converged scene's launches are many
     R rot[EPT][9], rin[EPT][NR], kk[EPT][3], em[EPT];
     uint2 lt[EPT], inc[EPT];
 #pragma unroll
@@ -750,7 +751,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
             // the refinement replaced r by the true residual: beta from its r.r and the r.r that
             // built p; the tolerance is relative to the first sweep's |r|
             err = sqrt(total) / in.normb;
-            if (total == 0.0 || err <= in.tol) { record_stop(ins, first, 1, 1, err); go = false; }
+            if (total == 0.0 || err <= in.tol) { record_stop(ins, first, mark, 1, 1, err); go = false; }
             beta = total / in.rho_last;
             if (go && first && threadIdx.x == 0) {
                 ins->rho_slot[1] = total; ins->beta = beta; ins->iter = 1; ins->err = err;
@@ -758,15 +759,15 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
         } else if (iter == 1) {
             const double normb = sqrt(total);
             err = sqrt(total) / normb;
-            if (normb == 0.0) { record_stop(ins, first, 4, 0, 1.0); go = false; }
-            else if (err <= in.tol && !in.first_solve) { record_stop(ins, first, 1, 1, err); go = false; }
+            if (normb == 0.0) { record_stop(ins, first, mark, 4, 0, 1.0); go = false; }
+            else if (err <= in.tol && !in.first_solve) { record_stop(ins, first, mark, 1, 1, err); go = false; }
             if (go && first && threadIdx.x == 0) {
                 ins->normb = normb; ins->rho_slot[1] = total; ins->iter = 1; ins->err = err;
             }
         } else if (iter > 1) {
             err = sqrt(total) / in.normb;
-            if (iter > in.max_iter) { record_stop(ins, first, 0, in.max_iter, in.err); go = false; }
-            else if (err <= in.tol) { record_stop(ins, first, 1, iter, err); go = false; }
+            if (iter > in.max_iter) { record_stop(ins, first, mark, 0, in.max_iter, in.err); go = false; }
+            else if (err <= in.tol) { record_stop(ins, first, mark, 1, iter, err); go = false; }
             beta = total / (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
             if (go && first && threadIdx.x == 0) {
                 ins->rho_slot[iter & 1] = total; ins->beta = beta; ins->iter = iter; ins->err = err;
@@ -1009,26 +1010,27 @@ __global__ __launch_bounds__(TB) void k_tile_exact(TileArgs<R, NR> a, int iter, 
         const int j = threadIdx.x + k * TB;
         if (j <= td.ln_count) lptr[j] = ptr_r[k];
     }
-    if (in.stopped) return;
+    const int mark = iter > 0 ? stop_mark(iter, 0) : 0;
+    if (stopped_before(in.stopped, mark)) return;
     const bool first = (td.flags & kTileFirst) != 0;
     // ---- 3. scalars: rho, the tolerance test, beta (CGLinearSolver.inl:130-196)
     double beta = 0.0;
     if (iter == 1) {
         const double bb = in.dots[kDotBB];
         const double normb = sqrt(bb);
-        if (normb == 0.0) { record_stop(ins, first, 4, 0, 1.0); return; }
+        if (normb == 0.0) { record_stop(ins, first, mark, 4, 0, 1.0); return; }
         // rho = r.r: b.b from a cold start; warmStart: the r.r of r = b - A x
         const double rho = in.warm_start ? in.dots[kDotRR] : bb;
         const double err = sqrt(rho) / normb;
-        if (err <= in.tol && !in.first_solve) { record_stop(ins, first, 1, 1, err); return; }
+        if (err <= in.tol && !in.first_solve) { record_stop(ins, first, mark, 1, 1, err); return; }
         if (first && threadIdx.x == 0) {
             ins->normb = normb; ins->rho_slot[1] = rho; ins->iter = 1; ins->err = err;
         }
     } else if (iter > 1) {
-        if (iter > in.max_iter) { record_stop(ins, first, 0, in.max_iter, in.err); return; }
+        if (iter > in.max_iter) { record_stop(ins, first, mark, 0, in.max_iter, in.err); return; }
         const double rho = in.dots[kDotRR];
         const double err = sqrt(rho) / in.normb;
-        if (err <= in.tol) { record_stop(ins, first, 1, iter, err); return; }
+        if (err <= in.tol) { record_stop(ins, first, mark, 1, iter, err); return; }
         beta = rho / (iter & 1 ? in.rho_slot[0] : in.rho_slot[1]);
         if (first && threadIdx.x == 0) {
             ins->rho_slot[iter & 1] = rho; ins->beta = beta; ins->iter = iter; ins->err = err;
@@ -1382,7 +1384,8 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
     if (zbuf) ld3(zbuf, n, zv);
     ld3(p, n, pv);
     ld3(q, n, qv);
-    if (in.stopped) return;
+    const int mark = stop_mark(iter, 1);
+    if (stopped_before(in.stopped, mark)) return;
     VT m = 0;
     int8_t fx = 0, ct = 0;
     float B[9];
@@ -1406,9 +1409,9 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
     if constexpr (EXACT) den = in.dots[kDotPQ];
     else den = sum_terms<kBlock, true>(pden + rg.t0, rg.nt, part, sh[0]);
     const bool exempt = (iter == 1 && in.first_solve);
-    if (den == 0.0) { record_stop(ins, first, 3, iter, in.err); if (first && t == 0) ins->den = den; return; }
+    if (den == 0.0) { record_stop(ins, first, mark, 3, iter, in.err); if (first && t == 0) ins->den = den; return; }
     if (fabs(den) <= in.thr && !exempt) {
-        record_stop(ins, first, 2, iter, in.err);
+        record_stop(ins, first, mark, 2, iter, in.err);
         if (first && t == 0) ins->den = den;
         return;
     }
