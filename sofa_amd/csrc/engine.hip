@@ -388,6 +388,8 @@ struct InnerCg {
     float* z;                       // with a preconditioner: z = P^-1 r, staged by the operator
     const float *dinv, *binv;       // ... the inverted diagonal (3 per node) / 3x3 blocks (9)
     double *pden, *prho;            // prho: |r|^2 partials per node block (iteration 1 included)
+    bool geo;                       // the operator recomputes the element record
+    const float *x, *x0;            // ... from these positions and rest positions
 };
 void launch_inner_cg(const InnerCg& c, hipStream_t s);
 
@@ -463,6 +465,7 @@ struct EngineT : EngineBase {
     // the float operator's record (FP32, SPLIT, MIXED's inner CG): rest shape and K in float (k_rest_float)
     float *restf = nullptr, *kmatf = nullptr;
     float *rot32 = nullptr, *emass32 = nullptr;    // MIXED: float rotations (per step) and edge masses
+    float *x32 = nullptr, *x0_32 = nullptr;        // MIXED: float positions (per step) and rest positions
     float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *d32 = nullptr, *sp32 = nullptr;
     double *pden32 = nullptr, *prho32 = nullptr, *prr = nullptr;
     InstDev* inst_in = nullptr;
@@ -493,9 +496,11 @@ struct EngineT : EngineBase {
         bool plane = false;             // some scene has a PlaneForceField
         bool pcg = false;               // some scene solves with PCGLinearSolver
         bool warm = false;              // some scene's CGLinearSolver has warmStart
-        hipGraphExec_t gexec = nullptr;
+        bool geo = false;               // the operator recomputes the element record (recomputes())
+        hipGraphExec_t gexec[2] = {};   // the captured step, without and with geo
         ~LaunchSet() {
-            if (gexec) (void)hipGraphExecDestroy(gexec);
+            for (hipGraphExec_t g : gexec)
+                if (g) (void)hipGraphExecDestroy(g);
             for (void* ptr : {a, b, c, o, l, (void*)scenes})
                 if (ptr) (void)hipFree(ptr);
         }
@@ -525,7 +530,7 @@ struct EngineT : EngineBase {
         void* ptrs[] = {x, v, f, b, r, p, q, xcg, mass, fixed, inc_ptr, inc, tet, rot, rest, kmat, ef, ef2,
                         inst, partial, partial2, tiles_d, ranges_d, ltet, ln_gid, ln_inc_ptr, ln_pslot, sh_gid, sh_ptr,
                         ln_inc, sp0, sp1, pbb, pden, prho, p2, em_ptr, em_nbr, em_val, emass, osc_node,
-                        osc_mean, osc_amp, osc_w, osc_phase, restf, kmatf, rot32, emass32, r32, p32, q32,
+                        osc_mean, osc_amp, osc_w, osc_phase, restf, kmatf, rot32, emass32, x32, x0_32, r32, p32, q32,
                         d32, sp32, pden32, prho32, prr, inst_in, sh_of, nd, x0, contact, inc_rank, pinv, zv,
                         inc_arank, sh_acnt, ln_lead, dinv32, binv32, z32};
         for (void* ptr : ptrs)
@@ -1001,7 +1006,7 @@ struct EngineT : EngineBase {
         em_val = nullptr; emass = nullptr; osc_node = nullptr; osc_mean = osc_amp = osc_w = osc_phase = nullptr;
         inst = nullptr; partial = partial2 = nullptr; tiles_d = nullptr; ranges_d = nullptr; ltet = nullptr;
         ln_gid = ln_inc_ptr = ln_pslot = sh_gid = sh_ptr = nullptr; ln_inc = nullptr; sp0 = sp1 = nullptr;
-        pbb = pden = prho = nullptr; restf = kmatf = rot32 = emass32 = nullptr;
+        pbb = pden = prho = nullptr; restf = kmatf = rot32 = emass32 = x32 = x0_32 = nullptr;
         r32 = p32 = q32 = d32 = sp32 = nullptr; pden32 = prho32 = prr = nullptr; inst_in = nullptr; sh_of = nullptr; inc_rank = nullptr;
         pinv = nullptr; zv = nullptr; inc_arank = nullptr; sh_acnt = nullptr; ln_lead = nullptr; dinv32 = nullptr;
         binv32 = z32 = nullptr;
@@ -1049,7 +1054,7 @@ struct EngineT : EngineBase {
         if (mixed) {
             rot32 = dalloc<float>(9 * E);
             emass32 = dalloc<float>(E);
-            for (float** vec : {&r32, &p32, &q32, &d32}) {
+            for (float** vec : {&r32, &p32, &q32, &d32, &x32, &x0_32}) {
                 *vec = dalloc<float>(3 * N);
                 HIPCHK(hipMemset(*vec, 0, 3 * N * sizeof(float)));
             }
@@ -1140,6 +1145,10 @@ struct EngineT : EngineBase {
         put_at(ln_inc, ib0, P.ln_inc);
         if (mixed) {
             put_at(emass32, eb0, th.eh.em_lo);
+            std::vector<float> xf(3 * (size_t)(n + 1), 0.0f);
+            for (int i = 0; i < 3 * n; i++) xf[i] = (float)s.rest[i];
+            put_at(x32, 3 * (int64_t)nb0, xf);
+            put_at(x0_32, 3 * (int64_t)nb0, xf);
         }
         // tiles and their local nodes (each tile's list keeps one extra entry for its end)
         const int T = (int)P.t_ebegin.size();
@@ -1317,7 +1326,11 @@ struct EngineT : EngineBase {
     void prepare_set(const int32_t* ids, int n, hipStream_t s) {
         std::vector<int32_t> want(ids, ids + n);
         auto it = sets.find(want);
-        if (it != sets.end()) { cur = it->second.get(); return; }
+        if (it != sets.end()) {
+            cur = it->second.get();
+            cur->geo = recomputes(cur->na);
+            return;
+        }
         if (sets.size() >= 4096) {       // bounded cache: drop every set (nothing is in flight after the sync)
             HIPCHK(hipDeviceSynchronize());
             sets.clear();
@@ -1377,6 +1390,7 @@ struct EngineT : EngineBase {
         ls->scenes = (int*)sc;
         ls->maxit = maxit;
         ls->n = n;
+        ls->geo = recomputes(ls->na);
         cur = ls.get();
         sets[want] = std::move(ls);
         (void)s;
@@ -1569,9 +1583,7 @@ struct EngineT : EngineBase {
     template <bool WIDE, bool PLANE>
     void launch_apply_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp,
                         const double* pin, double* pd, int pin_nodes) {
-        // (set_apply_variant 1 and 3 on a float engine: the host's rest shape, always read back)
-        const bool geo = ta.rot == rot && !(std::is_same<R, float>::value && (apply_variant & 1)) &&
-                         (int64_t)na * kTileElems * (12 + NR) * (int64_t)sizeof(R) > kRecordCached;
+        const bool geo = recomputing();
         if (variant_threads(apply_variant) == 512) {
             const auto op = geo ? k_tile_apply<R, NR, VT, 512, WIDE, PLANE, true> : k_tile_apply<R, NR, VT, 512, WIDE, PLANE>;
             op<<<na, 512, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0);
@@ -1580,8 +1592,22 @@ struct EngineT : EngineBase {
             op<<<na, 256, 0, s>>>(ta, it, rr, pp, qq, sp, pin, pd, pin_nodes, x, x0);
         }
     }
-    // a launch set's record beyond this does not stay in the last-level cache (k_tile_apply's GEO)
-    static constexpr int64_t kRecordCached = 256 << 20;
+    // whether the CG operator (MIXED: the inner one) recomputes the element record of `tiles` tiles
+    // (k_tile_apply's GEO).  In float, beyond the record that stays in the L2s of the XCDs (8 x 4 MB, the node
+    // vectors beside it): recomputing costs the latency of one more phase, which small sets notice.  In double it
+    // costs more arithmetic than the last-level cache's bandwidth saves, until the record and the vectors outgrow
+    // that (256 MB).  Sets of beams of 82,000 tetrahedra, 25 iterations, ms/step recomputed and read back, by MB of
+    // record: FP32 11 0.328 and 0.332, 23 0.394 and 0.412, 45 0.56 and 0.62, 107 1.08 and 1.09, 141 1.34 and 1.32,
+    // 174 1.66 and 1.73, 253 2.28 and 2.92; SPLIT 11 0.382 and 0.381, 23 0.456 and 0.486, 174 2.00 and 2.47; MIXED
+    // 11 0.387 and 0.386, 23 0.446 and 0.468, 174 1.92 and 2.04; FP64 26 0.49 and 0.47, 92 1.00 and 0.98, 131 1.27
+    // and 1.28, 158 1.43 and 1.47, 249 2.09 and 2.56.
+    static constexpr int64_t kRecordFloat = 16ll << 20, kRecordDouble = 144ll << 20;
+    bool recomputes(int64_t tiles) const {
+        const int64_t record = mixed ? 18 * (int64_t)sizeof(float) : (12 + NR) * (int64_t)sizeof(R);
+        return tiled && tiles * kTileElems * record > (mixed || std::is_same<R, float>::value ? kRecordFloat : kRecordDouble);
+    }
+    // ... in the current launch set (set_apply_variant 1 and 3 on a float engine: the host's rest shape, read back)
+    bool recomputing() const { return cur->geo && !(std::is_same<R, float>::value && (apply_variant & 1)); }
     template <bool PLANE>
     void launch_exact_t(int na, hipStream_t s, const TileArgs<R, NR>& ta, int it, const VT* rr, VT* pp, VT* qq, VT* sp) {
         switch (apply_variant) {
@@ -1608,7 +1634,8 @@ struct EngineT : EngineBase {
         int best = 0;
         float best_us = 0;
         for (int v = 0; v < kApplyVariants; v++) {
-            if (!exact_tiled() && (v & 1)) {   // the kernel of v - 1 on another rest shape
+            // outside the reference order v is the kernel of v - 1 on another rest shape, if that one reads it back
+            if (!exact_tiled() && (v & 1) && !(std::is_same<R, float>::value && cur->geo)) {
                 if (us_out) us_out[v] = us_out[v - 1];
                 continue;
             }
@@ -1653,12 +1680,12 @@ struct EngineT : EngineBase {
         ta.emass = emass;
         ta.nd = nd;
         ta.rot = rot;
-        ta.rot_row = Etot;
         ta.rest = rest;
         ta.kmat = kmat;
         if constexpr (std::is_same<R, float>::value)
             if (!(apply_variant & 1)) { ta.rest = restf; ta.kmat = kmatf; }
         ta.rot32 = rot32;
+        ta.x32 = x32;
         return ta;
     }
 
@@ -1704,13 +1731,15 @@ struct EngineT : EngineBase {
         ic.ta.contact = contact;
         ic.ta.emass = emass32;
         ic.ta.nd = nullptr;
-        ic.ta.rot = rot32; ic.ta.rot_row = Etot; ic.ta.rest = restf; ic.ta.kmat = kmatf;
-        ic.ta.rot32 = nullptr;
+        ic.ta.rot = rot32; ic.ta.rest = restf; ic.ta.kmat = kmatf;
+        ic.ta.rot32 = nullptr; ic.ta.x32 = nullptr;
         // PCGLinearSolver with a Jacobi preconditioner: the inner CG runs preconditioned (in the node
         // kernels: the operator reads z)
         ic.z = cur->pcg ? z32 : nullptr;
         ic.dinv = dinv32;
         ic.binv = binv32;
+        ic.geo = cur->geo;
+        ic.x = x32; ic.x0 = x0_32;
         ic.fb = fb; ic.nb = nb;
         ic.na = cur->na; ic.nfb = cur->nb; ic.nnb = cur->nc; ic.maxit = cur->maxit;
         ic.wide = cur->maxpart > kWavePartials;
@@ -1749,10 +1778,11 @@ struct EngineT : EngineBase {
 
     void reset_graph() override {
         for (auto& kv : sets)
-            if (kv.second->gexec) {
-                (void)hipGraphExecDestroy(kv.second->gexec);
-                kv.second->gexec = nullptr;
-            }
+            for (hipGraphExec_t& g : kv.second->gexec)
+                if (g) {
+                    (void)hipGraphExecDestroy(g);
+                    g = nullptr;
+                }
     }
 
     // a merged step in concurrent branches: the scenes are split into G groups, each stepped by its
@@ -1798,13 +1828,16 @@ struct EngineT : EngineBase {
         }
         // a copy: step_set may empty the plan cache (prepare_set's bounded cache of launch sets)
         const std::vector<std::vector<int32_t>> groups = it->second;
+        int64_t tiles = 0;   // the branches run side by side: the cache holds the records of all
+        if (tiled)
+            for (int k = 0; k < n; k++) tiles += (int64_t)place[ids[k]].tiles.size();
         if (branch_turns && exact_tiled()) { step_turns(groups, nsteps, s, G); return; }
         for (int st = 0; st < nsteps; st++) {
             HIPCHK(hipEventRecord(fork_ev, s));
             for (int g = 1; g < G; g++) HIPCHK(hipStreamWaitEvent(aux[g - 1], fork_ev, 0));
             for (int g = 0; g < G; g++) {
                 const std::vector<int32_t>& grp = groups[g];
-                step_set(grp.data(), (int)grp.size(), 1, g == 0 ? s : aux[g - 1]);
+                step_set(grp.data(), (int)grp.size(), 1, g == 0 ? s : aux[g - 1], tiles);
             }
             for (int g = 1; g < G; g++) {
                 HIPCHK(hipEventRecord(join_ev[g - 1], aux[g - 1]));
@@ -1878,9 +1911,11 @@ struct EngineT : EngineBase {
         else step_set(ids, n, nsteps, s);
     }
 
-    // `nsteps` steps of one launch set (the listed scenes in one launch per phase) on `s`
-    void step_set(const int32_t* ids, int n, int nsteps, hipStream_t s) {
+    // `nsteps` steps of one launch set (the listed scenes in one launch per phase) on `s`, with `tiles` of
+    // them and of the sets beside it (0: it runs alone)
+    void step_set(const int32_t* ids, int n, int nsteps, hipStream_t s, int64_t tiles = 0) {
         prepare_set(ids, n, s);
+        if (tiles > 0) cur->geo = recomputes(tiles);
         if (!use_graphs) {
             for (int st = 0; st < nsteps; st++) launch_step(n, s);
             HIPCHK(hipGetLastError());
@@ -1888,7 +1923,7 @@ struct EngineT : EngineBase {
         }
         // the whole step (RHS, every CG iteration, update) is captured once per launch set and
         // replayed: one graph launch per step instead of 3 n_cg + 5 kernel launches
-        hipGraphExec_t& gexec = cur->gexec;
+        hipGraphExec_t& gexec = cur->gexec[cur->geo];
         if (!gexec && nsteps > 0) {
             hipGraph_t graph = nullptr;
             HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -2157,18 +2192,25 @@ struct EngineT : EngineBase {
             iterate_exact(ev, na, 1, s, nullptr, nullptr);
             k_finalize<false><<<1, kBlock, 0, s>>>(cur->scenes, inst, partial, exact_ready());
         } else {
-            TileArgs<R, NR> ta = tile_args();
+            const TileArgs<R, NR> ta = tile_args();
             const int64_t nE = (int64_t)scenes[scene].tets.size() / 4, e0 = elem_begin(scene);
             bool exact = false;
             if constexpr (std::is_same<R, double>::value) exact = exact_tiled();
-            if (!exact && nE > 0) {
-                // the rotations of the engine's positions (ev.rot keeps addForce's), in the scene's own share of
-                // the force calls' scratch (12 VT per element, from 12 e0): another scene's force call may be
-                // using its share on another stream.  Rows of nE; element e is at e - e0 of a row.
-                R* const rot_cg = reinterpret_cast<R*>(ef + 12 * e0) - e0;
-                k_rotations<R, VT><<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, s>>>(tet, e0, e0 + nE, x, rot_cg, nE);
-                ta.rot = rot_cg;
-                ta.rot_row = nE;
+            // the rotations are those of the engine's positions: the operator recomputes them with the rest of the
+            // record; where it may not (set_apply_variant 1 and 3 on a float engine) they take the place of
+            // addForce's, which wait in the scene's own share of the force calls' scratch
+            cur->geo = true;
+            const bool swap = !exact && nE > 0 && !recomputing();
+            R* const kept = reinterpret_cast<R*>(ef + 12 * e0);
+            const auto move = [&](bool back) {
+                for (int k = 0; k < 9; k++) {
+                    R *row = rot + k * Etot + e0, *to = kept + k * nE;
+                    HIPCHK(hipMemcpyAsync(back ? row : to, back ? to : row, nE * sizeof(R), hipMemcpyDeviceToDevice, s));
+                }
+            };
+            if (swap) {
+                move(false);
+                k_rotations<R, VT><<<(unsigned)((nE + kBlock - 1) / kBlock), kBlock, 0, s>>>(tet, e0, e0 + nE, x, rot, Etot);
             }
             const FinBlk* fb = (const FinBlk*)cur->b;
             const NodeBlk* nbk = (const NodeBlk*)cur->c;
@@ -2200,6 +2242,7 @@ struct EngineT : EngineBase {
                 }
             }
             k_solve_end<<<1, 64, 0, s>>>(cur->scenes, 1, inst);
+            if (swap) move(true);
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(xvec, xcg + 3 * (int64_t)nb0, 3 * (size_t)n * sizeof(VT), hipMemcpyDeviceToDevice, s));
@@ -2407,15 +2450,19 @@ EngineBase* make_engine_split() {
     return e;
 }
 
+template <bool GEO>
+static auto inner_operator(const InnerCg& c) {
+    return c.wide ? (c.plane ? k_tile_apply<float, 6, float, kTileThreads, true, true, GEO>
+                             : k_tile_apply<float, 6, float, kTileThreads, true, false, GEO>)
+                  : (c.plane ? k_tile_apply<float, 6, float, kTileThreads, false, true, GEO>
+                             : k_tile_apply<float, 6, float, kTileThreads, false, false, GEO>);
+}
 void launch_inner_cg(const InnerCg& c, hipStream_t s) {
     const float* rs = c.z ? c.z : c.r;   // the vector p is formed from (p = rs + beta p)
     for (int it = 1; it <= c.maxit; it++) {
         if (c.na > 0) {
-            const auto op = c.wide ? (c.plane ? k_tile_apply<float, 6, float, kTileThreads, true, true>
-                                              : k_tile_apply<float, 6, float, kTileThreads, true, false>)
-                                   : (c.plane ? k_tile_apply<float, 6, float, kTileThreads, false, true>
-                                              : k_tile_apply<float, 6, float, kTileThreads, false, false>);
-            op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, nullptr, nullptr);
+            const auto op = c.geo ? inner_operator<true>(c) : inner_operator<false>(c);
+            op<<<c.na, kTileThreads, 0, s>>>(c.ta, it, rs, c.p, c.q, c.sp, c.prho, c.pden, 1, c.x, c.x0);
         }
         if (c.nnb > 0)
             k_update<float><<<c.nnb, kUpdateThreads, 0, s>>>(c.nb, c.ta.inst, c.ta.ranges, it, c.sn, c.sp, c.ta.mass, c.ta.fixed,

@@ -267,8 +267,7 @@ struct TileArgs {
     double* __restrict__ nd;            // reference order: per-node dot terms
     // the operator's element record, SoA: rotations (written by the step's force pass), rest shape, K
     const R *rot, *rest, *kmat;
-    int64_t rot_row;                    // length of a row of rot (rest and kmat: ev.E)
-    float* rot32;                       // MIXED: the inner operator's rotations, written by the force pass
+    float *rot32, *x32;                 // MIXED: the inner operator's rotations and positions, written by the force pass
 };
 
 // consistent-mass edge terms of one element, folded into its nodal contributions (which the
@@ -447,6 +446,10 @@ __global__ __launch_bounds__(TB) void k_tile_rhs(TileArgs<R, NR> a, const VT* __
         const int j = threadIdx.x + m * TB;
         if (j < td.ln_count) {
             lx[3 * j] = (R)xt[m][0]; lx[3 * j + 1] = (R)xt[m][1]; lx[3 * j + 2] = (R)xt[m][2];
+            if (a.x32) {   // every tile of a shared node writes the same value
+                const float xf[3] = {(float)xt[m][0], (float)xt[m][1], (float)xt[m][2]};
+                st3(a.x32, gid[m], xf);
+            }
             lv[3 * j] = (R)vt[m][0]; lv[3 * j + 1] = (R)vt[m][1]; lv[3 * j + 2] = (R)vt[m][2];
         }
     }
@@ -638,19 +641,21 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
 //   2. by the waves that have nodes: the scalars (rho, the tolerance test, beta), then p = r + beta p and
 //      what the node sums need of each node, staged in LDS;
 //   3. each element's contributions into LDS, 12 rows of kTileRow;
-//   4. a thread per (node, component): the contributions in ascending element id;
+//   4. a thread per (node, component), GEO: per node: the contributions in ascending element id;
 //   5. by the waves that have nodes: interior nodes finished (q), a shared node's sum left as the tile's
 //      partial, p.q as one partial per tile.
 // The element's rotation, rest shape and K are read back (18 floats, 21 doubles), not recomputed from the
-// positions: 460 instead of 610 vector instructions per wave in float.  What bounds it: on a large mesh
-// VALU issue (half of the time), LDS (a third) and the latency of the phases of the four tiles that a CU
-// holds (FP64: two, by registers and LDS); on a small one that latency alone.  Measured, before (geometry
-// recomputed, a thread per node for staging and sums) and after: FP32 1.31M tetrahedra 32.2 -> 29.9 us, 24
-// beams of 0.6M 24.9 -> 22.6, 18,954 7.2 -> 6.6; SPLIT 150k 11.1 -> 10.2; FP64 360k 24.9 -> 22.8.
-// GEO: the record recomputed from the positions all the same (same bits), for launch sets whose record does
-// not stay in the 256 MB last-level cache from one iteration to the next.  256 beams of 8.9M tetrahedra, recomputed
-// and read back: FP32 5.9 and 6.8 ms/step, SPLIT 7.7 and 9.2, FP64 12.0 and 13.9; the operator
-// of 1.31M tetrahedra in float (94 MB of record) 33.4 and 29.7 us, of 0.6M 25.6 and 22.7, of 360k in double 23.6 and 22.4.
+// positions: 460 instead of 610 vector instructions per wave in float, and a phase less.  GEO: recomputed from
+// the positions x, x0 all the same (same bits), for sets whose record does not stay cached from one iteration to
+// the next (EngineT::recomputes has the line), the sums then by the threads that have a node's p in registers, which
+// takes back the phase and its LDS traffic.  What bounds it: on a large mesh VALU issue (half of the time), LDS (a
+// third) and the latency of the phases of the four tiles that a CU holds (FP64: two, by registers and LDS); on a
+// small one that latency alone.  Measured, launches one after the other, with all recomputed and a thread per node for
+// staging and sums, read back, and GEO: FP32 18,954 tetrahedra 8.2, 7.3, 7.5 us, 101,250 8.4, 7.6, 7.8, 1.31M 33.4, 29.2,
+// 28.7; SPLIT 150k 12.1, 10.0, 10.6; FP64 360k 28.8, 22.4, 22.7; 256 beams of 8.9M FP32 169, 199, 156, SPLIT 211, 246,
+// 184, FP64 379, 427, 346.  (Between the launches of a step the update passes over the vectors: the line is the step's.)
+// The step of those 256 beams, ms, read back, GEO with the sums by component, and GEO: FP32 6.77, 5.95, 5.57; SPLIT 9.2,
+// 7.68, 7.44; MIXED 25.3, 22.3, 20.9.
 // PLANE = false: no scene of the launch has a PlaneForceField; WIDE = false: no scene has more than
 // kWavePartials partials of r.r, which are then in flight with the gathers.
 constexpr int kNodeMass = 1 << 12;   // the node's sum starts from the mass term
@@ -711,7 +716,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
             inc[m] = reinterpret_cast<const uint2*>(a.tn.inc + td.inc_begin)[k];   // four incidences
             if (!GEO) {
 #pragma unroll
-                for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.rot_row + td.e_begin))[k];
+                for (int i = 0; i < 9; i++) rot[m][i] = (a.rot + (i * a.ev.E + td.e_begin))[k];
 #pragma unroll
                 for (int i = 0; i < NR; i++) rin[m][i] = (a.rest + (i * a.ev.E + td.e_begin))[k];
             }
@@ -791,7 +796,7 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
                         lu[3 * j + i] = pv[m][i];
                         if (GEO) { lc[3 * j + i] = (R)xt[m][i]; lc[3 * kTileNodes + 3 * j + i] = (R)x0t[m][i]; }
                     }
-                    lmass[j] = ms[m];
+                    if (!GEO) lmass[j] = ms[m];
                     lnode[j] = (uint16_t)(s0[m] | (in.m_cg != 0.0 && interior ? kNodeMass : 0));
                 }
             }
@@ -843,25 +848,38 @@ __global__ __launch_bounds__(TB) void k_tile_apply(TileArgs<R, NR> a, int iter, 
     }
     __syncthreads();
     // ---- 4. per-node sums in ascending element id, from LDS only
-    const int n3 = 3 * td.ln_count;
+    if constexpr (!GEO) {
+        const int n3 = 3 * td.ln_count;
 #pragma unroll 1
-    for (int j = threadIdx.x; j < n3; j += TB) {
-        const int n = j / 3, c = j - 3 * n;
-        const int nf = lnode[n], i0 = nf & (kNodeMass - 1);
-        const int i1 = n + 1 < td.ln_count ? (int)(lnode[n + 1] & (kNodeMass - 1)) : ninc;
-        VT acc = 0;
-        if (nf & kNodeMass) mass_term(in, lmass[n], in.m_cg, lu[j], acc);
-        sum_component(linc, i0, i1, lc + c * kTileRow, acc);
-        lu[j] = acc;
+        for (int j = threadIdx.x; j < n3; j += TB) {
+            const int n = j / 3, c = j - 3 * n;
+            const int nf = lnode[n], i0 = nf & (kNodeMass - 1);
+            const int i1 = n + 1 < td.ln_count ? (int)(lnode[n + 1] & (kNodeMass - 1)) : ninc;
+            VT acc = 0;
+            if (nf & kNodeMass) mass_term(in, lmass[n], in.m_cg, lu[j], acc);
+            sum_component(linc, i0, i1, lc + c * kTileRow, acc);
+            lu[j] = acc;
+        }
+        __syncthreads();
     }
-    __syncthreads();
     // ---- 5. the nodes' results
     double pq = 0.0;
 #pragma unroll
     for (int m = 0; m < NPT; m++) {
         const int j = threadIdx.x + m * TB;
         if (w0 + m * TB < td.ln_count && j < td.ln_count) {
-            VT qn[3] = {lu[3 * j], lu[3 * j + 1], lu[3 * j + 2]};
+            VT qn[3] = {0, 0, 0};
+            if constexpr (GEO) {
+                const int i1 = j + 1 < td.ln_count ? (int)(lnode[j + 1] & (kNodeMass - 1)) : ninc;
+                if (in.m_cg != 0.0 && psl[m] < 0) {
+#pragma unroll
+                    for (int i = 0; i < 3; i++) mass_term(in, ms[m], in.m_cg, pv[m][i], qn[i]);
+                }
+                sum_incidences<true>(linc, s0[m], i1, lc, qn);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 3; i++) qn[i] = lu[3 * j + i];
+            }
             if (psl[m] < 0) {
                 if (PLANE && ct[m]) plane_dforce(in, in.k_cg, pv[m], qn);
                 if (fx[m]) { qn[0] = 0; qn[1] = 0; qn[2] = 0; }
@@ -1173,7 +1191,7 @@ static __global__ __launch_bounds__(kBlock) void k_rest_float(const int4* __rest
 // follow a force pass (component-level CG)
 template <typename R, typename VT>
 __global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ tet, int64_t e0, int64_t e1,
-                                                       const VT* __restrict__ x, R* __restrict__ rot, int64_t row) {
+                                                       const VT* __restrict__ x, R* __restrict__ rot, int64_t E) {
     const int64_t e = e0 + (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (e >= e1) return;
     const int4 t = tet[e];
@@ -1185,7 +1203,7 @@ __global__ __launch_bounds__(kBlock) void k_rotations(const int4* __restrict__ t
         for (int i = 0; i < 3; i++) p[n][i] = (R)x[3 * (int64_t)v[n] + i];
     rotation_large(p[0], p[1], p[2], ro);
 #pragma unroll
-    for (int i = 0; i < 9; i++) rot[i * row + e] = ro[i];
+    for (int i = 0; i < 9; i++) rot[i * E + e] = ro[i];
 }
 
 // reference order, after the tile apply: the shared nodes' p = r + beta p, q = (1 + h rm) M p

@@ -43,8 +43,8 @@ def footprint_bytes(precision, nodes, tets, reference_order=False, scenes=1):
     if precision in (capi.FP32, capi.SPLIT, capi.MIXED):
         per_tet += (6 + 3) * 4                 # the operator's rest shape and K in float
     if precision == capi.MIXED:
-        # float r, p, q, d and shared partials; float rotations and edge masses
-        per_node += 4 * 3 * 4 + 3 * 4
+        # float r, p, q, d, x, x0 and shared partials; float rotations and edge masses
+        per_node += 6 * 3 * 4 + 3 * 4
         per_tet += (9 + 1) * 4
     per_scene = 0
     if reference_order:

@@ -172,8 +172,8 @@ def test_cg_solve_keeps_the_force_calls_rotations(prec):
 
 
 @pytest.mark.parametrize("first", [0, 1])
-@pytest.mark.parametrize("prec", ["FP64_TILED", "FP32", "SPLIT"])
-def test_cg_solve_beside_force_calls(prec, first):
+@pytest.mark.parametrize("prec,variant", [("FP64_TILED", 0), ("FP32", 0), ("FP32", 1), ("SPLIT", 0), ("SPLIT", 3)])
+def test_cg_solve_beside_force_calls(prec, variant, first):
     """cg_solve of one scene on one stream while force calls of another scene of the same engine are in flight on
     a second stream: scenes share no buffer, so each has the bits that it has alone."""
     from sofa_amd import workloads
@@ -185,6 +185,7 @@ def test_cg_solve_beside_force_calls(prec, first):
     for s in specs:
         workloads.add_to_engine(eng, s)
     eng.commit()
+    eng.set_apply_variant(variant)
     a, b = first, 1 - first
     rng = np.random.default_rng(5)
     dev = lambda v: capi.DeviceArray(np.ascontiguousarray(v, dtype=dt))
@@ -209,3 +210,64 @@ def test_cg_solve_beside_force_calls(prec, first):
     eng.close()
     assert np.any(got[0][0]) and np.any(got[0][1])
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("branches", [1, 4])
+@pytest.mark.parametrize("prec", ["FP32", "SPLIT", "MIXED"])
+def test_record_line(prec, branches):
+    """A set of scenes whose element records exceed 16 MB together, in one launch sequence and in branches that each
+    stay below (the operator recomputes the records), against each scene alone (it reads them back): the same
+    bits, scenes of one material and of a material per element, with and without a plane."""
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: record line {prec} {branches} branches", flush=True)
+    specs = [_spec((9, 9, 33), k) for k in ("one", "materials", "plane")]
+    out = []
+    for together in (True, False):
+        eng = capi.Engine(0, getattr(capi, prec))
+        ids = [workloads.add_to_engine(eng, specs[k % 3]) for k in range(30)]
+        eng.commit()
+        eng.set_graphs(True)
+        eng.set_branches(branches)
+        mb = [eng.tiling(i)["tiles"] * 512 * 72 / 2 ** 20 for i in ids]
+        assert sum(mb) > 16 > 2 * max(mb) and (branches == 1 or sum(mb) / branches < 10)
+        for group in ([ids] if together else [[i] for i in ids[:3]]):
+            eng.step(group, 2)
+        out.append([eng.read(i)[:2] for i in ids[:3]])
+        eng.close()
+    for (x, v), (xs, vs) in zip(*out):
+        assert np.any(v) and np.array_equal(x, xs) and np.array_equal(v, vs)
+
+
+@pytest.mark.parametrize("prec,variant,n,bar", [("FP32", 0, (9, 9, 33), 1e-4), ("FP32", 1, (9, 9, 33), 1e-4),
+                                                ("FP32", 2, (33, 33, 65), 1e-4), ("FP32", 3, (33, 33, 65), 1e-4),
+                                                ("SPLIT", 0, (33, 33, 65), 1e-4), ("SPLIT", 1, (9, 9, 33), 1e-4),
+                                                ("FP64_TILED", 0, (9, 9, 33), 1e-10), ("FP64_TILED", 1, (41, 41, 129), 1e-10)])
+def test_cg_solve_rotations(prec, variant, n, bar):
+    """cg_solve on positions turned by one radian (the rotations of the last step are those of the rest positions), in
+    scenes of few and many records and every operator variant, against the untiled FP64 engine.  Bars: a few ulp of the vectors per
+    operation (1e-16 double, 1e-7 float), times the 10 iterations, times 100 for what CG makes of them."""
+    from sofa_amd import workloads
+    capi = _capi()
+    print(f"case: cg_solve on turned positions {prec} {variant} {n}", flush=True)
+    spec = _spec(n, "one")
+    c, s = np.cos(1.0), np.sin(1.0)
+    x = spec["pos"] @ np.array([[c, s, 0.0], [-s, c, 0.0], [0.0, 0.0, 1.0]])
+    rhs = np.random.default_rng(3).standard_normal(x.shape)
+    got = []
+    for p in ("FP64", prec):
+        dt = np.float32 if p == "FP32" else np.float64
+        eng = capi.Engine(0, getattr(capi, p))
+        sid = workloads.add_to_engine(eng, spec)
+        eng.commit()
+        if p != "FP64":
+            eng.set_apply_variant(variant)
+        eng.write(sid, x)
+        dev = lambda a: capi.DeviceArray(np.ascontiguousarray(a, dtype=dt))
+        xd, f, b, sol = dev(x), dev(np.zeros(x.shape)), dev(rhs), dev(np.zeros(x.shape))
+        if p == "FP64":        # the untiled engine's rotations are the last force call's
+            eng.fem_add_force(sid, xd.ptr, f.ptr)
+        eng.cg_solve(sid, 1.0, 0.0, -1e-3, b.ptr, sol.ptr)
+        got.append(sol.numpy().astype(np.float64))
+        eng.close()
+    assert np.linalg.norm(got[1] - got[0]) <= bar * np.linalg.norm(got[0])
