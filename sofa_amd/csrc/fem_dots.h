@@ -15,15 +15,18 @@
 // sums, so a binade to round to, and form its M and A.  A fifth wave walks the previous round's 64
 // pieces from the exact sum so far, all at once by a prefix scan up to the first whose condition
 // fails (another binade than guessed, a crossing, a tie, a term of the sum's own size), which it
-// takes by 64 dependent adds.  The binades of a growing sum are crossed about log2(n) times, mostly
-// within the first pieces; about 18 pieces of a sum fail (emulated on beams of 2,500 to 41,000
-// nodes, both dot products of CG).
+// takes by dependent adds, with the ones right behind it that look as if they failed too (a piece that
+// would keep the rule has the same sum either way).  The binades of a growing sum are crossed about log2(n)
+// times, mostly within the first pieces; about 18 pieces of a sum fail (emulated on beams of 2,500 to 41,000
+// nodes, both dot products of CG).  Of a sum whose terms change sign most pieces fail: it is the chain.
 //
 // What bounds it: one CU's latency.  A round takes 2,200 cycles (0.9 us: 470 to issue its loads, 280 to
-// stage them, 970 + 490 of arithmetic at one wave per SIMD; the walk, 1,050, runs beside it), a
-// failing piece 1,500.  Rounds are of 4,096 terms because three of them fit the LDS beside one
-// operator tile.  Measured alone on n squared normal deviates: 7.7 us for 8,192, 14.0 for 32,768, 72.7
-// for 262,144; the chain takes 3.7 ns a term (30, 121, 970).  In the step of 16 beams of 500 to
+// stage them, 970 + 490 of arithmetic at one wave per SIMD; the walk, 1,050, runs beside it), the chain
+// 3.7 ns a term.  Its three rounds of 4,096 terms fill 113 KB of LDS: no tile of the operator fits beside it
+// (68 KB in double), so with branches it waits for a CU that another branch's operator leaves free.
+// Measured, calls of vDot in a row, n = 512, 1,000, 4,096, 8,100, 21,825, 56,889 nodes: squares 6.7, 7.1, 7.9, 11.0, 18.6, 35.5
+// us (the chain alone 6.7, 7.7, 27.7, 54, 146, 371); products of either sign 6.7, 8.7, 19.9, 38, 96, 168, with the failing
+// pieces one by one 8.0, 11.5, 31.9, 62, 158, 238 (the chain alone as above).  In the step of 16 beams of 500 to
 // 42,000 nodes a dot product went from 45.6 us (the chain in 8 segments run at once from candidate
 // starts, four launches) to 16-23 in one, the step from 5.2 to 3.6 ms.
 #pragma once
@@ -40,7 +43,7 @@ constexpr int kScanRound = 64 * kScanWaves * kScanPer;
 constexpr int kScanResult = 64 * kScanWaves;     // the thread that has the sum
 // a term's place in LDS: two doubles of padding behind each lane's own, so that the lanes' reads
 // of their own terms spread over the banks
-__device__ __forceinline__ int scan_at(int i) { return i + 2 * (i / kScanPer); }
+__device__ __forceinline__ constexpr int scan_at(int i) { return i + 2 * (i / kScanPer); }
 
 static_assert(kScanWaves == 4 && kScanLanes == 4 && kScanRound == 64 * 64, "quads of lanes, 64 pieces a round");
 
@@ -142,6 +145,13 @@ __device__ __forceinline__ void scan_load(Terms term, int base, int own, int n, 
     }
 }
 
+// the h-th 32 terms of a round
+__device__ __forceinline__ void scan_half(const double* buf, int h, double q[32]) {
+    const double* c = buf + scan_at(32) * h;
+#pragma unroll
+    for (int i = 0; i < 32; i++) q[i] = c[scan_at(i)];
+}
+
 // 0.0 + term(0) + term(1) + ... + term(n - 1), n >= 1, every add rounded in that order; all
 // kScanThreads threads of the workgroup call it, thread kScanResult has the result
 template <typename Terms>
@@ -233,15 +243,23 @@ __device__ __forceinline__ double scan_sum(Terms term, int n) {
                     s = lane_value(at + m, 63);
                     break;
                 }
+                // the failing piece and the next ones that may fail too (as far as their approximate starts tell):
+                // the chain, half a piece of terms on its way while the half before is added
                 const int f = __builtin_ctzll(fails);
+                const unsigned long long keep = ~(fails >> f);
+                const int end = keep ? f + __builtin_ctzll(keep) : 64;
                 s = lane_value(at, f);
-                const double* c = c0 + scan_at(f * 64);
-                double q[64];
+                double q0[32], q1[32];
+                scan_half(c0, 2 * f, q0);
+                for (int h = 2 * f; h < 2 * end; h += 2) {
+                    scan_half(c0, h + 1, q1);
 #pragma unroll
-                for (int i = 0; i < 64; i++) q[i] = c[scan_at(i)];
+                    for (int i = 0; i < 32; i++) s = s + q0[i];
+                    scan_half(c0, min(h + 2, 127), q0);
 #pragma unroll
-                for (int i = 0; i < 64; i++) s = s + q[i];
-                g = f + 1;
+                    for (int i = 0; i < 32; i++) s = s + q1[i];
+                }
+                g = end;
             }
         }
         __syncthreads();
