@@ -409,11 +409,8 @@ struct EngineT : EngineBase {
     int4* tet = nullptr;
     R *rot = nullptr, *rest = nullptr, *kmat = nullptr;
     // read-back: two halves of pinned memory, made at commit, a half as large as the largest scene's state
-    // but at most kStageMost.  The host's first read of such memory costs 1.5 us a page, so a new engine's first read pays
-    // for all that it passes through; each chunk costs 14 us, so small halves slow every later one.  First and later reads,
-    // us, with halves of 256 KiB, 512 KiB and 2 MiB: 21,825 nodes in double 361 and 152, 563 and 110, 784 and 123; 56,889 592
-    // and 350, 737 and 295, 1,919 and 320; 279,873 in float 1,421 and 1,100, 1,797 and 1,080, 3,095 and 1,020.
-    static constexpr int64_t kStageMost = 512 << 10;
+    // but at most kStageMost (8 MiB of it took 250 us to make, as much as a small scene's whole set-up)
+    static constexpr int64_t kStageMost = 2 << 20;
     int64_t stage_half = 0;
     char* stage = nullptr;
     hipEvent_t stage_ev[2] = {};
