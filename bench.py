@@ -33,9 +33,9 @@ import numpy as np
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
-# hardware queues of this process (read by HIP when the library initialises it): 8, so that the
-# reference-order engine's concurrent branches get queues of their own (HIP's default is 4, two
-# of which its own streams hold)
+# hardware queues of this process (read by HIP when the library initialises it): 8, so that
+# concurrent branches (--branches) get queues of their own (HIP's default is 4, two of which its own
+# streams hold)
 if int(os.environ.get("GPU_MAX_HW_QUEUES", "4")) < 8:
     os.environ["GPU_MAX_HW_QUEUES"] = "8"
 

@@ -257,9 +257,9 @@ int sofa_amd_engine_set_graphs(sofa_amd_engine eng, int enable);
  * (largest node counts dealt round-robin), each advanced by its own launch sequence on its own
  * stream, forked from and joined back into the step's stream, so that one group's latency-bound
  * phases overlap the others' kernels.  0 (default): on FP64_TILED engines in the reference's
- * summation order, whose node-after-node dot products are single-wave chains, one branch per
+ * summation order, whose node-after-node dot products are one workgroup per scene, one branch per
  * hardware queue the runtime leaves free (HIP's GPU_MAX_HW_QUEUES, 4 unless set, minus the two
- * its own streams hold), at most 4; else 1.  At most 8, and at most one branch per two scenes.
+ * its own streams hold), at most 2; else 1.  At most 8, and at most one branch per two scenes.
  * Branches only run concurrently on distinct hardware queues.  Results do not depend on it (scenes are
  * independent).  No reference counterpart. */
 int sofa_amd_engine_set_branches(sofa_amd_engine eng, int branches);
@@ -267,12 +267,12 @@ int sofa_amd_engine_set_branches(sofa_amd_engine eng, int branches);
 /* FP64_TILED engines in the reference's summation order, stepped in more than one branch: 1
  * makes the branches' operator phases take turns: in every CG iteration each group's
  * operator and finalize kernels wait for the previous group's (round-robin), so that one group's
- * two node-after-node dot products (single-wave chains) run while the GPU runs another group's
- * operator alone, instead of every group's operator at once and then every group's chains on an
- * idle GPU.  Such steps are launched directly, without graphs (a graph per branch cannot wait
+ * two node-after-node dot products (one workgroup per scene) run while the GPU runs another
+ * group's operator alone, instead of every group's operator at once and then every group's dot
+ * products on an idle GPU.  Such steps are launched directly, without graphs (a graph per branch cannot wait
  * for another branch's kernels).  0 (default): the branches run freely, each replayed from its own
- * graph when graphs are on (measured faster on the 256-beam mix: 21.6 against 22.3 ms/step with
- * 4 branches).  Results do not depend on it.  No reference counterpart. */
+ * graph when graphs are on (measured faster on the 256-beam mix: 17.4 against 18.5 ms/step with
+ * 2 branches).  Results do not depend on it.  No reference counterpart. */
 int sofa_amd_engine_set_branch_turns(sofa_amd_engine eng, int enable);
 
 /* FP64_TILED engines in the reference's summation order (set before the scenes are placed): how

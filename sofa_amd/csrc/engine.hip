@@ -1787,22 +1787,22 @@ struct EngineT : EngineBase {
 
     // a merged step in concurrent branches: the scenes are split into G groups, each stepped by its
     // own launch sequence on its own stream (forked from and joined back into `s` by events), so
-    // that one group's latency-bound phases (the reference order's node-after-node dot products:
-    // one wave per scene, one dependent add per node) overlap the other groups' element and node
-    // kernels.  Scenes are dealt to the groups by node count, largest first, round-robin: each
-    // group holds one of the G longest dot-product chains and about 1/G of the work.
+    // that one group's latency-bound phases (the reference order's node-after-node dot products: one
+    // workgroup per scene) overlap the other groups' element and node kernels.  Scenes are dealt to the
+    // groups by node count, largest first, round-robin: each group holds one of the G longest dot
+    // products and about 1/G of the work.
     static constexpr int kMaxBranches = 8;
     std::map<std::vector<int32_t>, std::vector<std::vector<int32_t>>> branch_plans;
     hipStream_t aux[kMaxBranches - 1] = {};
     hipEvent_t fork_ev = nullptr, join_ev[kMaxBranches - 1] = {};
     // the default: one branch per hardware queue the runtime's own streams leave free (HIP gives a
-    // process GPU_MAX_HW_QUEUES of them, 4 unless set; two are taken), at most 4 (measured on the
-    // 256-beam mix with 8 queues: 1 branch 30.6 ms/step, 2 26.0, 3 24.0, 4 23.7); branches sharing
-    // a queue run one after the other
+    // process GPU_MAX_HW_QUEUES of them, 4 unless set; two are taken), at most 2.  Measured with 8 queues,
+    // 1, 2, 3 and 4 branches, ms/step: 8 beams 1.93, 1.81, 1.76, 4.54; 16 2.31, 2.06, 2.07, 4.84; 64 4.49, 4.06,
+    // 4.09, 6.35; 256 18.0, 17.4, 17.4, 19.1 (with 4 queues 2.36, 2.90, 5.21 and 18.5 in 4 branches, the rest as with 8)
     static int default_branches() {
         const char* e = std::getenv("GPU_MAX_HW_QUEUES");
         const int queues = e ? std::atoi(e) : 4;
-        return std::max(1, std::min(4, queues - 2));
+        return std::max(1, std::min(2, queues - 2));
     }
     int branch_count(int n) const {
         const int g = branches > 0 ? branches : (exact_tiled() ? default_branches() : 1);
@@ -1848,14 +1848,12 @@ struct EngineT : EngineBase {
 
     // the branches' operator phases taking turns (the reference order's step): per CG iteration
     // each group's operator and finalize wait for the previous group's (round-robin over the
-    // groups), so that while one group runs its two node-after-node dot products (one wave per
+    // groups), so that while one group runs its two node-after-node dot products (one workgroup per
     // scene) the GPU runs the other groups' operators one at a time, instead of every group's
-    // operator at once and then every group's chains on an idle GPU.  Launched directly: a graph
+    // operator at once and then every group's dot products on an idle GPU.  Launched directly: a graph
     // per group cannot wait for another group's kernels.  Off by default: measured on the 256-beam
-    // mix (4 branches, 8 queues) 22.3 ms/step against 21.6 running freely -- a group's operator
-    // alone takes no less time than beside the others' (185-211 us for a quarter of the beams),
-    // its turn's wait adds about 200 us per iteration, and each group's own chain of dependent
-    // phases (two dot chains of about 190 us, its operator, finalize and update) sets the step.
+    // mix (2, 3 and 4 branches, 8 queues) 18.5, 19.4 and 22.5 ms/step against 17.4, 17.4 and 19.0
+    // running freely (18.0 in one branch) -- a group's operator alone takes about as long as beside the others'.
     hipEvent_t turn_ev[kMaxBranches] = {};
     void step_turns(const std::vector<std::vector<int32_t>>& groups, int nsteps, hipStream_t s, int G) {
         LaunchSet* ls[kMaxBranches] = {};
