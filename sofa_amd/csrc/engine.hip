@@ -920,11 +920,12 @@ struct EngineT : EngineBase {
         contact = dalloc<int8_t>(Ntot);
         HIPCHK(hipMemset(contact, 0, std::max<int64_t>(1, Ntot)));
         upload(mass, massh); upload(fixed, fixh);
+        if (inch.empty()) inch.assign(1, 0);   // entry 0, which a node of no element reads (Contributions)
         upload(inc_ptr, cnt); upload(inc, inch);
         upload(tet, teth); upload(rot, roth); upload(rest, resth); upload(kmat, kh);
         upload(em_ptr, emp); upload(em_nbr, emn); upload(em_val, emv);
         upload(osc_node, oscn); upload(osc_mean, oscm); upload(osc_amp, osca); upload(osc_w, oscw); upload(osc_phase, oscp);
-        ef = dalloc<VT>(12 * Etot);
+        ef = dalloc<VT>(12 * std::max<int64_t>(1, Etot));
         ef2 = dalloc<VT>(12 * Etot);
         p2 = dalloc<VT>(3 * Ntot);
         HIPCHK(hipMemset(p2, 0, 3 * Ntot * sizeof(VT)));

@@ -208,16 +208,15 @@ struct Contributions {
     VT c[B];
     __device__ __forceinline__ void slots(const int* __restrict__ inc, int s, int s1) {
 #pragma unroll
-        for (int t = 0; t < B; t++) slot[t] = inc[min(s + t, s1 - 1)];
+        for (int t = 0; t < B; t++) slot[t] = inc[max(min(s + t, s1 - 1), 0)];
     }
     __device__ __forceinline__ void values(const VT* __restrict__ ef) {
 #pragma unroll
         for (int t = 0; t < B; t++) c[t] = ef[3 * (int64_t)slot[t]];
     }
-    // the first eight values, and the next eight slots, on their way (a node of no element: nothing is read;
-    // an engine whose scenes have no element has no entry of inc or ef that may be)
+    // the first eight values, and the next eight slots, on their way (a node of no element reads another's, or
+    // entry 0, which every engine's lists and contributions have, and adds nothing)
     __device__ __forceinline__ void begin(const int* __restrict__ inc, int s0, int s1, const VT* __restrict__ ef) {
-        if (s0 >= s1) return;
         slots(inc, s0, s1);
         values(ef);
         if (s0 + B < s1) slots(inc, s0 + B, s1);
