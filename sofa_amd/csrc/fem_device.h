@@ -103,6 +103,13 @@ struct alignas(64) InstDev {
     int dot_fallbacks, pad_fb;
 };
 
+// a kernel argument that is first used behind another wait, loaded by the time that `with` has arrived (left
+// to the compiler, its load may come where it is used: one more trip to memory in a 5 us kernel)
+__device__ __forceinline__ int arrived(int v, int with) {
+    asm volatile("" : "+s"(v) : "s"(with));
+    return v;
+}
+
 // which entry of InstDev::dots a dot-product launch (k_scandot, k_seqdot) writes
 constexpr int kDotBB = 0, kDotPQ = 1, kDotRR = 2;
 

@@ -750,9 +750,10 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
                                                              VT* __restrict__ z = nullptr) {
     __shared__ double sh[kBlock], pr[kNodeThreads];
     const Blk bk = nblk[xcd_item()];
+    const int mark = stop_mark(arrived(it, bk.inst), 1);
     InstDev* ins = &inst[bk.inst];
     const InstDev in = *ins;
-    if (stopped_before(in.stopped, stop_mark(it, 1))) return;
+    if (stopped_before(in.stopped, mark)) return;
     const int j = threadIdx.x / 3, c = threadIdx.x - 3 * j;
     const int n = min(bk.begin + j, bk.end - 1);
     const bool live = bk.begin + j < bk.end;
@@ -765,7 +766,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_cg_update(const Blk* __restric
         const bool exempt = it == 1 && in.first_solve;
         const int stop = den == 0.0 ? 3 : fabs(den) <= in.thr && !exempt ? 2 : 0;
         if (stop) {
-            if (record) { ins->den = den; ins->stopped = stop_mark(it, 1); ins->end_reason = stop; ins->last_iters = it; }
+            if (record) { ins->den = den; ins->stopped = mark; ins->end_reason = stop; ins->last_iters = it; }
             return;
         }
     }

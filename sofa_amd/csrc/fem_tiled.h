@@ -1385,6 +1385,7 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
     __shared__ double sh[2][kBlock / 64];
     __shared__ double upper[EXACT ? 1 : kUpdateThreads - kBlock + 1];
     const NodeBlk nb = nb_[xcd_item()];
+    const int mark = stop_mark(arrived(iter, nb.scene), 1);
     InstDev* ins = &inst[nb.scene];
     const InstDev in = *ins;
     const Ranges rg = ranges[nb.scene];
@@ -1402,7 +1403,6 @@ __global__ __launch_bounds__(kUpdateThreads) void k_update(const NodeBlk* __rest
     if (zbuf) ld3(zbuf, n, zv);
     ld3(p, n, pv);
     ld3(q, n, qv);
-    const int mark = stop_mark(iter, 1);
     if (stopped_before(in.stopped, mark)) return;
     VT m = 0;
     int8_t fx = 0, ct = 0;
