@@ -1594,18 +1594,19 @@ struct EngineT : EngineBase {
         }
     }
     // whether the CG operator (MIXED: the inner one) recomputes the element record of `tiles` tiles
-    // (k_tile_apply's GEO).  In float, beyond the record that stays in the L2s of the XCDs (8 x 4 MB, the node
-    // vectors beside it): recomputing costs the latency of one more phase, which small sets notice.  In double it
-    // costs more arithmetic than the last-level cache's bandwidth saves, until the record and the vectors outgrow
-    // that (256 MB).  Sets of beams of 82,000 tetrahedra, 25 iterations, ms/step recomputed and read back, by MB of
-    // record: FP32 11 0.328 and 0.332, 23 0.394 and 0.412, 45 0.56 and 0.62, 107 1.08 and 1.09, 141 1.34 and 1.32,
-    // 174 1.66 and 1.73, 253 2.28 and 2.92; SPLIT 11 0.382 and 0.381, 23 0.456 and 0.486, 174 2.00 and 2.47; MIXED
-    // 11 0.387 and 0.386, 23 0.446 and 0.468, 174 1.92 and 2.04; FP64 26 0.49 and 0.47, 92 1.00 and 0.98, 131 1.27
-    // and 1.28, 158 1.43 and 1.47, 249 2.09 and 2.56.
-    static constexpr int64_t kRecordFloat = 16ll << 20, kRecordDouble = 144ll << 20;
+    // (k_tile_apply's GEO): beyond this the record and the node vectors together no longer stay in the 256 MB
+    // last-level cache from one iteration to the next; sooner with double vectors beside a float record.  Sets of
+    // beams of 82,000 tetrahedra (and an ellipsoid of a material per element), 25 iterations, ms/step recomputed and
+    // read back, by MB of record: FP32 141 1.34 and 1.32 (148 1.96 and 1.92), 158 1.50 and 1.52, 174 1.66 and 1.73, 253
+    // 2.28 and 2.92 (218 2.70 and 3.28); MIXED 141 1.56 and 1.59 (148 6.16 and 6.05), 174 1.92 and 2.04, 253 2.66 and 3.35
+    // (218 8.5 and 10.4); FP64 131 1.27 and 1.28, 158 1.43 and 1.47, 249 2.09 and 2.56; SPLIT 79 1.04 and 1.09 (92 1.62 and
+    // 1.65), 107 1.31 and 1.37, 141 1.67 and 1.83, 174 2.00 and 2.47.  Below the line neither wins throughout: recomputing
+    // is up to 10 % ahead at 20 to 60 MB of such beams (FP32 45 MB 0.56 and 0.62), behind on the ellipsoid at 92 MB (FP32 1.36
+    // and 1.31) and where latency rules (11 MB 0.328 and 0.332, SPLIT 0.382 and 0.381, FP64 26 MB 0.49 and 0.47).
+    static constexpr int64_t kRecordCached = (std::is_same<R, VT>::value ? 150ll : 96ll) << 20;
     bool recomputes(int64_t tiles) const {
         const int64_t record = mixed ? 18 * (int64_t)sizeof(float) : (12 + NR) * (int64_t)sizeof(R);
-        return tiled && tiles * kTileElems * record > (mixed || std::is_same<R, float>::value ? kRecordFloat : kRecordDouble);
+        return tiled && tiles * kTileElems * record > kRecordCached;
     }
     // ... in the current launch set (set_apply_variant 1 and 3 on a float engine: the host's rest shape, read back)
     bool recomputing() const { return cur->geo && !(std::is_same<R, float>::value && (apply_variant & 1)); }
