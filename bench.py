@@ -119,8 +119,9 @@ def apply_roofline(eng, reps, pe, pv, nrec, E, N, node_extra=0):
     """The dominant kernel: the tiled CG operator (p = r + beta p staged in LDS, element K p,
     per-node sums in LDS, q of tile-owned nodes, partials of shared nodes) over every scene of the
     engine in one launch, timed with HIP events on its stream.  k_tile_exact (reference order)
-    recomputes the element geometry (rotation, rest coordinates) from the node positions;
-    k_tile_apply reads it back, bytes that an operator can do without and that are not counted here.
+    recomputes the element geometry (rotation, rest coordinates) from the node positions, and so does
+    k_tile_apply on sets of this size; on smaller ones it reads it back, bytes that an operator can do
+    without and that are not counted here.
     Algorithmic bytes per launch: E (16 + nrec p_e) + N 18 p_v
       per element: 16 B of indices (4 local node ids + 4 incidence slots, u16 each) and nrec
                    reals: the stiffness entries K00, K01, K33 (3) where elements have their own
@@ -286,11 +287,7 @@ def mix_paths(specs, args):
         row.update({"value": E * args.steps / (total_ms / 1e3), "ms_per_step": total_ms / args.steps,
                     "p50_ms": float(np.percentile(lat, 50)), "p99_ms": float(np.percentile(lat, 99))})
         if prec == "FP64_TILED" and seq:
-            # the node-after-node dot products by exact parallel rounding (the library's default, the
-            # chain's bits)
-            row["dot_segments"] = {"segments": 8, "window": 32,
-                                   "fallbacks": int(sum(eng.stats(i)["dot_fallbacks"] for i in ids)),
-                                   "steps": args.error_steps + args.warmup + args.steps}
+            row["dot_products"] = "exact parallel rounding (the bits of the node-after-node chain)"
         if name in _PATH_BYTES:
             pe, pv, extra = _PATH_BYTES[name]
             r = apply_roofline(eng, args.apply_reps, pe, pv, 0, E, N, node_extra=extra)

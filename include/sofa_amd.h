@@ -67,9 +67,10 @@ typedef struct sofa_amd_cg_stats {
     double  err;            /* last sqrt(r.r)/|b|                                            */
     double  den;            /* last p.A.p                                                    */
     double  time;           /* context time of the scene                                     */
-    int32_t dot_fallbacks;  /* FP64_TILED in the reference order with dot products in segments
-                               without candidates (window 0): boundaries summed by the chain
-                               since the scene was placed; else 0                                */
+    int32_t dot_fallbacks;  /* FP64_TILED in the reference order, scenes of 8192 nodes or more, while
+                               sofa_amd_engine_set_dot_segments has a window of 0: segments - 1 per
+                               dot product since the scene was placed; else 0 (no sum runs in
+                               segments: it counts what was asked for)                           */
     int32_t reserved;       /* 0                                                                 */
 } sofa_amd_cg_stats;
 

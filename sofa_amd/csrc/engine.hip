@@ -346,8 +346,8 @@ struct EngineBase {
     bool stepped = false;             // a step has been enqueued
     int branches = 0;                 // concurrent branches of a merged step (0: the engine's default)
     bool branch_turns = false;        // the branches' operator phases take turns (reference order)
-    int dot_segments = 8;             // reference-order dots on FP64_TILED: segments run at once
-    int dot_window = 32;              // ... candidate start values per side of each boundary
+    int dot_segments = 8;             // reference-order dots on FP64_TILED: 1, or a window of 0: the chain of
+    int dot_window = 32;              // dependent adds (k_seqdot), else exact parallel rounding (k_scandot)
     double* vdot_part = nullptr;      // vDot's per-block partials (grown on demand)
     int64_t vdot_len = 0;
     virtual int autotune(int reps, hipStream_t s, float* us_out) = 0;
@@ -1798,9 +1798,10 @@ struct EngineT : EngineBase {
     hipStream_t aux[kMaxBranches - 1] = {};
     hipEvent_t fork_ev = nullptr, join_ev[kMaxBranches - 1] = {};
     // the default: one branch per hardware queue the runtime's own streams leave free (HIP gives a
-    // process GPU_MAX_HW_QUEUES of them, 4 unless set; two are taken), at most 2.  Measured with 8 queues,
-    // 1, 2, 3 and 4 branches, ms/step: 8 beams 1.93, 1.81, 1.76, 4.54; 16 2.31, 2.06, 2.07, 4.84; 64 4.49, 4.06,
-    // 4.09, 6.35; 256 18.0, 17.4, 17.4, 19.1 (with 4 queues 2.36, 2.90, 5.21 and 18.5 in 4 branches, the rest as with 8)
+    // process GPU_MAX_HW_QUEUES of them, 4 unless set; two are taken), at most 2.  Measured in processes of
+    // 4 and 8 queues, on the caller's stream and the engine's, 1, 2, 3 and 4 branches, ms/step: 8 beams 1.9, 1.75, 1.8-4.4,
+    // 2.5-4.4; 16 2.4, 2.1, 2.1, 1.95-4.7; 64 4.5, 4.2, 4.1, 4.1-6.5; 256 18.2, 17.5, 17.5, 17.3-19.4: more than two gain
+    // little and depend on the queues that the streams come to share
     static int default_branches() {
         const char* e = std::getenv("GPU_MAX_HW_QUEUES");
         const int queues = e ? std::atoi(e) : 4;

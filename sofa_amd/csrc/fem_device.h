@@ -31,7 +31,8 @@ namespace sofa_amd {
 constexpr int kBlock = 256;   // threads per block for every kernel (4 wave64)
 
 // ---------------------------------------------------------------------------------------
-// per-scene device record; one per scene, written by the last block of each reduction
+// per-scene device record; one per scene, written by the scene's first block (CG iterations), the last
+// block of a reduction (the start of a solve) or a kernel of one workgroup per scene
 // ---------------------------------------------------------------------------------------
 // A kernel copies the record at its head (const InstDev in = *ins) and reads the copy: the fields it
 // uses are then fetched by scalar loads that are all in flight with its first gathers.  Read where
@@ -98,8 +99,7 @@ struct alignas(64) InstDev {
     double* lm_x0;
     const double* lm_keys;
     int lm_n, lm_nk, lm_relative, lm_x0_set;
-    // reference-order dot products asked for in segments without candidates: boundaries summed by
-    // the chain (counted since the scene was placed)
+    // segments - 1 per reference-order dot product while a window of 0 is set (since the scene was placed)
     int dot_fallbacks, pad_fb;
 };
 
@@ -124,8 +124,8 @@ constexpr int kDotBB = 0, kDotPQ = 1, kDotRR = 2;
 // alone, 4.2 ns with groups of 16, 3.7 ns with 32, 4.1 ns with 64).  The last chunk is padded with +0.0, which leaves the sum
 // unchanged: s + 0.0 == s for every s but -0.0, and a sum that starts at +0.0 is never -0.0 under
 // round-to-nearest.  The scene's scalar lands in InstDev::dots[which]; a stopped scene is skipped.
-// `boundaries`: segment boundaries the caller asked for without candidates (window 0), every one
-// of them a fallback to the chain, counted for scenes of kSeqCounted nodes or more.
+// `boundaries`: what the caller's choice of segments with a window of 0 adds to dot_fallbacks, for scenes of
+// kSeqCounted nodes or more (an accounting that callers of set_dot_segments read: nothing runs in segments).
 constexpr int kSeqChunk = 1024, kSeqGroup = 32, kSeqCounted = 8192;
 __device__ __forceinline__ void seq_group_load(const double* c, double g[kSeqGroup]) {
     const double2* c2 = reinterpret_cast<const double2*>(c);

@@ -645,7 +645,7 @@ __global__ __launch_bounds__(kBlock) void k_fin_rhs(const FinBlk* __restrict__ f
 //   5. by the waves that have nodes: interior nodes finished (q), a shared node's sum left as the tile's
 //      partial, p.q as one partial per tile.
 // The element's rotation, rest shape and K are read back (18 floats, 21 doubles), not recomputed from the
-// positions: 460 instead of 610 vector instructions per wave in float, and a phase less.  GEO: recomputed from
+// positions: a phase less, and 417 vector instructions per wave on 256 beams in float, 482 with GEO.  GEO: recomputed from
 // the positions x, x0 all the same (same bits), for sets whose record does not stay cached from one iteration to
 // the next (EngineT::recomputes has the line), the sums then by the threads that have a node's p in registers, which
 // takes back the phase and its LDS traffic.  What bounds it: on a large mesh VALU issue (half of the time), LDS (a

@@ -50,7 +50,7 @@ def footprint_bytes(precision, nodes, tets, reference_order=False, scenes=1):
     if reference_order:
         per_tet += 4 * 2 * 3 * pv + 4 * 2
         per_node += 8
-        # the segmented dot products' prediction chunks (plain and modelled) and candidate sums
+        # a margin (the size of buffers that the dot products kept per scene; they keep none now)
         per_scene += 8 * (2 * 64 + 1800)
     return per_node * nodes + per_tet * tets + per_scene * scenes
 
